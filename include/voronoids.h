@@ -82,6 +82,11 @@ int vo_tri_run(vo_tri* t);
  * max_simplex_id convention (creation order differs from the reference's). */
 int vo_tri_counts(const vo_tri* t, int64_t* n_vertices, int64_t* n_simplices, int64_t* max_simplex_id);
 
+/* the sphere DelaunayTree::new gives simplex 0 (src/delaunay_tree.rs:389-412, :544-566): the
+ * bounding sphere's center[dim] and ten times its radius (radius 1 where it is zero: no points,
+ * one point, or all points equal) */
+int vo_tri_root_sphere(const vo_tri* t, double* center, double* radius);
+
 /* live simplices: simplices[n_s*(dim+1)] vertex ids (reference id space, positively
  * oriented), neighbors[n_s*(dim+1)] = index (in this export) of the simplex across the face
  * opposite each vertex, or -1 on the hull of the super simplex.  Either pointer may be NULL. */

@@ -91,14 +91,7 @@ class DelaunayTree:
         _lib.check(_lib.lib().vo_tri_create(device, self.dim, p.ctypes.data_as(_dp), p.shape[0], ctypes.byref(h)))
         self._h = h
         self._n_input = 0
-        # the sphere DelaunayTree::new stores on simplex 0: (bounding-sphere center, 10 x radius)
-        # (an empty or single-point input, which has no super simplex in the reference, uses radius 1)
-        c = np.zeros(3)
-        r = ctypes.c_double(0.0)
-        if p.shape[0]:
-            _lib.check(_lib.lib().vo_bounding_sphere(self.dim, p.ctypes.data_as(_dp), p.shape[0],
-                                                     c.ctypes.data_as(_dp), ctypes.byref(r)))
-        self._root_sphere = (c[:self.dim].tolist(), 10.0 * (r.value if r.value > 0 else 1.0))
+        self._root_sphere = self._frame()
         if tuned:
             for key, value in _tuned(self.dim).items():
                 self.config(key, value)
@@ -108,12 +101,15 @@ class DelaunayTree:
         p = _as_points(vertices, self.dim)
         _lib.check(_lib.lib().vo_tri_reset(self._h, p.ctypes.data_as(_dp), p.shape[0]))
         self._n_input = 0
-        c = np.zeros(3)
+        self._root_sphere = self._frame()
+
+    def _frame(self) -> tuple[list, float]:
+        """the sphere DelaunayTree::new stores on simplex 0: (bounding-sphere center, 10 x radius)
+        (an empty or single-point input, which has no super simplex in the reference, uses radius 1)"""
+        c = (ctypes.c_double * 3)()
         r = ctypes.c_double(0.0)
-        if p.shape[0]:
-            _lib.check(_lib.lib().vo_bounding_sphere(self.dim, p.ctypes.data_as(_dp), p.shape[0],
-                                                     c.ctypes.data_as(_dp), ctypes.byref(r)))
-        self._root_sphere = (c[:self.dim].tolist(), 10.0 * (r.value if r.value > 0 else 1.0))
+        _lib.check(_lib.lib().vo_tri_root_sphere(self._h, c, ctypes.byref(r)))
+        return list(c)[:self.dim], r.value
 
     def close(self) -> None:
         if getattr(self, "_h", None):

@@ -32,6 +32,23 @@ inline int fail(int code, const std::string& msg) {
 // bounding_sphere, src/geometry.rs:99-141: per-axis min/max folds, center (hi+lo)/2, radius
 // the larger corner distance, then one pass in input order multiplying the radius by 1.5 for
 // every point the current sphere does not strictly contain (in_sphere, :91-97).
+inline double corner_radius(int D, const double* lo, const double* hi, double* c) {
+    for (int i = 0; i < D; ++i) c[i] = (hi[i] + lo[i]) / 2.0;
+    double su = 0.0, sl = 0.0;
+    for (int i = 0; i < D; ++i) su += (hi[i] - c[i]) * (hi[i] - c[i]);
+    for (int i = 0; i < D; ++i) sl += (lo[i] - c[i]) * (lo[i] - c[i]);
+    const double ud = std::sqrt(su), ld = std::sqrt(sl);
+    return ud > ld ? ud : ld;
+}
+// the pass from point `start` on
+inline double grow_radius(int D, const double* pts, int64_t start, int64_t n, const double* c, double rad) {
+    for (int64_t k = start; k < n; ++k) {
+        double dist = 0.0;
+        for (int i = 0; i < D; ++i) dist += (c[i] - pts[k * D + i]) * (c[i] - pts[k * D + i]);
+        if (!(dist < rad * rad)) rad = rad * 1.5;
+    }
+    return rad;
+}
 inline void bounding_sphere(int D, const double* pts, int64_t n, double* c, double* r) {
     double lo[3], hi[3];
     for (int i = 0; i < D; ++i) {
@@ -41,19 +58,8 @@ inline void bounding_sphere(int D, const double* pts, int64_t n, double* c, doub
             lo[i] = std::fmin(lo[i], pts[k * D + i]);
             hi[i] = std::fmax(hi[i], pts[k * D + i]);
         }
-        c[i] = (hi[i] + lo[i]) / 2.0;
     }
-    double su = 0.0, sl = 0.0;
-    for (int i = 0; i < D; ++i) su += (hi[i] - c[i]) * (hi[i] - c[i]);
-    for (int i = 0; i < D; ++i) sl += (lo[i] - c[i]) * (lo[i] - c[i]);
-    const double ud = std::sqrt(su), ld = std::sqrt(sl);
-    double rad = ud > ld ? ud : ld;
-    for (int64_t k = 0; k < n; ++k) {
-        double dist = 0.0;
-        for (int i = 0; i < D; ++i) dist += (c[i] - pts[k * D + i]) * (c[i] - pts[k * D + i]);
-        if (!(dist < rad * rad)) rad = rad * 1.5;
-    }
-    *r = rad;
+    *r = grow_radius(D, pts, 0, n, c, corner_radius(D, lo, hi, c));
 }
 
 // circumsphere, src/geometry.rs:2-56, in the reference's evaluation order.  Returns false when

@@ -149,7 +149,9 @@ struct vo_tri {
     int* misc1 = nullptr;              // nk, nf, status of the single point
     int big_cap = 1 << 20;
     // hints
-    int* hint = nullptr;
+    int* hint = nullptr;               // kept over resets while it is large enough
+    int64_t hint_cap = 0;
+    bool hinted = false;               // it belongs to the present tree (set up at its first stage)
     int hlevels = 0;
     float glo[3] = {0, 0, 0};
     float ginv = 1;
@@ -160,6 +162,7 @@ struct vo_tri {
     QEntry* q = nullptr;
     int qcap = 0;
     CEntry* cache = nullptr;
+    bool cache_used = false;           // exact signs may have been written since it was cleared
     uint32_t cmask = 0;
     double* ws = nullptr;
     int ws_cap = 0, ws_threads = 0;
@@ -255,6 +258,68 @@ Ctx make_ctx(const vo_tri* t) {
     c.pend_cap = t->win_cap;
     c.region = nullptr;
     return c;
+}
+
+// Folds of the bounding sphere over n points (row-major, D columns): per block the least and
+// largest coordinate of each axis and whether a coordinate is not finite.  One stream over the
+// points, 24 B each (3D); the blocks' results go to the host, which folds the few of them.
+struct Bounds {
+    double lo[3], hi[3];
+    int bad, pad;
+};
+constexpr int kBoundBlocks = 256;
+template <int D> __global__ void __launch_bounds__(256) k_point_bounds(const double* pts, int64_t n, Bounds* out) {
+    __shared__ Bounds s_b[4];
+    Bounds b;
+    for (int k = 0; k < 3; ++k) {
+        b.lo[k] = INFINITY;
+        b.hi[k] = -INFINITY;
+    }
+    b.bad = b.pad = 0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        for (int k = 0; k < D; ++k) {
+            const double x = pts[i * D + k];
+            b.bad |= !(fabs(x) < INFINITY);
+            b.lo[k] = fmin(b.lo[k], x);
+            b.hi[k] = fmax(b.hi[k], x);
+        }
+    for (int o = 32; o > 0; o >>= 1) {
+        for (int k = 0; k < D; ++k) {
+            b.lo[k] = fmin(b.lo[k], __shfl_xor(b.lo[k], o, 64));
+            b.hi[k] = fmax(b.hi[k], __shfl_xor(b.hi[k], o, 64));
+        }
+        b.bad |= __shfl_xor(b.bad, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) s_b[threadIdx.x >> 6] = b;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w) {
+            for (int k = 0; k < D; ++k) {
+                b.lo[k] = fmin(b.lo[k], s_b[w].lo[k]);
+                b.hi[k] = fmax(b.hi[k], s_b[w].hi[k]);
+            }
+            b.bad |= s_b[w].bad;
+        }
+        out[blockIdx.x] = b;
+    }
+}
+
+// the first point at or after `start` that the sphere (c, r2 = r * r) does not strictly contain
+// (the reference's in_sphere: squared distance summed over the axes in order)
+template <int D>
+__global__ void __launch_bounds__(256) k_first_outside(const double* pts, int64_t n, int64_t start, double c0, double c1,
+                                                       double c2, double r2, unsigned long long* first) {
+    const double c[3] = {c0, c1, c2};
+    unsigned long long best = ~0ull;
+    for (int64_t i = start + (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+        double dist = 0.0;
+        for (int k = 0; k < D; ++k) dist += (c[k] - pts[i * D + k]) * (c[k] - pts[i * D + k]);
+        if (!(dist < r2)) {
+            best = (unsigned long long)i;
+            break;
+        }
+    }
+    if (best != ~0ull) atomicMin(first, best);
 }
 
 // next window = pending losers followed by fresh points head .. head + nfresh - 1
@@ -602,21 +667,43 @@ int grow_points(vo_tri* t, int64_t cap) {
     return 0;
 }
 
-int upload_super(vo_tri* t) {
-    std::vector<double> x64((size_t)t->M * t->S, 0.0);
-    std::vector<float> x32((size_t)t->M * t->S, 0.0f);
-    std::vector<int> vm(t->M);
-    for (int v = 0; v < t->M; ++v) {
-        for (int k = 0; k < t->D; ++k) {
-            x64[v * t->S + k] = t->sv[v][k];
-            x32[v * t->S + k] = (float)(t->sv[v][k] - t->c[k]);
-        }
-        vm[v] = v;
+// An empty tree: the super vertices, the first simplex's record, the round state and cleared
+// statistics, as one launch (as copies and clears of its own each of these costs a submission:
+// a reset at n = 40 took 89 us with eight of them and a reallocated hint grid, 21 us so)
+struct InitTree {
+    double x64[16];
+    float x32[16];
+    int4 rec[8];
+};
+__global__ void __launch_bounds__(256) k_init_tree(InitTree in, int M, int S, int rec_bytes, double* X64, float* X32,
+                                                   int* vmap, char* rec, RoundState* st, Counters* cnt) {
+    const int i = threadIdx.x;
+    if (i < M * S) {
+        X64[i] = in.x64[i];
+        X32[i] = in.x32[i];
     }
-    VO_HIP(hipMemcpyAsync(t->X64, x64.data(), sizeof(double) * x64.size(), hipMemcpyHostToDevice, t->s));
-    VO_HIP(hipMemcpyAsync(t->X32, x32.data(), sizeof(float) * x32.size(), hipMemcpyHostToDevice, t->s));
-    VO_HIP(hipMemcpyAsync(t->vmap, vm.data(), sizeof(int) * vm.size(), hipMemcpyHostToDevice, t->s));
-    VO_HIP(hipStreamSynchronize(t->s));
+    if (i < M) vmap[i] = i;
+    if (i < rec_bytes / 16) reinterpret_cast<int4*>(rec)[i] = in.rec[i];
+    static_assert(sizeof(RoundState) % 16 == 0 && sizeof(Counters) % 16 == 0, "cleared 16 bytes at a time");
+    int4* w = reinterpret_cast<int4*>(st);
+    for (int k = i; k < (int)(sizeof(RoundState) / 16); k += 256) w[k] = make_int4(0, 0, 0, 0);
+    w = reinterpret_cast<int4*>(cnt);
+    for (int k = i; k < (int)(sizeof(Counters) / 16) * kCntStripes; k += 256) w[k] = make_int4(0, 0, 0, 0);
+    __syncthreads();
+    if (i == 0) st->n_tets = 1;
+}
+
+int init_tree(vo_tri* t) {
+    InitTree in = {};
+    for (int v = 0; v < t->M; ++v)
+        for (int k = 0; k < t->D; ++k) {
+            in.x64[v * t->S + k] = t->sv[v][k];
+            in.x32[v * t->S + k] = (float)(t->sv[v][k] - t->c[k]);
+        }
+    root_record(t->D, t->tet0, 0, t->sv, t->c, reinterpret_cast<unsigned char*>(in.rec));
+    hipLaunchKernelGGL(k_init_tree, dim3(1), dim3(256), 0, t->s, in, t->M, t->S, record_bytes(t->D), t->X64, t->X32, t->vmap,
+                       t->rec, t->st, t->cnt);
+    VO_HIP(hipGetLastError());
     return 0;
 }
 
@@ -662,6 +749,7 @@ int check_err(vo_tri* t) {
 int run_exact(vo_tri* t, int nq) {
     if (nq <= 0) return 0;
     nq = std::min(nq, t->qcap);
+    t->cache_used = true;
     const int threads = 64;
     const int blocks = std::max(1, std::min((nq + threads - 1) / threads, t->ws_threads / threads));
     VO_HIP(hipEventRecord(t->ev[4], t->s));
@@ -1181,6 +1269,7 @@ int absorb_halted_plan(vo_tri* t, const RunPlan& P, bool flags = false) {
     const bool exact_done = P.exact_dev != 0;
     if (exact_done && P.nq_done > 0) t->st_host->n_q = P.nq_done;
     if (P.launched && t->st_host->n_q > 0) t->exact_dev = 1;
+    if (t->exact_dev) t->cache_used = true;
     if (P.launched && (rc = finish_round(t, P.nwin, P.nfresh, nullptr, 0.f, 0.f, exact_done))) return rc;
     if ((rc = check_err(t))) return rc;
     if (P.halt & HALT_STALL) return fail(VO_ERR_INTERNAL, "no progress for 64 rounds");
@@ -1432,6 +1521,87 @@ struct Scratch {
     }
 };
 
+// From this many points on the bounding sphere (and the check for non-finite coordinates) is
+// folded on the device: the upload, two kernels and two readbacks take about 45 us, the host
+// 7 ns a point (3D: 10 k points 70 us, 4 M 26 ms; device 3.7 ms, nearly all of it the upload).
+constexpr int64_t kDeviceFrame = 1 << 13;
+
+bool all_finite(const double* x, int64_t n) {
+    for (int64_t i = 0; i < n; ++i)
+        if (!std::isfinite(x[i])) return false;
+    return true;
+}
+
+// set_frame with the folds on the device, the same values bit for bit: the folds of least and
+// largest are exact in any order, the sums and roots of the two corners are the host's, and the
+// pass that grows the radius goes from one point outside the sphere to the next in input order.
+// An axis whose coordinates are all zero is left to the host (there the order of +0 and -0 picks
+// the sign of the center).
+int device_frame(vo_tri* t, const double* pts, int64_t n, double* c, double* r) {
+    const int D = t->D;
+    Scratch mem(t);
+    double* dp;
+    Bounds* db;
+    unsigned long long* df;
+    int rc;
+    if ((rc = mem.get(&dp, (size_t)n * D)) || (rc = mem.get(&db, (size_t)kBoundBlocks)) || (rc = mem.get(&df, 1))) return rc;
+    VO_HIP(hipMemcpyAsync(dp, pts, sizeof(double) * (size_t)n * D, hipMemcpyHostToDevice, t->s));
+    if (D == 3) hipLaunchKernelGGL(k_point_bounds<3>, dim3(kBoundBlocks), dim3(256), 0, t->s, dp, n, db);
+    else hipLaunchKernelGGL(k_point_bounds<2>, dim3(kBoundBlocks), dim3(256), 0, t->s, dp, n, db);
+    VO_HIP(hipGetLastError());
+    std::vector<Bounds> hb(kBoundBlocks);
+    VO_HIP(hipMemcpyAsync(hb.data(), db, sizeof(Bounds) * kBoundBlocks, hipMemcpyDeviceToHost, t->s));
+    VO_HIP(hipStreamSynchronize(t->s));
+    double lo[3], hi[3];
+    for (int k = 0; k < D; ++k) {
+        lo[k] = INFINITY;
+        hi[k] = -INFINITY;
+        for (const Bounds& b : hb) {
+            lo[k] = std::fmin(lo[k], b.lo[k]);
+            hi[k] = std::fmax(hi[k], b.hi[k]);
+        }
+    }
+    for (const Bounds& b : hb)
+        if (b.bad) return fail(VO_ERR_INVALID, "non-finite coordinate");
+    for (int k = 0; k < D; ++k)
+        if (lo[k] == 0.0 && hi[k] == 0.0) {
+            set_frame(D, pts, n, c, r);
+            return 0;
+        }
+    c[0] = c[1] = c[2] = 0.0;
+    double rad = corner_radius(D, lo, hi, c);
+    int64_t start = 0;
+    for (int grown = 0;; ++grown) {
+        // (a radius that growing no longer changes, or one too small to square, grows on the host)
+        if (grown == 8 || !(rad * rad > 0.0) || !std::isfinite(rad)) {
+            rad = grow_radius(D, pts, start, n, c, rad);
+            break;
+        }
+        unsigned long long first = ~0ull;
+        VO_HIP(hipMemsetAsync(df, 0xFF, sizeof(first), t->s));
+        if (D == 3)
+            hipLaunchKernelGGL(k_first_outside<3>, dim3(1024), dim3(256), 0, t->s, dp, n, start, c[0], c[1], c[2], rad * rad, df);
+        else
+            hipLaunchKernelGGL(k_first_outside<2>, dim3(1024), dim3(256), 0, t->s, dp, n, start, c[0], c[1], 0.0, rad * rad, df);
+        VO_HIP(hipGetLastError());
+        VO_HIP(hipMemcpyAsync(&first, df, sizeof(first), hipMemcpyDeviceToHost, t->s));
+        VO_HIP(hipStreamSynchronize(t->s));
+        if (first >= (unsigned long long)n) break;
+        rad = rad * 1.5;
+        start = (int64_t)first + 1;
+    }
+    *r = rad > 0.0 ? rad : 1.0;
+    return 0;
+}
+
+// the frame of a point set (set_frame), or VO_ERR_INVALID for a non-finite coordinate
+int point_frame(vo_tri* t, const double* pts, int64_t n, double* c, double* r) {
+    if (n >= kDeviceFrame) return device_frame(t, pts, n, c, r);
+    if (!all_finite(pts, n * t->D)) return fail(VO_ERR_INVALID, "non-finite coordinate");
+    set_frame(t->D, pts, n, c, r);
+    return 0;
+}
+
 int bit_length(int64_t x) {
     int b = 0;
     while (x > 0) {
@@ -1612,11 +1782,14 @@ int vo_tri_create(int hip_device, int dim, const double* pts, int64_t n, vo_tri*
     *out = nullptr;
     if (dim != 2 && dim != 3) return fail(VO_ERR_INVALID, "dim must be 2 or 3");
     if (n < 0 || (n > 0 && !pts)) return fail(VO_ERR_INVALID, "bad point buffer");
-    for (int64_t i = 0; i < n * dim; ++i)
-        if (!std::isfinite(pts[i])) return fail(VO_ERR_INVALID, "non-finite coordinate");
     int ndev = 0;
-    VO_HIP(hipGetDeviceCount(&ndev));
-    if (hip_device < 0 || hip_device >= ndev) return fail(VO_ERR_INVALID, "no such HIP device");
+    const hipError_t counted = hipGetDeviceCount(&ndev);
+    if (counted != hipSuccess || hip_device < 0 || hip_device >= ndev) {
+        if (!all_finite(pts, n * dim)) return fail(VO_ERR_INVALID, "non-finite coordinate");
+        VO_HIP(counted);
+        return fail(VO_ERR_INVALID, "no such HIP device");
+    }
+    if (n < kDeviceFrame && !all_finite(pts, n * dim)) return fail(VO_ERR_INVALID, "non-finite coordinate");
     VO_HIP(hipSetDevice(hip_device));
     vo_tri* t = new vo_tri();
     t->dev = hip_device;
@@ -1632,10 +1805,6 @@ int vo_tri_create(int hip_device, int dim, const double* pts, int64_t n, vo_tri*
     if (hipStreamCreateWithFlags(&t->s, hipStreamNonBlocking) != hipSuccess) return bail(fail(VO_ERR_HIP, "stream"));
     for (auto& e : t->ev)
         if (hipEventCreate(&e) != hipSuccess) return bail(fail(VO_ERR_HIP, "event"));
-    set_frame(dim, pts, n, t->c, &t->r);
-    t->R = t->r * 10.0;
-    super_vertices(dim, t->c, t->R, t->sv);
-    first_simplex_order(dim, t->sv, t->tet0);
     // windows: capacity and per-point cavity buffers
     // a window never holds more than the set's points
     {
@@ -1669,24 +1838,15 @@ int vo_tri_create(int hip_device, int dim, const double* pts, int64_t n, vo_tri*
         (rc = dev_alloc(&t->pflag, t->win_cap)))
         return bail(rc);
     t->fix_cap = 2 * t->win_cap;
+    if ((rc = point_frame(t, pts, n, t->c, &t->r))) return bail(rc);
+    t->R = t->r * 10.0;
+    super_vertices(dim, t->c, t->R, t->sv);
+    first_simplex_order(dim, t->sv, t->tet0);
     if (hipHostMalloc((void**)&t->st_host, sizeof(RoundState)) != hipSuccess) return bail(fail(VO_ERR_OOM, "pinned"));
-    hipMemsetAsync(t->st, 0, sizeof(RoundState), t->s);
-    hipMemsetAsync(t->cnt, 0, sizeof(Counters) * kCntStripes, t->s);
     hipMemsetAsync(t->cache, 0xFF, sizeof(CEntry) * ((size_t)t->cmask + 1), t->s);
     if ((rc = grow_points(t, std::max<int64_t>(n, 16)))) return bail(rc);
-    if ((rc = upload_super(t))) return bail(rc);
-    if ((rc = grow_tets(t, 1024))) return bail(rc);
-    {
-        unsigned char r0[128];
-        root_record(dim, t->tet0, 0, t->sv, t->c, r0);
-        if (hipMemcpyAsync(t->rec, r0, (size_t)record_bytes(dim), hipMemcpyHostToDevice, t->s) != hipSuccess)
-            return bail(fail(VO_ERR_HIP, "init record"));
-    }
-    RoundState init = {};
-    init.n_tets = 1;
-    if (hipMemcpyAsync(t->st, &init, sizeof(init), hipMemcpyHostToDevice, t->s) != hipSuccess ||
-        hipStreamSynchronize(t->s) != hipSuccess)
-        return bail(fail(VO_ERR_HIP, "init"));
+    if ((rc = grow_tets(t, 1024)) || (rc = init_tree(t))) return bail(rc);
+    if (hipStreamSynchronize(t->s) != hipSuccess) return bail(fail(VO_ERR_HIP, "init"));
     *out = t;
     return 0;
 }
@@ -1702,12 +1862,14 @@ int vo_tri_reset(vo_tri* t, const double* pts, int64_t n) {
     if (!t) return fail(VO_ERR_INVALID, "null handle");
     if (n < 0 || (n > 0 && !pts)) return fail(VO_ERR_INVALID, "bad point buffer");
     const int dim = t->D;
-    for (int64_t i = 0; i < n * dim; ++i)
-        if (!std::isfinite(pts[i])) return fail(VO_ERR_INVALID, "non-finite coordinate");
     VO_HIP(hipSetDevice(t->dev));
     VO_HIP(hipStreamSynchronize(t->s));
     // the frame and super simplex of the new point set, as vo_tri_create
-    set_frame(dim, pts, n, t->c, &t->r);
+    double c[3], r;
+    int rc;
+    if ((rc = point_frame(t, pts, n, c, &r))) return rc;
+    for (int k = 0; k < 3; ++k) t->c[k] = c[k];
+    t->r = r;
     t->R = t->r * 10.0;
     super_vertices(dim, t->c, t->R, t->sv);
     first_simplex_order(dim, t->sv, t->tet0);
@@ -1734,21 +1896,18 @@ int vo_tri_reset(vo_tri* t, const double* pts, int64_t n) {
     t->edited = false;
     // device state: super vertices, the first record, cleared round state and statistics, no
     // cached exact signs (they are keyed by vertex ids), and a new hint grid at the next stage
-    if (t->hint) {
-        hipFree(t->hint);
-        t->hint = nullptr;
-    }
-    int rc;
-    if ((rc = grow_points(t, std::max<int64_t>(n, 16))) || (rc = upload_super(t))) return rc;
-    unsigned char r0[128];
-    root_record(dim, t->tet0, 0, t->sv, t->c, r0);
-    VO_HIP(hipMemcpyAsync(t->rec, r0, (size_t)record_bytes(dim), hipMemcpyHostToDevice, t->s));
-    RoundState init = {};
-    init.n_tets = 1;
-    VO_HIP(hipMemcpyAsync(t->st, &init, sizeof(init), hipMemcpyHostToDevice, t->s));
-    VO_HIP(hipMemsetAsync(t->cnt, 0, sizeof(Counters) * kCntStripes, t->s));
-    VO_HIP(hipMemsetAsync(t->cache, 0xFF, sizeof(CEntry) * ((size_t)t->cmask + 1), t->s));
+    t->hinted = false;
+    if ((rc = grow_points(t, std::max<int64_t>(n, 16))) || (rc = init_tree(t))) return rc;
+    if (t->cache_used) VO_HIP(hipMemsetAsync(t->cache, 0xFF, sizeof(CEntry) * ((size_t)t->cmask + 1), t->s));
+    t->cache_used = false;
     VO_HIP(hipStreamSynchronize(t->s));
+    return 0;
+}
+
+int vo_tri_root_sphere(const vo_tri* t, double* center, double* radius) {
+    if (!t || !center || !radius) return fail(VO_ERR_INVALID, "null argument");
+    for (int k = 0; k < t->D; ++k) center[k] = t->c[k];
+    *radius = t->R;
     return 0;
 }
 
@@ -1789,15 +1948,22 @@ int vo_tri_stage(vo_tri* t, const double* pts, int64_t n, uint64_t seed) {
     const int64_t n_after = t->n_pts + n;
     // walk-start hints: grids of 2^l cells per axis over the bounding sphere's box, finest
     // level about 4 points a cell; level 0 holds the initial simplex
-    if (!t->hint) {
+    if (!t->hinted) {
         const int L = hint_levels(D, n_after);
         t->hlevels = L;
         const int64_t cells = hint_cells(D, L);
         for (int k = 0; k < 3; ++k) t->glo[k] = (float)(-t->r);
         t->ginv = (float)(1.0 / (2.0 * t->r));
-        if ((rc = dev_alloc(&t->hint, cells))) return rc;
+        if (cells > t->hint_cap) {
+            hipFree(t->hint);
+            t->hint = nullptr;
+            t->hint_cap = 0;
+            if ((rc = dev_alloc(&t->hint, cells))) return rc;
+            t->hint_cap = cells;
+        }
         VO_HIP(hipMemsetAsync(t->hint, 0xFF, sizeof(int) * cells, t->s));
         VO_HIP(hipMemsetAsync(t->hint, 0, sizeof(int), t->s));
+        t->hinted = true;
     }
     // simplex capacity for everything staged (uniform data creates ~27 (3D) / 6 (2D) per point)
     choose_reuse(t, n_after - t->inserted - t->dups);
@@ -2194,7 +2360,7 @@ int vo_tri_locate(vo_tri* t, const double* p, int32_t* killed, int64_t killed_ca
         if (!std::isfinite(p[k])) return fail(VO_ERR_INVALID, "non-finite coordinate");
     VO_HIP(hipSetDevice(t->dev));
     const Ctx c = make_ctx(t);
-    const int start = t->hint ? -1 : 0;          // no hint grid before the first stage: the first record
+    const int start = t->hinted ? -1 : 0;          // no hint grid before the first stage: the first record
     float f[3] = {0, 0, 0};
     double x[3] = {0, 0, 0};
     for (int k = 0; k < D; ++k) {
