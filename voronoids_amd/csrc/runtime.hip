@@ -105,7 +105,6 @@ struct vo_tri {
     int tet0[4] = {0, 1, 2, 3};
     // points
     int64_t n_pts = 0, vcap = 0, head = 0;
-    std::vector<int32_t> input_of;     // point index -> input index
     double* X64 = nullptr;
     float* X32 = nullptr;
     int* cp = nullptr;
@@ -322,24 +321,88 @@ __global__ void __launch_bounds__(256) k_first_outside(const double* pts, int64_
     if (best != ~0ull) atomicMin(first, best);
 }
 
-// next window = pending losers followed by fresh points head .. head + nfresh - 1
-// staged points in priority order: slot i takes input point perm[i] (pts row-major, D columns);
-// X64 / X32 rows have stride S with the unused components 0, X32 = fl32(x - c) (the double
-// difference rounded once, as on the host), vmap = the point's reference vertex id
-__global__ void k_stage_points(const double* pts, const int32_t* perm, int64_t n, int D, int S, double c0, double c1,
-                               double c2, double* X64, float* X32, int* vmap, int64_t id0) {
-    const double cc[3] = {c0, c1, c2};
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t src = perm[i];
-        for (int k = 0; k < S; ++k) {
-            const double x = k < D ? pts[src * D + k] : 0.0;
-            X64[i * S + k] = x;
-            X32[i * S + k] = k < D ? (float)(x - cc[k]) : 0.0f;
+// ---------------------------------------------------------------- staging
+// The priority order (priority_order, a Fisher-Yates shuffle over splitmix64(seed)) without its
+// serial chain.  Step i (i = n - 1 down to 1) swaps positions i and j_i <= i, and j_i follows from
+// seed and i alone.  Nothing moves into or out of position i after step i, so
+//   perm[i] = the value at position j_i just before step i,
+// and a value sits at position q before step i if the last step to swap with q, the least step
+// s > i with j_s = q, put it there: then it is the value that was at position s before step s;
+// without such a step it is q itself.  That walk is one list search per hop: the steps with
+// j_s = q are linked at head[q] (about one per position, at most some tens at the lowest
+// positions), and an element takes about two hops.  The host's shuffle was a random pass over
+// its caches, one step after another; the whole stage 2D n = 10M 66 -> 7.5 ms, 3D n = 4M
+// 18 -> 4.2 ms, where the device's two kernels (2D n = 10M) are 1.6 ms and the upload the rest.
+__device__ __forceinline__ int shuffle_step(uint64_t seed, int64_t n, int64_t i) {
+    uint64_t z = seed + (uint64_t)(n - i) * 0x9E3779B97F4A7C15ull;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    z ^= z >> 31;
+    return (int)__umul64hi(z, (uint64_t)(i + 1));
+}
+__global__ void __launch_bounds__(256) k_shuffle_links(uint64_t seed, int64_t n, int* head, int* next) {
+    for (int64_t i = 1 + (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        next[i] = atomicExch(&head[shuffle_step(seed, n, i)], (int)i);
+}
+// the least step above i that swapped with position q, -1 if none did
+__device__ __forceinline__ int shuffle_above(const int* head, const int* next, int q, int i) {
+    int best = -1;
+    for (int s = head[q]; s >= 0; s = next[s])
+        if (s > i && (best < 0 || s < best)) best = s;
+    return best;
+}
+
+// Staged points in priority order: slot i takes input point perm[i], from the list in perm or
+// (perm null) from the links (head null: input order); pts row-major, D columns.  X64 / X32 rows
+// have stride S with the unused components 0, X32 = fl32(x - c) (the double difference rounded
+// once, as on the host), vmap = the point's reference vertex id, cp = no conflict pointer yet.
+// A first stage also empties the hint grid (cells; its first holds the first simplex).  Every
+// point is read by one lane: `bad`, if given, is set for a coordinate that is not finite.
+struct StagePlan {
+    const double* pts;
+    const int32_t* perm;
+    const int *head, *next;
+    uint64_t seed;
+    int64_t n, id0, cells;
+    int D, S;
+    double c[3];
+    double* X64;
+    float* X32;
+    int *vmap, *cp, *hint;
+    int* bad;
+};
+__global__ void __launch_bounds__(256) k_stage_points(StagePlan p) {
+    const int64_t i0 = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
+    for (int64_t i = i0; i < p.cells; i += stride) p.hint[i] = i == 0 ? 0 : -1;
+    for (int64_t i = i0; i < p.n; i += stride) {
+        int64_t src = i;
+        if (p.perm) src = p.perm[i];
+        else if (p.head) {
+            int q = i > 0 ? shuffle_step(p.seed, p.n, i) : 0;
+            for (int s = shuffle_above(p.head, p.next, q, (int)i); s >= 0; s = shuffle_above(p.head, p.next, q, q)) q = s;
+            src = q;
         }
-        vmap[i] = (int)(id0 + src);
+        bool ok = true;
+        for (int k = 0; k < p.S; ++k) {
+            const double x = k < p.D ? p.pts[src * p.D + k] : 0.0;
+            ok &= fabs(x) < INFINITY;
+            p.X64[i * p.S + k] = x;
+            p.X32[i * p.S + k] = k < p.D ? (float)(x - p.c[k]) : 0.0f;
+        }
+        p.vmap[i] = (int)(p.id0 + src);
+        p.cp[i] = -1;
+        if (!ok && p.bad) *p.bad = 1;
     }
 }
 
+// coordinates of the points in input order (out rows of D), from the vertex tables
+__global__ void __launch_bounds__(256) k_input_coords(const double* X64, const int* vmap, int64_t n, int D, int S, int id0,
+                                                      double* out) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        for (int k = 0; k < D; ++k) out[(int64_t)(vmap[i] - id0) * D + k] = X64[i * S + k];
+}
+
+// next window = pending losers followed by fresh points head .. head + nfresh - 1
 __global__ void k_window(int* win, const int* pend, int npend, int head, int nfresh) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < npend) win[i] = pend[i];
@@ -1876,7 +1939,6 @@ int vo_tri_reset(vo_tri* t, const double* pts, int64_t n) {
     // host state of an empty tree; the round counter goes on, so that every reservation key
     // of the new set is below the keys left in the records of the old one
     t->n_pts = t->head = 0;
-    t->input_of.clear();
     // records above the count stay fresh (all 0xFF: dead), which the allocation stripes rely on:
     // a chunk's unused slots lie below the count and must not look live
     if (t->n_tets > 1)
@@ -1916,62 +1978,87 @@ int vo_tri_stage(vo_tri* t, const double* pts, int64_t n, uint64_t seed) {
     if (n < 0 || (n > 0 && !pts)) return fail(VO_ERR_INVALID, "bad point buffer");
     if (n == 0) return 0;
     const int D = t->D, S = t->S, M = t->M;
-    for (int64_t i = 0; i < n * D; ++i)
-        if (!std::isfinite(pts[i])) return fail(VO_ERR_INVALID, "non-finite coordinate");
+    // (large sets are checked by the lanes that read them)
+    const bool dev_check = n >= kDeviceFrame;
+    if (!dev_check && !all_finite(pts, n * D)) return fail(VO_ERR_INVALID, "non-finite coordinate");
     VO_HIP(hipSetDevice(t->dev));
     int rc;
-    if ((rc = grow_points(t, t->n_pts + n))) return rc;
-    const std::vector<int32_t> perm =
-        t->local_order ? priority_order_local(D, pts, n, seed, t->c, t->r, t->local_order) : priority_order(n, seed);
-    // ids are committed (n_pts, input_of) only once every upload and allocation has succeeded,
-    // so that a failed stage leaves the handle as it was
-    const int64_t base_in = t->n_pts;
-    std::vector<int32_t> in_of(n);
-    for (int64_t i = 0; i < n; ++i) in_of[i] = (int32_t)(base_in + perm[i]);
-    const int64_t v0 = M + t->n_pts;
-    {
-        // the points as given and the order go up; the device puts them in order (a gather in
-        // random order costs the host ~190 ms at n = 4M, the device well under a millisecond)
-        DevBuf<double> dpts;
-        DevBuf<int32_t> dperm;
-        if ((rc = dev_alloc(&dpts.p, (size_t)n * D)) || (rc = dev_alloc(&dperm.p, (size_t)n))) return rc;
-        VO_HIP(hipMemcpyAsync(dpts.p, pts, sizeof(double) * (size_t)n * D, hipMemcpyHostToDevice, t->s));
-        VO_HIP(hipMemcpyAsync(dperm.p, perm.data(), sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, t->s));
-        const int grid = (int)std::min<int64_t>((n + 255) / 256, 4096);
-        hipLaunchKernelGGL(k_stage_points, dim3(grid), dim3(256), 0, t->s, dpts.p, dperm.p, n, D, S, t->c[0], t->c[1],
-                           D == 3 ? t->c[2] : 0.0, t->X64 + v0 * S, t->X32 + v0 * S, t->vmap + v0,
-                           (int64_t)(2 * M + base_in));
-        VO_HIP(hipGetLastError());
-        VO_HIP(hipStreamSynchronize(t->s));     // before the staging buffers are freed
+    // (room for half as many points again, so that points added one at a time do not move the tables each time)
+    if (t->n_pts + n > t->vcap &&
+        (rc = grow_points(t, std::max(t->n_pts + n, t->n_pts > 0 ? std::min(t->vcap * 3 / 2, (int64_t)INT32_MAX / 2 - M) : 0))))
+        return rc;
+    // vertex ids are committed (n_pts) only once every upload and allocation has succeeded, so
+    // that a failed stage leaves the handle as it was
+    const int64_t v0 = M + t->n_pts, n_after = t->n_pts + n;
+    Scratch mem(t);
+    StagePlan p = {};
+    double* dpts;
+    if ((rc = mem.get(&dpts, (size_t)n * D))) return rc;
+    VO_HIP(hipMemcpyAsync(dpts, pts, sizeof(double) * (size_t)n * D, hipMemcpyHostToDevice, t->s));
+    p.pts = dpts;
+    p.seed = seed;
+    p.n = n;
+    p.id0 = 2 * M + t->n_pts;
+    p.D = D;
+    p.S = S;
+    for (int k = 0; k < 3; ++k) p.c[k] = t->c[k];
+    p.X64 = t->X64 + v0 * S;
+    p.X32 = t->X32 + v0 * S;
+    p.vmap = t->vmap + v0;
+    p.cp = t->cp + t->n_pts;
+    const dim3 grid((unsigned)std::min<int64_t>((n + 255) / 256, 8192));
+    std::vector<int32_t> perm;
+    if (t->local_order) {
+        // (sorted on the host, so checked there first)
+        if (dev_check && !all_finite(pts, n * D)) return fail(VO_ERR_INVALID, "non-finite coordinate");
+        perm = priority_order_local(D, pts, n, seed, t->c, t->r, t->local_order);
+        int32_t* dperm;
+        if ((rc = mem.get(&dperm, (size_t)n))) return rc;
+        VO_HIP(hipMemcpyAsync(dperm, perm.data(), sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, t->s));
+        p.perm = dperm;
+    } else if (n > 1) {
+        int *head, *next;
+        if ((rc = mem.get(&head, (size_t)n)) || (rc = mem.get(&next, (size_t)n))) return rc;
+        VO_HIP(hipMemsetAsync(head, 0xFF, sizeof(int) * (size_t)n, t->s));
+        hipLaunchKernelGGL(k_shuffle_links, grid, dim3(256), 0, t->s, seed, n, head, next);
+        p.head = head;
+        p.next = next;
     }
-    VO_HIP(hipMemsetAsync(t->cp + t->n_pts, 0xFF, sizeof(int) * n, t->s));
-    const int64_t n_after = t->n_pts + n;
+    int bad = 0;
+    if (dev_check) {
+        if ((rc = mem.get(&p.bad, 1))) return rc;
+        VO_HIP(hipMemsetAsync(p.bad, 0, sizeof(int), t->s));
+    }
     // walk-start hints: grids of 2^l cells per axis over the bounding sphere's box, finest
     // level about 4 points a cell; level 0 holds the initial simplex
+    const int L = t->hinted ? t->hlevels : hint_levels(D, n_after);
     if (!t->hinted) {
-        const int L = hint_levels(D, n_after);
-        t->hlevels = L;
-        const int64_t cells = hint_cells(D, L);
-        for (int k = 0; k < 3; ++k) t->glo[k] = (float)(-t->r);
-        t->ginv = (float)(1.0 / (2.0 * t->r));
-        if (cells > t->hint_cap) {
+        p.cells = hint_cells(D, L);
+        if (p.cells > t->hint_cap) {
             hipFree(t->hint);
             t->hint = nullptr;
             t->hint_cap = 0;
-            if ((rc = dev_alloc(&t->hint, cells))) return rc;
-            t->hint_cap = cells;
+            if ((rc = dev_alloc(&t->hint, p.cells))) return rc;
+            t->hint_cap = p.cells;
         }
-        VO_HIP(hipMemsetAsync(t->hint, 0xFF, sizeof(int) * cells, t->s));
-        VO_HIP(hipMemsetAsync(t->hint, 0, sizeof(int), t->s));
+        p.hint = t->hint;
+    }
+    hipLaunchKernelGGL(k_stage_points, grid, dim3(256), 0, t->s, p);
+    VO_HIP(hipGetLastError());
+    if (dev_check) VO_HIP(hipMemcpyAsync(&bad, p.bad, sizeof(int), hipMemcpyDeviceToHost, t->s));
+    VO_HIP(hipStreamSynchronize(t->s));     // before the caller's buffer and the scratch go
+    if (bad) return fail(VO_ERR_INVALID, "non-finite coordinate");
+    if (!t->hinted) {
+        t->hlevels = L;
+        for (int k = 0; k < 3; ++k) t->glo[k] = (float)(-t->r);
+        t->ginv = (float)(1.0 / (2.0 * t->r));
         t->hinted = true;
     }
     // simplex capacity for everything staged (uniform data creates ~27 (3D) / 6 (2D) per point)
     choose_reuse(t, n_after - t->inserted - t->dups);
     const int64_t want = (int64_t)t->n_tets + records_per_point(t) * (n_after - t->inserted - t->dups) + 4096;
     if ((rc = grow_tets(t, want))) return rc;
-    VO_HIP(hipStreamSynchronize(t->s));
     t->n_pts = n_after;
-    t->input_of.insert(t->input_of.end(), in_of.begin(), in_of.end());
     return 0;
 }
 
@@ -2169,7 +2256,7 @@ static int canonical_radix(const vo_tri* t, CanonOut& out) {
     if (dn.own) hipFree(dn.p);
     dn.p = nullptr;
     const int first = 2 * M;
-    const int nb = std::max(1, bit_length((int64_t)t->input_of.size() - 1));
+    const int nb = std::max(1, bit_length(t->n_pts - 1));
     const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(4096, (nl + 255) / 256));
     // ---- simplices
     int64_t& nt = out.nt;
@@ -2325,8 +2412,11 @@ int run_check(vo_tri* t, int pairs, int64_t* out) {
 int vertex_of_id(const vo_tri* t, int64_t id) {
     const int64_t in = id - 2 * t->M;
     if (in < 0) return -1;
-    for (size_t i = 0; i < t->input_of.size(); ++i)
-        if (t->input_of[i] == in) return (int)(t->M + i);
+    std::vector<int> vm((size_t)t->n_pts);
+    if (vm.empty() || hipMemcpy(vm.data(), t->vmap + t->M, sizeof(int) * vm.size(), hipMemcpyDeviceToHost) != hipSuccess)
+        return -1;
+    for (size_t i = 0; i < vm.size(); ++i)
+        if (vm[i] == id) return (int)(t->M + i);
     return -1;
 }
 
@@ -2417,9 +2507,9 @@ int vo_tri_set_vertex(vo_tri* t, int64_t id, const double* coords, int records) 
     const int D = t->D, S = t->S;
     for (int k = 0; k < D; ++k)
         if (!std::isfinite(coords[k])) return fail(VO_ERR_INVALID, "non-finite coordinate");
+    VO_HIP(hipSetDevice(t->dev));
     const int vi = vertex_of_id(t, id);
     if (vi < 0) return fail(VO_ERR_INVALID, "no input point has vertex id " + std::to_string(id));
-    VO_HIP(hipSetDevice(t->dev));
     double x64[4] = {0, 0, 0, 0};
     float x32[4] = {0, 0, 0, 0};
     for (int k = 0; k < D; ++k) {
@@ -2596,12 +2686,17 @@ int vo_tri_vertices(const vo_tri* t, double* coords) {
         const int src = v < M ? v : (D == 3 ? (v == 2 * M - 1 ? 1 : 0) : v - M);   // ghosts copy super vertices
         for (int k = 0; k < D; ++k) coords[v * D + k] = t->sv[src][k];
     }
-    std::vector<double> x((size_t)t->n_pts * S);
-    if (t->n_pts)
-        VO_HIP(hipMemcpy(x.data(), t->X64 + (size_t)M * S, sizeof(double) * x.size(), hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < t->n_pts; ++i) {
-        const int64_t in = t->input_of[i];
-        for (int k = 0; k < D; ++k) coords[(2 * M + in) * D + k] = x[i * S + k];
+    if (t->n_pts) {
+        Scratch mem(t);
+        double* out;
+        int rc;
+        if ((rc = mem.get(&out, (size_t)t->n_pts * D))) return rc;
+        hipLaunchKernelGGL(k_input_coords, dim3((unsigned)std::min<int64_t>((t->n_pts + 255) / 256, 8192)), dim3(256), 0, t->s,
+                           t->X64 + (size_t)M * S, t->vmap + M, t->n_pts, D, S, 2 * M, out);
+        VO_HIP(hipGetLastError());
+        VO_HIP(hipMemcpyAsync(coords + (size_t)2 * M * D, out, sizeof(double) * (size_t)t->n_pts * D, hipMemcpyDeviceToHost,
+                              t->s));
+        VO_HIP(hipStreamSynchronize(t->s));
     }
     return 0;
 }
