@@ -73,11 +73,15 @@ template <int D, int G> constexpr int kGroupAC =
 
 // LDS list scans, four entries per ds_read_b128 (entries at or past n are ignored: they may
 // hold another point's values)
+// whether an entry's value >> SHIFT equals x
+template <int SHIFT>
 __device__ __forceinline__ bool lds_contains(const int* list, int n, int x) {
     const int4* q = reinterpret_cast<const int4*>(list);
     for (int j = 0; j < n; j += 4) {
         const int4 w = q[j >> 2];
-        if ((w.x == x) | ((j + 1 < n) & (w.y == x)) | ((j + 2 < n) & (w.z == x)) | ((j + 3 < n) & (w.w == x))) return true;
+        if (((w.x >> SHIFT) == x) | ((j + 1 < n) & ((w.y >> SHIFT) == x)) | ((j + 2 < n) & ((w.z >> SHIFT) == x)) |
+            ((j + 3 < n) & ((w.w >> SHIFT) == x)))
+            return true;
     }
     return false;
 }
@@ -95,12 +99,26 @@ __device__ __forceinline__ int lds_find(const int* list, int n, int x) {
     return -1;
 }
 
+// Cavity membership by a hash table in LDS (open addressing, -1 = free) instead of a scan of the
+// killed list.  A scan costs one dependent LDS read per four members, on every pass, and another
+// over the pass's own finds; a lookup is one read or two whatever the cavity's size, and the
+// inserting compare-and-swap sorts out the lanes that found the same simplex.  3D with 16 lanes or
+// more per point, whose cavities hold 16 simplices and up to 80 (with the queue of the search:
+// run at n = 4M 79.9 -> 74.4 ms, 10^5 18.1 -> 16.5 ms).  In 2D (3 simplices) and with 8
+// lanes or fewer (a table per point would take 8 KB and more of LDS per wavefront, and with it a
+// third of the wavefronts) the list is scanned.
+template <int D, int G> constexpr bool kCavityHash = D == 3 && G >= 16;
+template <int D, int G> constexpr int kHashSize = kCavityHash<D, G> ? 256 : 4;
+static_assert(VO_GROUP_KC3 + 64 <= 256, "a full killed list and one pass's finds fit the table");
+__device__ __forceinline__ int hash_slot(int n) { return (int)((unsigned)n * 0x9E3779B1u >> 24); }
+
 // LDS of one wavefront of the lane-group cavity search
 template <int D, int G> struct alignas(16) CavityLds {
     int4 adj[Group<G>::NG][kGroupAC<D, G>];   // adjacency of the first members of each point's cavity
     int4 na[64];                               // adjacency of each lane's candidate
-    int cav[Group<G>::NG][kGroupKC<D>];        // killed lists
-    int tmp[64];
+    int cav[Group<G>::NG][kGroupKC<D>];        // killed lists: simplex << 2 | the face it was entered by
+    int tab[Group<G>::NG][kHashSize<D, G>];    // members by hash
+    int tmp[kCavityHash<D, G> ? 4 : 64];
 };
 
 // One wavefront's share of a round's cavity searches: window slots it.off + kb + lane group for
@@ -117,7 +135,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
     static_assert(KC % 4 == 0, "int4 scans");
     constexpr int AC = kGroupAC<D, G>;
     auto& s_cav = L.cav;
-    auto& s_tmp = L.tmp;
+    [[maybe_unused]] auto& s_tmp = L.tmp;
     auto& s_adj = L.adj;
     auto& s_na = L.na;
     const Group<G> g;
@@ -258,33 +276,44 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
         if (s0 == SIGN_UNDECIDED) st = ST_DEFER;
         else if (s0 <= 0) { st = ST_DUP; if (lead) lc.dups++; }
     }
-    // ---- cavity: level-synchronous breadth-first search
+    // ---- cavity: breadth-first search.  The (member, face) pairs found so far form one queue,
+    // M of the first member and D of each further one, whose entry face leads back to a member; a
+    // pass takes the next G of them, across levels.
     // With abort_early every member is reserved when it is found; the value the reservation
     // replaced (kold) is examined one pass later, once that pass's loads have returned, so the
     // check adds no wait.  A value below the point's key is a higher-priority point of this round
     // (earlier rounds have larger keys): the point cannot win and stops searching.
-    int nk = 0, nf = 0, lo = 0, hi = 0, ci = 0;
+    constexpr bool HASH = kCavityHash<D, G>;
+    constexpr int HS = kHashSize<D, G>;
+    int nk = 0, nf = 0, ci = 0;
     bool bfs = st == ST_OK;
     unsigned long long kold = ~0ull;
+    if constexpr (HASH) {
+        for (int j = g.gl; j < HS / 4; j += G) reinterpret_cast<int4*>(L.tab[g.gid])[j] = make_int4(-1, -1, -1, -1);
+        __builtin_amdgcn_wave_barrier();
+    }
     if (bfs) {
         if (lead) {
-            s_cav[g.gid][0] = t;
+            s_cav[g.gid][0] = t << 2;
+            if constexpr (HASH) L.tab[g.gid][hash_slot(t)] = t;
             if (c.abort_early) kold = atomicMin(kres_p<D>(c, t), key);
         }
         nk = 1;
-        hi = 1;
     }
     __builtin_amdgcn_wave_barrier();
     while (__any(bfs)) {
-        const int items = bfs ? (hi - lo) * M : 0;
+        const int items = bfs ? M + D * (nk - 1) : 0;
         const int i = ci + g.gl;
         const bool valid = bfs && i < items;
-        int tet = 0, face = 0, n = -1, s = 0, nb = -1;
+        int tet = 0, face = 0, n = -1, s = 0, nb = -1, hs = 0;
         bool hull = false, test = false;
         if (valid) {
-            const int mi = lo + i / M;
-            tet = s_cav[g.gid][mi];
-            face = i % M;
+            // the first member's faces in order, a further one's from the face after its entry on
+            const int mi = i < M ? 0 : 1 + (i - M) / D;
+            const int e = s_cav[g.gid][mi];
+            tet = e >> 2;
+            face = i < M ? i : (e & 3) + 1 + (i - M) % D;
+            if (face >= M) face -= M;
             // the LDS entry, or past AC (rare: large cavities) the record's, read by a volatile
             // load: a plain one let the compiler merge the two addresses into one flat load,
             // slower than an LDS read on the common path
@@ -293,7 +322,17 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             hull = nb < 0;
             if (!hull) {
                 n = nb >> 2;
-                test = !lds_contains(s_cav[g.gid], nk, n);
+                if constexpr (HASH) {
+                    hs = hash_slot(n);
+                    int x = L.tab[g.gid][hs];
+                    while (x != -1 && x != n) {
+                        hs = (hs + 1) & (HS - 1);
+                        x = L.tab[g.gid][hs];
+                    }
+                    test = x == -1;
+                } else {
+                    test = !lds_contains<2>(s_cav[g.gid], nk, n);
+                }
                 if (test) {
                     F an[4];
                     int4 na;
@@ -306,9 +345,21 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
         const unsigned long long und = g.ballot(test && s == SIGN_UNDECIDED);
         const unsigned long long lostm = g.ballot(bfs && kold < key);
         bool isnew = test && s != SIGN_UNDECIDED && s > 0;
-        s_tmp[g.lane] = isnew ? n : -1;
-        __builtin_amdgcn_wave_barrier();
-        if (isnew && lds_contains(s_tmp + g.gid * G, g.gl, n)) isnew = false;
+        if constexpr (HASH) {
+            // (a lookup ended at the first free slot; another lane may have taken it since)
+            if (isnew) {
+                int old = atomicCAS(&L.tab[g.gid][hs], -1, n);
+                while (old != -1 && old != n) {
+                    hs = (hs + 1) & (HS - 1);
+                    old = atomicCAS(&L.tab[g.gid][hs], -1, n);
+                }
+                isnew = old == -1;
+            }
+        } else {
+            s_tmp[g.lane] = isnew ? n : -1;
+            __builtin_amdgcn_wave_barrier();
+            if (isnew && lds_contains<0>(s_tmp + g.gid * G, g.gl, n)) isnew = false;
+        }
         const bool isfac = valid && (hull || (test && s != SIGN_UNDECIDED && s <= 0));
         const unsigned long long newm = g.ballot(isnew), facm = g.ballot(isfac);
         const int cnew = __popcll(newm), cfac = __popcll(facm);
@@ -325,7 +376,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             } else {
                 if (isnew) {
                     const int at = nk + g.below(newm);
-                    s_cav[g.gid][at] = n;
+                    s_cav[g.gid][at] = nb;              // n << 2 | the face it shares with its finder
                     if (at < AC) s_adj[g.gid][at] = s_na[g.lane];
                     if (c.abort_early) kold = atomicMin(kres_p<D>(c, n), key);
                 }
@@ -340,20 +391,15 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
                 }
                 nk += cnew;
                 nf += cfac;
-                ci += G;
-                if (ci >= items) {
-                    lo = hi;
-                    hi = nk;
-                    ci = 0;
-                    if (lo == hi) bfs = false;
-                }
+                ci = min(ci + G, items);
+                if (ci >= M + D * (nk - 1)) bfs = false;
             }
         }
         __builtin_amdgcn_wave_barrier();
     }
     if (st == ST_OK) {
         for (int j = g.gl; j < nk; j += G) {
-            const int x = s_cav[g.gid][j];
+            const int x = s_cav[g.gid][j] >> 2;
             if (!c.abort_early) atomicMin(kres_p<D>(c, x), key);
             c.cav[(size_t)slot * c.kcap + (j)] = x;
         }
