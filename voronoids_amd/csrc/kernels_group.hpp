@@ -438,35 +438,36 @@ __global__ void __launch_bounds__(64, D == 3 ? VO_CAVITY_WAVES : VO_CAVITY_WAVES
     cavity_pass<D, G>(c, nwin, key_hi, slot_iter(c, nwin, Group<G>::NG), L);
 }
 
-// Partner of ridge k of facet j of a winner's cavity boundary (fv: the new simplices' vertex
-// tuples, p first, then the facet's D vertices): the ridge is the facet's vertices other than
-// fv[j][k]; the boundary of a cavity is a closed manifold, so exactly one other facet holds all
-// of the ridge.  Returns that facet and, in kk, the index (1..D) of its vertex off the ridge,
-// which is the face of its new simplex that the two new simplices share; -1 if none is found.
-// 3D: the tuple in LDS is the new simplex (p, f1, f2, f3); 2D: the facet (f1, f2) only
-// The scan reads four tuples per step (indices clamped to the list, so every read is in it)
-// before comparing, one LDS round trip per four facets.
-__device__ __forceinline__ int match_ridge(const int4* fv, int nf, int j, int k, int& kk) {
-    const int4 a = fv[j];
-    const int u = k == 1 ? a.z : a.y;
-    const int w = k == 3 ? a.z : a.w;
-    for (int j0 = 0; j0 < nf; j0 += 4) {
-        int4 o[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = fv[j0 + r < nf ? j0 + r : nf - 1];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int jj = j0 + r;
-            const bool hy = (o[r].y == u) | (o[r].y == w), hz = (o[r].z == u) | (o[r].z == w);
-            const bool hw = (o[r].w == u) | (o[r].w == w);
-            if (jj < nf && jj != j && (int)hy + (int)hz + (int)hw == 2) {
-                kk = !hy ? 1 : (!hz ? 2 : 3);
-                return jj;
-            }
-        }
+// Partners of the ridges of a winner's cavity boundary (fv: the new simplices' vertex tuples in
+// LDS, p first, then the facet's D vertices): ridge k of facet j is the facet's vertices other than
+// fv[j][k].  The boundary of a cavity is a closed manifold, so exactly one other facet holds all of
+// the ridge; its new simplex shares the face across the ridge.
+//
+// 3D: by a hash table of ridges (two entries per facet tuple, -1 = free; an entry is j * 3 + k - 1
+// of the ridge that came first).  Returns the entry of the ridge with the same two vertices, or -1
+// for the first of the two to come.  A scan of the facets reads up to nf tuples per ridge, 3 nf
+// ridges, 30 facets on average and up to 100: run at n = 4M 74.6 -> 66.8 ms, 10^5 16.6 -> 13.6 ms.
+template <int SIZE> __device__ __forceinline__ int match_ridge(const int4* fv, int* tab, int q) {
+    static_assert((SIZE & (SIZE - 1)) == 0, "a power of two");
+    const int4 a = fv[q / 3];
+    const int k = q % 3;
+    const int u = k == 0 ? a.z : a.y, w = k == 2 ? a.z : a.w;
+    const int lo = u < w ? u : w, hi = u < w ? w : u;
+    int h = (int)((((unsigned)lo * 0x9E3779B1u) ^ ((unsigned)hi * 0x85EBCA77u)) >> 16) & (SIZE - 1);
+    for (;;) {
+        const int o = atomicCAS(&tab[h], -1, q);
+        if (o == -1) return -1;
+        const int4 b = fv[o / 3];
+        const int m = o % 3;
+        const int bu = m == 0 ? b.z : b.y, bw = m == 2 ? b.z : b.w;
+        if ((bu == u && bw == w) || (bu == w && bw == u)) return o;
+        h = (h + 1) & (SIZE - 1);
     }
-    return -1;
 }
+// 2D (the facet (f1, f2), the ridge one vertex, about 6 facets): a scan, four tuples per step
+// (indices clamped to the list, so every read is in it) before comparing, one LDS round trip per
+// four facets.  Returns the partner facet and, in kk, the index (1..2) of its vertex off the
+// ridge, which is the face of its new simplex that the two new simplices share; -1 if none is found.
 __device__ __forceinline__ int match_ridge(const int2* fv, int nf, int j, int k, int& kk) {
     const int2 a = fv[j];
     const int u = k == 1 ? a.y : a.x;
@@ -591,6 +592,9 @@ __device__ __forceinline__ bool outside_next_star(const Ctx& c, int t, int i, in
 // LDS of one wavefront of the lane-group commit
 template <int D, int G> struct alignas(16) CommitLds {
     static constexpr int DW = (kGroupFC<D> * D + 31) / 32;   // one bit per (facet, ridge): internal face linked
+    // ridges by hash: a facet has 1.5 of them, so at most three quarters of the table fill
+    static constexpr int HS = D == 3 && kGroupMC<D, G> > 0 ? 2 * kGroupMC<D, G> : 4;
+    int tab[Group<G>::NG][HS];
     int fac[Group<G>::NG][kGroupFC<D>];                     // facet list, then the new simplices
     typename FacetTuple<D>::T fv[Group<G>::NG][kGroupMC<D, G> > 0 ? kGroupMC<D, G> : 1];   // facet tuples
     unsigned done[Group<G>::NG][DW];
@@ -779,27 +783,52 @@ __device__ __forceinline__ void commit_pass(const Ctx c, int nwin, unsigned long
         __builtin_amdgcn_wave_barrier();
         // phase 2: internal faces, one lane per (facet, ridge); each link is written from both
         // sides by the lane that finds it, and the other side's lane skips it when it comes later
-        for (int w = g.gl; w < DW; w += G) s_done[g.gid][w] = 0u;
-        __builtin_amdgcn_wave_barrier();
-        // matched in LDS: the facet sharing the ridge is the partner (no memory traffic)
-        for (int q = g.gl; nf <= MC && q < nf * D; q += G) {
-            if (s_done[g.gid][q >> 5] & (1u << (q & 31))) continue;
-            const int j = q / D, k = 1 + q % D;
-            int kk = 1;
-            const int jj = match_ridge(s_fv[g.gid], nf, j, k, kk);
-            const int Nj = reuse ? s_fac[g.gid][j] : base + j;
-            if (jj < 0) {
-                atomicOr(&c.st->err, ERR_WALK);
-                *a_ptr<D>(c, Nj, k) = -1;
-                continue;
+        // matched in LDS (no memory traffic)
+        if constexpr (D == 3) {
+            constexpr int HS = CommitLds<D, G>::HS;
+            int found = 0;
+            if (nf <= MC) {
+                for (int w = g.gl; w < HS / 4; w += G)
+                    reinterpret_cast<int4*>(L.tab[g.gid])[w] = make_int4(-1, -1, -1, -1);
+                __builtin_amdgcn_wave_barrier();
+                for (int q = g.gl; q < nf * D; q += G) {
+                    const int o = match_ridge<HS>(s_fv[g.gid], L.tab[g.gid], q);
+                    found += __popcll(g.ballot(o >= 0));
+                    if (o < 0) continue;
+                    const int j = q / D, k = 1 + q % D, jj = o / D, kk = 1 + o % D;
+                    const int Nj = reuse ? s_fac[g.gid][j] : base + j, Njj = reuse ? s_fac[g.gid][jj] : base + jj;
+                    *a_ptr<D>(c, Nj, k) = (Njj << 2) | kk;
+                    *a_ptr<D>(c, Njj, kk) = (Nj << 2) | k;
+                }
+                // (the lead took part in every step)
+                if (lead && 2 * found != nf * D) atomicOr(&c.st->err, ERR_WALK);
             }
-            const int Njj = reuse ? s_fac[g.gid][jj] : base + jj;
-            *a_ptr<D>(c, Nj, k) = (Njj << 2) | kk;
-            *a_ptr<D>(c, Njj, kk) = (Nj << 2) | k;
-            const int qq = jj * D + kk - 1;
-            atomicOr(&s_done[g.gid][qq >> 5], 1u << (qq & 31));
+        } else {
+            for (int w = g.gl; w < DW; w += G) s_done[g.gid][w] = 0u;
+            __builtin_amdgcn_wave_barrier();
+            for (int q = g.gl; nf <= MC && q < nf * D; q += G) {
+                if (s_done[g.gid][q >> 5] & (1u << (q & 31))) continue;
+                const int j = q / D, k = 1 + q % D;
+                int kk = 1;
+                const int jj = match_ridge(s_fv[g.gid], nf, j, k, kk);
+                const int Nj = reuse ? s_fac[g.gid][j] : base + j;
+                if (jj < 0) {
+                    atomicOr(&c.st->err, ERR_WALK);
+                    *a_ptr<D>(c, Nj, k) = -1;
+                    continue;
+                }
+                const int Njj = reuse ? s_fac[g.gid][jj] : base + jj;
+                *a_ptr<D>(c, Nj, k) = (Njj << 2) | kk;
+                *a_ptr<D>(c, Njj, kk) = (Nj << 2) | k;
+                const int qq = jj * D + kk - 1;
+                atomicOr(&s_done[g.gid][qq >> 5], 1u << (qq & 31));
+            }
         }
         // too many facets for the LDS tuples: rotate around the ridge through the killed simplices
+        if (D == 3 && nf > MC) {
+            for (int w = g.gl; w < DW; w += G) s_done[g.gid][w] = 0u;
+            __builtin_amdgcn_wave_barrier();
+        }
         for (int q = g.gl; nf > MC && q < nf * D; q += G) {
             if (s_done[g.gid][q >> 5] & (1u << (q & 31))) continue;
             const int j = q / D, k = 1 + q % D;
