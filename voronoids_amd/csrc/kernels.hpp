@@ -417,26 +417,6 @@ __device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readl
 
 // One atomic per wave per counter that any lane added to; all lanes of the wave must call this.
 // (The per-lane counts are 32-bit and so is their sum.)  The round kernels end with it: 17 sums of
-// 64-bit shuffles each, zero or not, were @@ of every round.
-// Inclusive prefix sum over the wavefront by DPP (row shifts within 16 lanes, then the rows'
-// last lanes broadcast onward): lane 63 has the total.  Every lane must be active.  A shuffle
-// goes through LDS; these stay in the vector ALU.
-template <int CTRL, int ROWS> __device__ __forceinline__ int dpp_add(int x) {
-    return x + __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xf, false);
-}
-__device__ __forceinline__ int wave_incl_scan(int x) {
-    x = dpp_add<0x111, 0xf>(x);        // row_shr:1, 2, 4, 8
-    x = dpp_add<0x112, 0xf>(x);
-    x = dpp_add<0x114, 0xf>(x);
-    x = dpp_add<0x118, 0xf>(x);
-    x = dpp_add<0x142, 0xa>(x);        // row_bcast:15 to rows 1 and 3
-    x = dpp_add<0x143, 0xc>(x);        // row_bcast:31 to rows 2 and 3
-    return x;
-}
-__device__ __forceinline__ int wave_total(int x) { return __builtin_amdgcn_readlane(wave_incl_scan(x), 63); }
-
-// One atomic per wave per counter that any lane added to; all lanes of the wave must call this.
-// (The per-lane counts are 32-bit and so is their sum.)  The round kernels end with it: 17 sums of
 // 64-bit shuffles each, zero or not, were 2 us of every launch (run at 3D n = 10^5
 // 13.5 -> 13.1 ms, 4M 66.8 -> 64.6, 2D n = 10M 31.0 -> 28.2).
 __device__ inline void flush_counters(Counters* c, const LocalCnt& l) {
