@@ -522,10 +522,8 @@ struct vo_engine {
     int abort_early = 1;               // as vo_tri_config "abort_early"
     int walk_budget = 0;               // as vo_tri_config "walk_budget"
     int reuse = 0;                     // as vo_tri_config "reuse" (0 or 1 here)
-    int2* fix = nullptr;               // shared facets of a round's winners (k_fix_shared)
     int outcome_flags = 1;             // as vo_tri_config "outcome_flags": lane-group commits write
     int* pflag = nullptr;              // per-slot outcomes (win_cap), appended by k_append_pending
-    int fix_cap = 0;
     float gamma0 = 0.2f;
     bool launched = false;
     int last_nwin = 0;
@@ -642,7 +640,7 @@ void engine_free(vo_engine* e) {
     void* ptrs[] = {e->a.X64, e->a.X32, e->a.cp, e->a.vmap, e->a.pset, e->a.rec, e->a.hint, e->a.sets,
                     e->win, e->pend[0], e->pend[1], e->cav, e->fac, e->fnb, e->nk, e->nf, e->status, e->big, e->cav1,
                     e->fac1, e->misc1, e->st, e->ctl, e->cnt, e->q, e->cache, e->ws, e->done, e->stage_d, e->out_d,
-                    e->fix, e->pflag};
+                    e->pflag};
     for (void* p : ptrs)
         if (p) hipFree(p);
     if (e->st_host) hipHostFree(e->st_host);
@@ -691,8 +689,7 @@ Ctx engine_ctx(vo_engine* e) {
     c.abort_early = e->abort_early;
     c.walk_budget = e->walk_budget;
     c.reuse = e->reuse;
-    c.fix = e->fix;
-    c.fix_cap = e->fix_cap;
+    c.shared = 1;
     c.M = e->M;
     c.win_cap = e->win_cap;
     c.kcap = e->kcap;
@@ -756,7 +753,7 @@ void launch_round_kernels(vo_engine* e, const Ctx& c, int G, int which) {
         const Ctx& c;
         int G, which, blocks;
         ~FixAfter() {
-            if (!which || G == 1 || c.reuse || !c.fix) return;
+            if (!which || G == 1 || !shared_facets(c)) return;
             if (e->D == 3) hipLaunchKernelGGL(k_fix_shared<3>, dim3(blocks), dim3(256), 0, e->s, c);
             else hipLaunchKernelGGL(k_fix_shared<2>, dim3(blocks), dim3(256), 0, e->s, c);
         }
@@ -1300,10 +1297,9 @@ int vo_engine_create(int hip_device, int dim, int64_t max_points, int64_t max_si
         (rc = dev_alloc(&E->misc1, 4)) || (rc = dev_alloc(&E->st, 1)) || (rc = dev_alloc(&E->ctl, 1)) ||
         (rc = dev_alloc(&E->cnt, kCntStripes)) || (rc = dev_alloc(&E->q, E->qcap)) ||
         (rc = dev_alloc(&E->cache, (size_t)E->cmask + 1)) || (rc = dev_alloc(&E->ws, (size_t)E->ws_threads * E->ws_cap)) ||
-        (rc = dev_alloc(&E->done, E->nslots)) || (rc = dev_alloc(&E->fix, (size_t)2 * E->win_cap)) ||
+        (rc = dev_alloc(&E->done, E->nslots)) ||
         (rc = dev_alloc(&E->pflag, E->win_cap)))
         return bail(rc);
-    E->fix_cap = 2 * E->win_cap;
     E->out_cap = (size_t)1 << 26;
     if ((rc = dev_alloc(&E->out_d, E->out_cap))) return bail(rc);
     if (hipHostMalloc((void**)&E->out_h, sizeof(int32_t) * E->out_cap) != hipSuccess)

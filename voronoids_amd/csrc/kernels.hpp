@@ -60,7 +60,7 @@ struct RoundState {
     alignas(256) int n_next_pending;  // losers and deferred points appended for the next window (a
                                       // round with outcome flags: from the statistics, round_totals)
     alignas(256) int n_q;             // exact-queue fill (may exceed capacity: excess dropped)
-    alignas(256) int n_fix;           // shared-facet links to repair after the commit (see Ctx::fix)
+    alignas(256) int n_fix;           // window slots of the round whose shared facets are to be linked
     unsigned int err;                 // sticky ERR_* bits
     int n_big;                        // points whose cavity outgrew the group kernel's LDS lists
     int n_nospace;                    // several sets: winners whose set had no simplex space left
@@ -163,9 +163,11 @@ struct Ctx {
     int filters;           // bit 0: FP32 tier on, bit 1: FP64 filter on (both on in production)
     int solo;              // the window holds one point: cavity membership is stamped in kres
     int reuse;             // lane-group commit: new simplices take the winner's killed records first
-    int2* fix;             // lane-group commit without reuse: a winner whose cavity touches a
-    int fix_cap;           // higher-priority one lists (new simplex, killed record << 2 | face) for
-                           // each shared facet; k_fix_shared links the two sides after the commit
+    int shared;            // lane-group commit without reuse: winners may share facets.  A winner
+                           // whose cavity touches a higher-priority one leaves (new simplex in fac,
+                           // killed record << 2 | face in fnb) for each shared facet at its slot's
+                           // lists, and their number in nf; k_fix_shared links the two sides after
+                           // the commit
     int abort_early;       // lane-group cavity search: reserve each member as it is found and stop
                            // once a reservation shows a higher-priority point of the round
     int walk_budget;       // lane-group cavity walk in windows of at least 64 points: a point that
@@ -1313,27 +1315,32 @@ __global__ void __launch_bounds__(256) k_check_pairs(Ctx c, int n, int nv, int4 
 // Round rule of the lane-group kernels.  Winners hold every kill; then either (shared facets)
 // a winner's cavity may touch a higher-priority winner's when the sphere test of the commit
 // admits it, the links across such facets being set by k_fix_shared, or (stricter, with record
-// reuse, or with no shared-facet list) the cavities of winners are also pairwise non-adjacent,
+// reuse, or with shared facets off) the cavities of winners are also pairwise non-adjacent,
 // which the commit checks through outside reservations (nres).
-__device__ __forceinline__ bool shared_facets(const Ctx& c) { return !c.reuse && c.fix != nullptr; }
+__host__ __device__ __forceinline__ bool shared_facets(const Ctx& c) { return !c.reuse && c.shared; }
 
 // ---------------------------------------------------------------- k_fix_shared
 // Links across the facets shared by two winners of a round (a lower-priority winner W next to a
 // higher-priority cavity, admitted by the commit's sphere test).  W built its new simplex N on
-// the facet without linking it, and listed (N, A << 2 | face) with A its killed simplex on the
-// facet.  Whatever is across that face of A now is N's neighbor: the higher-priority winner's
-// new simplex on the facet (its outside patch landed in A, which only it writes there), or, when
-// that point did not win, the old simplex across the facet, which nobody patched.  One thread per
-// entry; the two ends are set here, after every commit of the round has finished.
+// the facet without linking it, and left (N, A << 2 | face) at its window slot with A its killed
+// simplex on the facet.  Whatever is across that face of A now is N's neighbor: the higher-priority
+// winner's new simplex on the facet (its outside patch landed in A, which only it writes there),
+// or, when that point did not win, the old simplex across the facet, which nobody patched.  Four
+// lanes per slot; the two ends are set here, after every commit of the round has finished.
+// (One list for all winners needs a returning atomic on its length per winner, 11 ns each, one
+// after another: run at 2D n = 10M 28.4 -> 25.0 ms without it, 1M 7.6 -> 6.75, 3D n = 4M
+// 64.5 -> 64.1.)
 template <int D>
 __device__ __forceinline__ void fix_shared_pass(const Ctx& c, int first, int stride) {
-    const int n = min(c.st->n_fix, c.fix_cap);
-    for (int e = first; e < n; e += stride) {
-        const int2 f = c.fix[e];
-        if (f.x < 0) continue;                  // reserved by a point that then did not win
-        const int X = *a_ptr<D>(c, f.y >> 2, f.y & 3);
-        *a_ptr<D>(c, f.x, 0) = X;
-        if (X >= 0) *a_ptr<D>(c, X >> 2, X & 3) = f.x << 2;
+    const int n = 4 * c.st->n_fix;
+    for (int i = first; i < n; i += stride) {
+        const int slot = i >> 2, m = c.nf[slot];
+        for (int r = i & 3; r < m; r += 4) {
+            const int N = c.fac[(size_t)slot * c.fcap + r], fe = c.fnb[(size_t)slot * c.fcap + r];
+            const int X = *a_ptr<D>(c, fe >> 2, fe & 3);
+            *a_ptr<D>(c, N, 0) = X;
+            if (X >= 0) *a_ptr<D>(c, X >> 2, X & 3) = N << 2;
+        }
     }
 }
 template <int D>

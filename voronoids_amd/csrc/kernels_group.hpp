@@ -425,11 +425,10 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
 template <int D, int G>
 __global__ void __launch_bounds__(64, D == 3 ? VO_CAVITY_WAVES : VO_CAVITY_WAVES2) k_cavity_g(Ctx c, int nwin, unsigned long long key_hi) {
     __shared__ CavityLds<D, G> L;
-    // the shared-facet list starts empty for this round's commit (the launch before this one
-    // applied the previous round's)
     round_params(c, nwin, key_hi);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        c.st->n_fix = 0;
+        // the slots whose shared facets the launch after this round's commit links
+        c.st->n_fix = shared_facets(c) ? nwin : 0;
         // the slots whose outcomes this round's commit writes to pflag, for the next planning
         // launch; an empty round (after a planner halt) keeps the last compaction's count
         c.st->flag_n = c.pflag ? nwin : 0;
@@ -696,22 +695,7 @@ __device__ __forceinline__ void commit_pass(const Ctx c, int nwin, unsigned long
         }
         ok = ok && pass;
     }
-    bool win = st == ST_OK && g.ballot(!ok) == 0;
-    // entries of the shared-facet list, reserved by the lead; a full list makes the point wait
-    int fix_base = 0;
-    if (refined) {
-        int fb = 0;
-        if (win && lead && nsh > 0) {
-            fb = atomicAdd(&c.st->n_fix, nsh);
-            if (fb + nsh > c.fix_cap) {
-                for (int e2 = fb; e2 < c.fix_cap; ++e2) c.fix[e2] = make_int2(-1, -1);
-                fb = -1;
-            }
-        }
-        fb = g.bcast(fb, 0);
-        win = win && fb >= 0;
-        fix_base = fb;
-    }
+    const bool win = st == ST_OK && g.ballot(!ok) == 0;
     // Slots.  With reuse (and the facet tuples within the LDS match list), facet j's new simplex
     // takes the winner's killed record j for j < nr = min(nk, nf) and a fresh slot past that, so
     // that records stay about as many as live simplices and new ones land on lines the round has
@@ -720,8 +704,6 @@ __device__ __forceinline__ void commit_pass(const Ctx c, int nwin, unsigned long
     const int nr = reuse ? (nk < nf ? nk : nf) : 0;
     const int base = g.bcast(alloc_slots(c, win && lead, nf - nr, p), 0);
     const bool build = win && base >= 0;
-    if (refined && win && !build && lead)
-        for (int e2 = 0; e2 < nsh; ++e2) c.fix[fix_base + e2] = make_int2(-1, -1);
     // a winner's check loops ran to completion, so s_fac holds its whole facet list
     __builtin_amdgcn_wave_barrier();
     const int pv = c.M + p;
@@ -753,8 +735,8 @@ __device__ __forceinline__ void commit_pass(const Ctx c, int nwin, unsigned long
             __builtin_amdgcn_wave_barrier();
         }
         // phase 1: the new simplex of facet j, its outside link and the outside neighbor's patch;
-        // a shared facet (marked) is left unlinked and listed for k_fix_shared instead, and its
-        // mark is cleared for the lookups that follow
+        // a shared facet (marked) is left unlinked and noted for k_fix_shared instead, over the
+        // slot's lists (which LDS holds), and its mark is cleared for the lookups that follow
         int run = 0;
         for (int j0 = 0; !reuse && j0 < nf; j0 += G) {
             const int j = j0 + g.gl;
@@ -773,8 +755,11 @@ __device__ __forceinline__ void commit_pass(const Ctx c, int nwin, unsigned long
                 st_v<D>(c, N, nv);
                 store_star_coords<D>(c, xs, i, pf, N);
                 *a_ptr<D>(c, N, 0) = outside;
-                if (sh) c.fix[fix_base + run + g.below(shm)] = make_int2(N, fe);
-                else if (outside >= 0) *a_ptr<D>(c, outside >> 2, outside & 3) = N << 2;
+                if (sh) {
+                    const size_t fi = (size_t)slot * c.fcap + run + g.below(shm);
+                    c.fac[fi] = N;
+                    c.fnb[fi] = fe;
+                } else if (outside >= 0) *a_ptr<D>(c, outside >> 2, outside & 3) = N << 2;
                 if (nf <= MC) facet_tuple(s_fv[g.gid][j], nv);
                 if (sh) s_fac[g.gid][j] = fe;
             }
@@ -907,6 +892,7 @@ __device__ __forceinline__ void commit_pass(const Ctx c, int nwin, unsigned long
         q[1] = make_uint4((unsigned)nk, (unsigned)nf, 0u, 0u);
     }
 #endif
+    if (refined && lead && valid) c.nf[slot] = build ? nsh : 0;
     // cavities too large for the LDS lists are re-run alone after the round
     const bool big = lead && st == ST_OVERFLOW;
     bool again = lead && ((st == ST_OK && !build) || st == ST_DEFER || st == ST_LOST);

@@ -187,8 +187,6 @@ struct vo_tri {
     int reuse = -1;                    // new simplices take their winner's killed records first: 1 on,
                                        // 0 off, -1 only when append-only records would pass 2^29
     int reuse_on = 0;                  // this run's choice
-    int2* fix = nullptr;               // shared facets of the round's winners (k_fix_shared)
-    int fix_cap = 0;
     int shared_facets = 1;             // 0: the stricter rule (winners' cavities never adjacent)
     int min_window = 64;               // least points per round (8 measured ~2% slower at 3D 4M / 2D 10M)
     int64_t small_run = 64;            // runs of at most this many points use the host loop
@@ -244,8 +242,7 @@ Ctx make_ctx(const vo_tri* t) {
     c.abort_early = t->abort_early;
     c.walk_budget = t->walk_budget;
     c.reuse = t->reuse_on;
-    c.fix = t->shared_facets ? t->fix : nullptr;
-    c.fix_cap = t->fix_cap;
+    c.shared = t->shared_facets;
     c.win_cap = t->win_cap;
     c.kcap = t->kcap;
     c.fcap = t->fcap;
@@ -480,8 +477,8 @@ __global__ void k_add_offsets(int* out, const int* boff, int n) {
 }
 
 
-// the lists a device-planned chunk starts from are complete: no planning launch may apply the
-// shared-facet list or compact the outcome flags of a round finished before it
+// what a device-planned chunk starts from is complete: no planning launch may link the shared
+// facets or compact the outcome flags of a round finished before it
 __global__ void k_clear_fix(RoundState* st) {
     st->n_fix = 0;
     st->flag_n = 0;
@@ -509,13 +506,13 @@ __global__ void __launch_bounds__(kCntStripes) k_round_totals(const Counters* cn
 __device__ void plan_step(RunPlan& p, RoundState* st, bool absorb);
 
 // Block 0 plans the next round; blocks 1.. link the facets the last round's winners share (the
-// shared-facet list, as k_fix_shared) and compact its outcome flags into pend_dst, the pending
-// list of the next window (with Ctx::pflag).  The planner reads neither: one launch for all.
-// The list count is cleared by the next cavity kernel, which every planning launch precedes.
+// notes at the window's slots, as k_fix_shared) and compact its outcome flags into pend_dst, the
+// pending list of the next window (with Ctx::pflag).  The planner reads neither: one launch for all.
+// The next cavity kernel, which every planning launch precedes, sets the slot count of its round.
 template <int D>
 __global__ void __launch_bounds__(256) k_plan_one(RunPlan* P, Ctx c, const Counters* cnt, int* pend_dst) {
     if (blockIdx.x > 0) {
-        if (!c.reuse && c.fix) fix_shared_pass<D>(c, (blockIdx.x - 1) * blockDim.x + threadIdx.x, (gridDim.x - 1) * blockDim.x);
+        if (shared_facets(c)) fix_shared_pass<D>(c, (blockIdx.x - 1) * blockDim.x + threadIdx.x, (gridDim.x - 1) * blockDim.x);
         // the last round's outcome flags (st->flag_n slots) into the next window's pending list
         if (c.pflag)
             append_flagged(c.pflag, c.st->flag_n, pend_dst, c.pend_cap, &c.st->n_compact, &c.st->err, blockIdx.x - 1,
@@ -659,13 +656,14 @@ __global__ void __launch_bounds__(64 * kBootWaves<D>) k_boot(Ctx c, RunPlan* P, 
         c.pend_next = p.cur ? pend0 : pend1;
         cavity_pass<D, G>(c, nwin, key_hi, SlotIter{w * Group<G>::NG, NW * Group<G>::NG, nwin, 0}, U.cav[w]);
         __syncthreads();
+        if (threadIdx.x == 0) c.st->n_fix = shared_facets(c) ? nwin : 0;
         commit_pass<D, G>(c, nwin, key_hi, SlotIter{w * Group<G>::NG, NW * Group<G>::NG, nwin, 0}, U.com[w]);
         __syncthreads();
-        if (!c.reuse && c.fix) {
+        if (shared_facets(c)) {
             fix_shared_pass<D>(c, threadIdx.x, blockDim.x);
             __syncthreads();
         }
-        if (threadIdx.x == 0) c.st->n_fix = 0;     // applied: the next round's commit starts a new list
+        if (threadIdx.x == 0) c.st->n_fix = 0;     // linked
     }
     if (threadIdx.x == 0) {
         p.halt &= ~HALT_BOOT;
@@ -774,7 +772,7 @@ void free_all(vo_tri* t) {
     void* ptrs[] = {t->X64, t->X32, t->cp, t->vmap, t->rec, t->rec_spare, t->cmap, t->chist, t->reg_meta, t->win2,
                     t->regs, t->win, t->pend[0], t->pend[1],
                     t->cav, t->fac, t->fnb, t->nk, t->nf, t->status, t->hint, t->st, t->cnt, t->q, t->cache, t->ws,
-                    t->big, t->cav1, t->fac1, t->misc1, t->plan, t->fix, t->ast, t->pflag};
+                    t->big, t->cav1, t->fac1, t->misc1, t->plan, t->ast, t->pflag};
     for (void* p : ptrs)
         if (p) hipFree(p);
 #ifdef VO_POINT_PROBE
@@ -1016,7 +1014,7 @@ int launch_round(vo_tri* t, const Ctx& c, int nwin, unsigned long long key_hi, i
     VO_HIP(hipGetLastError());
     // links across the facets two winners share (only without reuse; the thread commit keeps to
     // disjoint, non-adjacent cavities)
-    if (fix && which && G != 1 && !c.reuse && c.fix) {
+    if (fix && which && G != 1 && shared_facets(c)) {
         const int fb = std::max(1, std::min(1024, nwin / 64 + 1));
         if (t->D == 3) hipLaunchKernelGGL(k_fix_shared<3>, dim3(fb), dim3(256), 0, t->s, c);
         else hipLaunchKernelGGL(k_fix_shared<2>, dim3(fb), dim3(256), 0, t->s, c);
@@ -1366,7 +1364,7 @@ int run_device_planned(vo_tri* t) {
     const bool flags = t->outcome_flags && !t->reuse_on && t->shared_facets && t->group != 1;
     while (t->head < t->n_pts || t->npend > 0) {
         if (t->npend > t->win_cap) return fail(VO_ERR_INTERNAL, "pending list beyond the window capacity");
-        // the shared-facet list and outcome flags of a round finished before this point are
+        // the shared facets and outcome flags of a round finished before this point are
         // applied already; the first planning launch must not apply them again (the cavity
         // kernels clear the counts after that)
         hipLaunchKernelGGL(k_clear_fix, dim3(1), dim3(1), 0, t->s, t->st);
@@ -1428,7 +1426,7 @@ int run_device_planned(vo_tri* t) {
                 if (flags) c.pflag = t->pflag;
                 // the plan, with the previous round's shared-facet links (the thread kernels of
                 // group_lanes 1 leave none) and pending list
-                const int fixb = (!c.reuse && c.fix && t->group != 1) ? std::max(1, std::min(1024, est_hi / 64 + 1)) : 0;
+                const int fixb = (shared_facets(c) && t->group != 1) ? std::max(1, std::min(1024, est_hi / 64 + 1)) : 0;
                 if (D == 3)
                     hipLaunchKernelGGL(k_plan_one<3>, dim3(1 + fixb), dim3(256), 0, t->s, t->plan, c, t->cnt, t->pend[cur]);
                 else
@@ -1897,10 +1895,9 @@ int vo_tri_create(int hip_device, int dim, const double* pts, int64_t n, vo_tri*
         (rc = dev_alloc(&t->cache, (size_t)t->cmask + 1)) || (rc = dev_alloc(&t->ws, (size_t)t->ws_threads * t->ws_cap)) ||
         (rc = dev_alloc(&t->big, t->win_cap)) || (rc = dev_alloc(&t->cav1, t->big_cap)) ||
         (rc = dev_alloc(&t->fac1, t->big_cap)) || (rc = dev_alloc(&t->misc1, 4)) ||
-        (rc = dev_alloc(&t->fix, (size_t)2 * t->win_cap)) || (rc = dev_alloc(&t->ast, kAllocStripes)) ||
+        (rc = dev_alloc(&t->ast, kAllocStripes)) ||
         (rc = dev_alloc(&t->pflag, t->win_cap)))
         return bail(rc);
-    t->fix_cap = 2 * t->win_cap;
     if ((rc = point_frame(t, pts, n, t->c, &t->r))) return bail(rc);
     t->R = t->r * 10.0;
     super_vertices(dim, t->c, t->R, t->sv);
