@@ -110,6 +110,8 @@ struct BatchCtl {
     int min_window;        // least fresh window of a set per round
     int big_window;        // windows at least this large aim at a higher winning fraction
     int slots;             // set slots that may be in use: one past the highest (host, before each replay)
+    int ahead;             // fresh points after the window that may be walked ahead (one set; see
+                           // kAheadWaves)
     int virt, vhead;       // virt = 1: the window is not written out: slots below npend are the
                            // pending list (Ctx::win), slot i >= npend is point vhead + i - npend
 };
@@ -704,8 +706,8 @@ template <int D> __device__ int conflict_slow(const Ctx& c, int4 v, int pv, Loca
     return SIGN_UNDECIDED;
 }
 
-// tiers 2 and 3 of an orientation test on vertex ids
-template <int D> __device__ int orient_slow(const Ctx& c, const int* ids, LocalCnt& lc) {
+// tiers 2 and 3 of an orientation test on vertex ids (queue false: tier 2 only, nothing queued)
+template <int D> __device__ int orient_slow(const Ctx& c, const int* ids, LocalCnt& lc, bool queue = true) {
     constexpr int S = VT<D>::S;
     const double* X = c.X64;
     int s = SIGN_UNDECIDED;
@@ -714,6 +716,7 @@ template <int D> __device__ int orient_slow(const Ctx& c, const int* ids, LocalC
         else s = t2_orient2d(X + S * ids[0], X + S * ids[1], X + S * ids[2]);
         if (s != SIGN_UNDECIDED) { lc.t2[0]++; return s; }
     }
+    if (!queue) return SIGN_UNDECIDED;
     uint32_t u[5] = {(uint32_t)ids[0], (uint32_t)ids[1], (uint32_t)ids[2], D == 3 ? (uint32_t)ids[3] : kEmpty, kEmpty};
     const uint32_t type = D == 3 ? PRED_ORIENT3 : PRED_ORIENT2;
     s = cache_lookup(c.cache, c.cmask, type, u);
@@ -739,7 +742,8 @@ template <int D> __device__ __forceinline__ int conflict_at(const Ctx& c, const 
 // orientation of simplex t (coordinates a[]) with vertex k replaced by p: < 0 means p lies
 // beyond face k
 template <int D> __device__ __forceinline__ int orient_at(const Ctx& c, const typename VT<D>::F* a, int t, int k,
-                                                          int pv, typename VT<D>::F pf, LocalCnt& lc) {
+                                                          int pv, typename VT<D>::F pf, LocalCnt& lc,
+                                                          bool queue = true) {
     if (c.filters & 1) {
         typename VT<D>::F b[4];
         for (int i = 0; i < D + 1; ++i) b[i] = i == k ? pf : a[i];
@@ -751,7 +755,7 @@ template <int D> __device__ __forceinline__ int orient_at(const Ctx& c, const ty
     const int4 v = ld_v<D>(c, t);
     int ids[4] = {v.x, v.y, v.z, v.w};
     ids[k] = pv;
-    return orient_slow<D>(c, ids, lc);
+    return orient_slow<D>(c, ids, lc, queue);
 }
 
 // coordinate record of replace_first(v, i, p) from the old record ox: p first, then the old

@@ -121,9 +121,26 @@ template <int D, int G> struct alignas(16) CavityLds {
     int tmp[kCavityHash<D, G> ? 4 : 64];
 };
 
+// Walking ahead.  A small round takes as long as its slowest point, and that is one whose walk
+// started far away: of some hundred fresh points a few walk 30 to 70 steps of 1 us each, where the
+// median walks 3 and its search takes 10 us.  A device-planned window is therefore followed by
+// slots of the fresh points that come after it, up to twice as many as the window has: they walk at
+// most kAheadSteps from where they are, write only their conflict pointer (and the hint of a walk
+// that ended) and search nothing.  When their round comes they are a step or two away.  The tree
+// does not change while this kernel runs, and a point's walk has no part in which points win, so
+// rounds and windows are the same with and without.  Only as many as make
+// up kAheadWaves wavefronts with the window's: a window that fills the chip is bound by its work,
+// and a walk split in two costs a few loads more.  Run at 3D n = 10^4 8.1 -> 6.8 ms, 10^5
+// 12.8 -> 11.1, 4M 63.8 -> 62.4, clustered 10^6 50.6 -> 47.6, 2D n = 10^6 6.9 -> 6.6.  (Steps 8 or
+// 24: 1% slower at 10^5.  Wavefronts: 3,072 in 3D leave clustered points at 48.5, 8,192 in 2D cost
+// 1%.  Four times the window instead of twice: the same.)
+template <int D> constexpr int kAheadWaves = D == 3 ? 8192 : 3072;
+constexpr int kAheadSteps = 12;
+
 // One wavefront's share of a round's cavity searches: window slots it.off + kb + lane group for
-// kb = it.base, it.base + it.stride, ... below it.lim.  Run by k_cavity_g (one wavefront per
-// block) and by the one-workgroup early-round kernel (one share per wavefront).
+// kb = it.base, it.base + it.stride, ... below it.lim; slots from nwin on walk ahead.  Run by
+// k_cavity_g (one wavefront per block) and by the one-workgroup early-round kernel (one share per
+// wavefront).
 template <int D, int G>
 __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long long key_hi, const SlotIter it,
                                             CavityLds<D, G>& L) {
@@ -144,6 +161,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
     const WinView wv = win_view(c);
     for (int kb = it.base; kb < it.lim; kb += it.stride) {
     const int slot = it.off + kb + g.gid;
+    const bool pre = slot >= nwin;         // (with XCD regions slots are below nwin, too)
     const bool valid = kb + g.gid < it.lim;
     int st = valid ? ST_OK : ST_IDLE;
     int p = 0, pv = 0, t = 0;
@@ -198,7 +216,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
     // resumes from there next round (only in windows of 64 or more, whose other points progress)
     bool walking = st == ST_OK;
     bool paused = false;
-    const int budget = (c.walk_budget > 0 && nwin >= 64) ? c.walk_budget : 0x7fffffff;
+    const int budget = pre ? kAheadSteps : (c.walk_budget > 0 && nwin >= 64) ? c.walk_budget : 0x7fffffff;
     int came = -1;
     uint32_t rng = mix32((uint32_t)p * 0x9E3779B9u + 0x632BE5ABu);
     F a[4];
@@ -224,7 +242,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             if (g.gl < M) {
                 nb = comp(aa, k);
                 test = !(nb >= 0 && (nb >> 2) == came);
-                if (test) s = orient_at<D>(c, a, t, k, pv, pf, lc);
+                if (test) s = orient_at<D>(c, a, t, k, pv, pf, lc, !pre);
             }
         }
         const unsigned long long und = g.ballot(test && s == SIGN_UNDECIDED);
@@ -242,7 +260,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             } else if (!neg) {
                 walking = false;
             } else if (nb_sel < 0 || step > kWalkLimit) {
-                if (lead) atomicOr(&c.st->err, nb_sel < 0 ? ERR_HULL : ERR_WALK);
+                if (lead && !pre) atomicOr(&c.st->err, nb_sel < 0 ? ERR_HULL : ERR_WALK);
                 st = ST_BROKEN;
                 walking = false;
             } else {
@@ -257,14 +275,15 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             }
         }
     }
-    if (st == ST_OK || st == ST_DEFER) {
+    if (st == ST_OK || (st == ST_DEFER && !pre)) {
         if (lead) {
             c.cp[p] = t;
             hint_store<D>(hint_view(c, p), pf, a, t);
         }
-    } else if (paused && lead) {
+    } else if ((paused || (st == ST_DEFER && pre)) && lead) {
         c.cp[p] = t;          // no hint: t need not be near p
     }
+    if (pre) st = ST_IDLE;
 #ifdef VO_POINT_PROBE
     pr_tw = (unsigned)(wall_clock64() - pr_t0);
 #endif
@@ -404,7 +423,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             c.cav[(size_t)slot * c.kcap + (j)] = x;
         }
     }
-    if (valid && lead) {
+    if (valid && lead && !pre) {
         c.nk[slot] = nk;
         c.nf[slot] = nf;
         c.status[slot] = st;
@@ -434,7 +453,9 @@ __global__ void __launch_bounds__(64, D == 3 ? VO_CAVITY_WAVES : VO_CAVITY_WAVES
         c.st->flag_n = c.pflag ? nwin : 0;
         if (nwin > 0) c.st->n_compact = 0;
     }
-    cavity_pass<D, G>(c, nwin, key_hi, slot_iter(c, nwin, Group<G>::NG), L);
+    int slots = nwin;
+    if (c.ctl && c.ctl->virt) slots += max(0, min(c.ctl->ahead, kAheadWaves<D> * Group<G>::NG - nwin));
+    cavity_pass<D, G>(c, nwin, key_hi, slot_iter(c, slots, Group<G>::NG), L);
 }
 
 // Partners of the ridges of a winner's cavity boundary (fv: the new simplices' vertex tuples in

@@ -550,6 +550,7 @@ __global__ void __launch_bounds__(256) k_plan_one(RunPlan* P, Ctx c, const Count
 
 __device__ void plan_step(RunPlan& p, RoundState* st, bool s_absorb) {
     p.ctl.nwin = 0;
+    p.ctl.ahead = 0;
     if (p.launched) {
         if (!s_absorb) {
             p.halt |= HALT_HOST;
@@ -599,6 +600,7 @@ __device__ void plan_step(RunPlan& p, RoundState* st, bool s_absorb) {
     p.chunk = (int)chunk;
     p.ctl.nwin = nwin;
     p.ctl.npend = p.npend;
+    p.ctl.ahead = min(p.n_pts - p.head - nfresh, 2 * nwin);
     p.ctl.virt = 1;            // pending points, then fresh points head .. (not written out)
     p.ctl.vhead = p.head;
     p.ctl.key_hi = (unsigned long long)(0xFFFFFFFFu - (uint32_t)p.rounds) << 32;
@@ -1433,7 +1435,10 @@ int run_device_planned(vo_tri* t) {
                     hipLaunchKernelGGL(k_plan_one<2>, dim3(1 + fixb), dim3(256), 0, t->s, t->plan, c, t->cnt, t->pend[cur]);
                 hipEvent_t* e = &t->rev[(size_t)(slot * R + r) * 3];
                 if (t->round_timing) VO_HIP(hipEventRecord(e[0], t->s));
-                if ((rc = launch_round(t, c, est_hi, 0, 0, Gc))) return rc;
+                // (the cavity search's blocks cover the points walked ahead, too)
+                const int per_wave = 64 / std::max(Gc, 4), most = (D == 3 ? kAheadWaves<3> : kAheadWaves<2>) * per_wave;
+                const int slots = std::max(est_hi, std::min(3 * est_hi, most));
+                if ((rc = launch_round(t, c, slots, 0, 0, Gc))) return rc;
                 if (t->round_timing) VO_HIP(hipEventRecord(e[1], t->s));
                 if ((rc = launch_round(t, c, est_hi, 0, 1, Gm, false))) return rc;
                 if (t->round_timing) VO_HIP(hipEventRecord(e[2], t->s));
