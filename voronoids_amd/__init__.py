@@ -28,7 +28,7 @@ import numpy as np
 
 from . import _lib
 from ._lib import VoError, VoStats
-from .batch import Engine, Server, SetResult, batch_triangulate
+from .batch import Engine, Server, SetResult, _rows, batch_triangulate
 
 __all__ = ["DelaunayTree", "PyDelauanyTree", "PyVertex", "PySimplex", "delaunay", "VoError", "Engine", "Server",
            "SetResult", "batch_triangulate"]
@@ -168,13 +168,7 @@ class DelaunayTree:
         nT, nE = ctypes.c_int64(), ctypes.c_int64()
         L = _lib.lib()
         _lib.check(L.vo_tri_canonical(self._h, ctypes.byref(T), ctypes.byref(nT), ctypes.byref(E), ctypes.byref(nE)))
-        try:
-            Ta = np.ctypeslib.as_array(T, shape=(max(nT.value, 1) * self.M,))[: nT.value * self.M].copy()
-            Ea = np.ctypeslib.as_array(E, shape=(max(nE.value, 1) * 2,))[: nE.value * 2].copy()
-        finally:
-            L.vo_free(ctypes.cast(T, ctypes.c_void_p))
-            L.vo_free(ctypes.cast(E, ctypes.c_void_p))
-        return Ta.reshape(-1, self.M), Ea.reshape(-1, 2)
+        return _rows(T, nT.value, self.M), _rows(E, nE.value, 2)
 
     def violations(self) -> int:
         n = ctypes.c_int64()

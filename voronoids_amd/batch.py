@@ -57,13 +57,7 @@ def canonical_from_simplices(simplices: np.ndarray, dim: int) -> tuple[np.ndarra
     L = _lib.lib()
     _lib.check(L.vo_result_canonical(ctypes.byref(r), ctypes.byref(T), ctypes.byref(nT), ctypes.byref(E),
                                      ctypes.byref(nE)))
-    try:
-        Ta = np.ctypeslib.as_array(T, shape=(max(nT.value, 1) * M,))[: nT.value * M].copy()
-        Ea = np.ctypeslib.as_array(E, shape=(max(nE.value, 1) * 2,))[: nE.value * 2].copy()
-    finally:
-        L.vo_free(ctypes.cast(T, ctypes.c_void_p))
-        L.vo_free(ctypes.cast(E, ctypes.c_void_p))
-    return Ta.reshape(-1, M), Ea.reshape(-1, 2)
+    return _rows(T, nT.value, M), _rows(E, nE.value, 2)
 
 
 def plain_simplices(points, seed: int = 0, device: int = 0) -> tuple[np.ndarray, int]:
@@ -133,20 +127,21 @@ def simplex_set_hash(simplices) -> int:
         return int(np.sum(h, dtype=np.uint64))
 
 
-def _take(r: _lib.VoSetResult) -> SetResult:
-    """wrap a C result's buffer as a numpy array without copying; vo_free runs when the array
-    is collected"""
-    M = r.dim + 1
-    n = r.n_simplices
-    addr = ctypes.cast(r.simplices, ctypes.c_void_p).value if r.simplices else None
+def _rows(p, n: int, width: int) -> np.ndarray:
+    """the n rows of a C result's buffer as a numpy array without copying; vo_free runs when the
+    array is collected"""
+    addr = ctypes.cast(p, ctypes.c_void_p).value if p else None
     if n > 0 and addr:
-        buf = (ctypes.c_int32 * (n * M)).from_address(addr)
+        buf = (ctypes.c_int32 * (n * width)).from_address(addr)
         weakref.finalize(buf, _lib.lib().vo_free, ctypes.c_void_p(addr))
-        s = np.frombuffer(buf, dtype=np.int32).reshape(n, M)
-    else:
-        s = np.zeros((0, M), np.int32)
-        if addr:
-            _lib.lib().vo_free(ctypes.c_void_p(addr))
+        return np.frombuffer(buf, dtype=np.int32).reshape(n, width)
+    if addr:
+        _lib.lib().vo_free(ctypes.c_void_p(addr))
+    return np.zeros((0, width), np.int32)
+
+
+def _take(r: _lib.VoSetResult) -> SetResult:
+    s = _rows(r.simplices, r.n_simplices, r.dim + 1)
     r.simplices = _i32p()
     return SetResult(r.tag, r.dim, r.status, r.n_points, r.points_duplicate, s, r.t_submit, r.t_admit, r.t_done,
                      r.rounds)

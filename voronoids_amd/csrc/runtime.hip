@@ -21,6 +21,7 @@
 
 #include "../../include/voronoids.h"
 #include "host_common.hpp"
+#include "readback.hpp"
 #include "kernels.hpp"
 #include "kernels_group.hpp"
 #include "compact.hpp"
@@ -206,6 +207,7 @@ struct vo_tri {
     double ms_run = 0, ms_cav = 0, ms_com = 0, ms_ex = 0, ms_other = 0;
     int64_t n_cav = 0, n_com = 0, n_solo = 0;
     bool dirty_dup = false;
+    vo_host::PinnedRing ring;          // large results on their way to the host
     bool edited = false;               // a simplex's vertices were swapped by hand (its adjacency was not)
 };
 
@@ -2181,9 +2183,10 @@ int vo_tri_export(const vo_tri* t, int32_t* simplices, int32_t* neighbors) {
     // the caller's arrays hold n_live rows (vo_tri_counts): never write past them
     if (nl != t->n_live) return fail(VO_ERR_INTERNAL, "live records differ from the live simplex count");
     const size_t bytes = sizeof(int32_t) * (size_t)nl * t->M;
-    if (simplices && nl) VO_HIP(hipMemcpy(simplices, ds.p, bytes, hipMemcpyDeviceToHost));
-    if (neighbors && nl) VO_HIP(hipMemcpy(neighbors, dn.p, bytes, hipMemcpyDeviceToHost));
-    return 0;
+    std::vector<Segment> out;
+    if (simplices) out.push_back({simplices, ds.p, bytes});
+    if (neighbors) out.push_back({neighbors, dn.p, bytes});
+    return read_back(t->s, t->dev, const_cast<vo_tri*>(t)->ring, out);
 }
 
 // Canonical form by buckets (canon.hpp).  *done = false when a bucket outgrows LDS.  Every array
@@ -2341,17 +2344,17 @@ static int canonical_device(const vo_tri* t, int32_t** T, int64_t* n_T, int32_t*
         nt = slow.nt;
         ne = slow.ne;
     }
-    *T = (int32_t*)std::malloc(sizeof(int32_t) * (size_t)std::max<int64_t>(1, nt * M));
-    *E = (int32_t*)std::malloc(sizeof(int32_t) * (size_t)std::max<int64_t>(1, ne * 2));
-    if (!*T || !*E) {
+    const size_t bt = sizeof(int32_t) * (size_t)nt * M, be = sizeof(int32_t) * (size_t)ne * 2;
+    *T = (int32_t*)result_alloc(bt);
+    *E = (int32_t*)result_alloc(be);
+    rc = *T && *E ? read_back(t->s, t->dev, const_cast<vo_tri*>(t)->ring, {{*T, dT, bt}, {*E, dE, be}})
+                  : fail(VO_ERR_OOM, "host allocation");
+    if (rc) {
         std::free(*T);
         std::free(*E);
         *T = *E = nullptr;
-        return fail(VO_ERR_OOM, "host allocation");
+        return rc;
     }
-    if (nt) VO_HIP(hipMemcpyAsync(*T, dT, sizeof(int32_t) * (size_t)nt * M, hipMemcpyDeviceToHost, t->s));
-    if (ne) VO_HIP(hipMemcpyAsync(*E, dE, sizeof(int32_t) * (size_t)ne * 2, hipMemcpyDeviceToHost, t->s));
-    VO_HIP(hipStreamSynchronize(t->s));
     *n_T = nt;
     *n_E = ne;
     return 0;
@@ -2696,9 +2699,9 @@ int vo_tri_vertices(const vo_tri* t, double* coords) {
         hipLaunchKernelGGL(k_input_coords, dim3((unsigned)std::min<int64_t>((t->n_pts + 255) / 256, 8192)), dim3(256), 0, t->s,
                            t->X64 + (size_t)M * S, t->vmap + M, t->n_pts, D, S, 2 * M, out);
         VO_HIP(hipGetLastError());
-        VO_HIP(hipMemcpyAsync(coords + (size_t)2 * M * D, out, sizeof(double) * (size_t)t->n_pts * D, hipMemcpyDeviceToHost,
-                              t->s));
-        VO_HIP(hipStreamSynchronize(t->s));
+        if ((rc = read_back(t->s, t->dev, const_cast<vo_tri*>(t)->ring,
+                            {{coords + (size_t)2 * M * D, out, sizeof(double) * (size_t)t->n_pts * D}})))
+            return rc;
     }
     return 0;
 }
