@@ -302,6 +302,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
     // replaced (kold) is examined one pass later, once that pass's loads have returned, so the
     // check adds no wait.  A value below the point's key is a higher-priority point of this round
     // (earlier rounds have larger keys): the point cannot win and stops searching.
+    const int kc = min(KC, c.kcap), fc = min(FC, c.fcap);      // (the first points' lists are shorter)
     constexpr bool HASH = kCavityHash<D, G>;
     constexpr int HS = kHashSize<D, G>;
     int nk = 0, nf = 0, ci = 0;
@@ -389,7 +390,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             } else if (und) {
                 st = ST_DEFER;
                 bfs = false;
-            } else if (nk + cnew > KC || nf + cfac > FC) {
+            } else if (nk + cnew > kc || nf + cfac > fc) {
                 st = ST_OVERFLOW;          // re-run alone with global-memory lists
                 bfs = false;
             } else {

@@ -96,6 +96,7 @@ struct RunPlan {
     int chunk_rate_milli;      // records reserved per window point x 1000 across the allocation
                                // stripes of a round (0: no stripes)
     int chunk;                 // the planned round's chunk per stripe
+    int rounds0, n_tets;       // k_seed: rounds before it; records after it
 };
 
 struct vo_tri {
@@ -675,8 +676,175 @@ __global__ void __launch_bounds__(64 * kBootWaves<D>) k_boot(Ctx c, RunPlan* P, 
     }
 }
 
+// ---------------------------------------------------------------- first points, all in LDS
+// The first points of an empty tree.  With few points in the tree a round has few winners, however
+// many it tries, and launched it takes 35 to 45 us (3D) and, planned on the host, 75.  Here one
+// workgroup runs the rounds with the tree's records, the points, the window's lists and the
+// round state in LDS (the same passes; their pointers are LDS pointers once inlined), as many
+// points a round as its wavefronts hold.  Killed records are reused, so that LDS holds about as
+// many records as live simplices; afterwards the record count is set past the simplices created, as
+// appending would have left it.  A round that would need the host (queued exact predicates, a
+// cavity beyond the lists, no room) ends the phase and its points go to the next window.
+//
+// A round takes 18 us here: no load leaves the CU, and what is left is issuing the passes'
+// instructions one wavefront per SIMD.  So sets that fit are done here whole (ALL points: run at
+// 3D n = 8 0.57 -> 0.12 ms, 40 1.85 -> 0.56, 64 2.4 -> 0.93; 2D n = 16 0.63 -> 0.14, 64 1.48 -> 0.38,
+// 128 0.79 -> 0.66, but 200 0.90 -> 0.94), and larger 3D sets only until the launched rounds win more
+// points in their time (FIRST: run at n = 10^3 3.18 -> 2.98 ms, 10^4 6.43 -> 6.21 with 48;
+// 32 and 80 are slower by 2%).  Larger 2D sets begin with k_boot, whose rounds take as long and
+// hold 64 points.
+//
+// Lanes per point, wavefronts, records, points; list capacities per point; the records set aside
+// for each point of a round: a winner needs 2 new ones in 2D, about 7 in 3D (should they run out
+// all the same, the winners that get none wait, and which ones those are depends on timing).
+template <int D> struct Seed;
+template <> struct Seed<3> {
+    static constexpr int G = 32, NW = 4, CAP = 752, LIM = 96, KC = 96, FC = 128, NEW = 12, ALL = 96, FIRST = 48;
+};
+template <> struct Seed<2> {
+    static constexpr int G = 16, NW = 8, CAP = 512, LIM = 128, KC = 64, FC = 96, NEW = 2, ALL = 128, FIRST = 0;
+};
 
+template <int D> struct SeedLds {
+    static constexpr int G = Seed<D>::G, NW = Seed<D>::NW, SLOTS = NW * (64 / G), NV = D + 1 + Seed<D>::LIM;
+    RoundState st;
+    Counters cnt;
+    alignas(16) char rec[(size_t)Seed<D>::CAP * Rec<D>::B];
+    union {
+        CavityLds<D, G> cav[NW];
+        CommitLds<D, G> com[NW];
+    } u;
+    double X64[NV * VT<D>::S];
+    float X32[NV * VT<D>::S];
+    int cp[Seed<D>::LIM];
+    int cav[SLOTS * Seed<D>::KC], fac[SLOTS * Seed<D>::FC], fnb[SLOTS * Seed<D>::FC];
+    int nk[SLOTS], nf[SLOTS], status[SLOTS], flag[SLOTS], win[SLOTS];
+    int nwin, hint;
+};
+static_assert(sizeof(SeedLds<3>) <= 160 * 1024 && sizeof(SeedLds<2>) <= 160 * 1024, "LDS of one CU");
 
+template <int D>
+__global__ void __launch_bounds__(64 * Seed<D>::NW) k_seed(Ctx g, RunPlan p, RunPlan* out, int* pend_out, int limit, int max_rounds) {
+    constexpr int G = Seed<D>::G, NW = Seed<D>::NW, CAP = Seed<D>::CAP, B = Rec<D>::B;
+    constexpr int SLOTS = SeedLds<D>::SLOTS, LIM = Seed<D>::LIM, M = D + 1, S = VT<D>::S;
+    __shared__ SeedLds<D> L;
+    const int tid = threadIdx.x, w = tid >> 6;
+    // the first record, the rest fresh (0xFF bytes); cleared state and statistics
+    for (int i = tid; i < CAP * B / 16; i += 64 * NW)
+        reinterpret_cast<int4*>(L.rec)[i] = i < B / 16 ? reinterpret_cast<const int4*>(g.rec)[i] : make_int4(-1, -1, -1, -1);
+    for (int i = tid; i < (int)(sizeof(RoundState) + sizeof(Counters)) / 4; i += 64 * NW) reinterpret_cast<int*>(&L.st)[i] = 0;
+    for (int i = tid; i < (M + min(p.n_pts, LIM)) * S; i += 64 * NW) {
+        L.X64[i] = g.X64[i];
+        L.X32[i] = g.X32[i];
+    }
+    for (int i = tid; i < LIM; i += 64 * NW) L.cp[i] = -1;
+    __syncthreads();
+    if (tid == 0) {
+        L.st.n_tets = 1;
+        L.hint = 0;
+    }
+    Ctx c = g;
+    c.rec = L.rec;
+    c.cav = L.cav;
+    c.fac = L.fac;
+    c.fnb = L.fnb;
+    c.nk = L.nk;
+    c.nf = L.nf;
+    c.status = L.status;
+    c.win = L.win;
+    c.pflag = L.flag;
+    c.st = &L.st;
+    c.cnt = &L.cnt;
+    c.X64 = L.X64;
+    c.X32 = L.X32;
+    c.cp = L.cp;
+    c.hint = &L.hint;                  // walks start at the first record
+    c.hlevels = 0;
+    c.kcap = Seed<D>::KC;
+    c.fcap = Seed<D>::FC;
+    c.win_cap = SLOTS;
+    c.tet_cap = CAP;
+    c.big_cap = 0;                     // a cavity beyond the lists: the point goes on to the next window
+    c.reuse = 1;
+    c.shared = 0;
+    c.ast = nullptr;
+    c.ctl = nullptr;
+    c.region = nullptr;
+    c.sets = nullptr;
+    c.walk_budget = 0;
+    // the round's bookkeeping, in every lane of the first wavefront
+    int npend = 0, nfresh = 0, nwin = 0;
+    unsigned long long won = 0;
+    for (int r = 0;; ++r) {
+        if (w == 0) {
+            if (r > 0) {               // absorb the last round: its points that go on come first
+                const int f = tid < nwin ? L.flag[tid] : -1;
+                const unsigned long long m = __ballot(f >= 0);
+                if (f >= 0) L.win[__popcll(m & ((1ull << tid) - 1ull))] = f;
+                const int again = __popcll(m), wins = (int)(L.cnt.winners - won);
+                won = L.cnt.winners;
+                p.inserted += wins;
+                p.dups += nwin - again - wins;
+                p.windows += nwin;
+                p.head += nfresh;
+                p.rounds++;
+                npend = again;
+            }
+            const bool stop = r == max_rounds || min(p.n_pts, p.head + SLOTS) > limit || L.st.err || L.st.n_big || L.st.n_q || L.st.n_tets + SLOTS * Seed<D>::NEW > CAP;
+            nfresh = min(p.n_pts - p.head, SLOTS - npend);
+            nwin = stop ? 0 : npend + nfresh;
+            if (tid >= npend && tid < nwin) L.win[tid] = p.head + tid - npend;
+            if (tid == 0) L.nwin = nwin;
+        }
+        __syncthreads();
+        const int n = L.nwin;
+        if (n == 0) break;
+        const unsigned long long key_hi = (unsigned long long)(0xFFFFFFFFu - (uint32_t)(p.rounds0 + r)) << 32;
+        const SlotIter it{w * Group<G>::NG, SLOTS, n, 0};
+        cavity_pass<D, G>(c, n, key_hi, it, L.u.cav[w]);
+        __syncthreads();
+        commit_pass<D, G>(c, n, key_hi, it, L.u.com[w]);
+        __syncthreads();
+    }
+    const int n_rec = min(L.st.n_tets, CAP);
+    for (int i = tid; i < n_rec * B / 16; i += 64 * NW)
+        reinterpret_cast<int4*>(g.rec)[i] = reinterpret_cast<const int4*>(L.rec)[i];
+    if (w == 0 && tid < npend) {
+        pend_out[tid] = L.win[tid];
+        g.cp[L.win[tid]] = L.cp[L.win[tid]];
+    }
+    if (tid == 0) {
+        const Counters& a = L.cnt;
+        Counters& b = g.cnt[0];
+        for (int k = 0; k < 2; ++k) {
+            b.t1[k] += a.t1[k];
+            b.t2[k] += a.t2[k];
+            b.t3[k] += a.t3[k];
+            b.def[k] += a.def[k];
+        }
+        b.walk_steps += a.walk_steps;
+        b.chain_hops += a.chain_hops;
+        b.killed += a.killed;
+        b.created += a.created;
+        b.winners += a.winners;
+        b.dups += a.dups;
+        b.pend += a.pend;
+        b.max_killed = a.max_killed > b.max_killed ? a.max_killed : b.max_killed;
+        b.max_facets = a.max_facets > b.max_facets ? a.max_facets : b.max_facets;
+        g.st->acc_winners += a.winners;
+        g.st->acc_live += (long long)a.created - (long long)a.killed;
+        g.st->acc_pend += a.pend;
+        g.st->err |= L.st.err & ~(unsigned)ERR_TETCAP;
+        // past the simplices created, unless this run reuses records (the skipped ones stay fresh)
+        const long long past = 1 + (long long)a.created;
+        const int n_tets = !g.reuse && past > n_rec && past <= g.tet_cap ? (int)past : n_rec;
+        g.st->n_tets = n_tets;
+        p.n_tets = n_tets;
+        p.npend = npend;
+        p.n_live += (long long)a.created - (long long)a.killed;
+        *out = p;
+    }
+}
 
 // grow the simplex records to cap (copying the first n_tets); new records are all 0xFF bytes:
 // dead, hull adjacency, reservations at the largest key
@@ -1341,15 +1509,48 @@ int absorb_halted_plan(vo_tri* t, const RunPlan& P, bool flags = false) {
     return 0;
 }
 
+int ensure_plan(vo_tri* t) {
+    int rc;
+    if (t->plan) return 0;
+    if (!t->plan_host && hipHostMalloc((void**)&t->plan_host, 2 * sizeof(RunPlan)) != hipSuccess)
+        return fail(VO_ERR_OOM, "pinned");
+    for (auto& e : t->chunk_ev)
+        if (!e) VO_HIP(hipEventCreate(&e));
+    if ((rc = dev_alloc(&t->plan, 1))) return rc;
+    return 0;
+}
+
+// How many points of an empty tree the one-workgroup phase takes.
+template <int D> int seed_limit_of(int64_t n) { return n <= Seed<D>::ALL ? (int)n : Seed<D>::FIRST; }
+int seed_limit(const vo_tri* t) { return t->D == 3 ? seed_limit_of<3>(t->n_pts) : seed_limit_of<2>(t->n_pts); }
+
+// the first points of an empty tree (k_seed); the host's state is then that of a run between rounds
+constexpr int kSeedMaxRounds = 4096;
+int run_seed(vo_tri* t, int limit) {
+    int rc;
+    if ((rc = ensure_plan(t))) return rc;
+    RunPlan p = plan_from_host(t);
+    p.rounds0 = (int)t->rounds;
+    const Ctx c = make_ctx(t);
+    if (t->D == 3)
+        hipLaunchKernelGGL(k_seed<3>, dim3(1), dim3(64 * Seed<3>::NW), 0, t->s, c, p, t->plan, t->pend[t->cur], limit,
+                           kSeedMaxRounds);
+    else
+        hipLaunchKernelGGL(k_seed<2>, dim3(1), dim3(64 * Seed<2>::NW), 0, t->s, c, p, t->plan, t->pend[t->cur], limit,
+                           kSeedMaxRounds);
+    VO_HIP(hipGetLastError());
+    VO_HIP(hipMemcpyAsync(&t->plan_host[0], t->plan, sizeof(RunPlan), hipMemcpyDeviceToHost, t->s));
+    if ((rc = sync_state(t)) || (rc = check_err(t))) return rc;
+    plan_to_host(t, t->plan_host[0]);
+    t->n_tets = t->plan_host[0].n_tets;
+    return 0;
+}
+
 int run_device_planned(vo_tri* t) {
     const int D = t->D, R = t->chunk_rounds;
     int rc;
     bool booted = false;
-    if (!t->plan) {
-        if ((rc = dev_alloc(&t->plan, 1))) return rc;
-        if (hipHostMalloc((void**)&t->plan_host, 2 * sizeof(RunPlan)) != hipSuccess) return fail(VO_ERR_OOM, "pinned");
-        for (auto& e : t->chunk_ev) VO_HIP(hipEventCreate(&e));
-    }
+    if ((rc = ensure_plan(t))) return rc;
     while ((int)t->rev.size() < 2 * R * 3) {
         hipEvent_t e;
         VO_HIP(hipEventCreate(&e));
@@ -2085,10 +2286,14 @@ int vo_tri_run(vo_tri* t) {
     // the per-round host decisions of compaction and XCD regions need the host loop; so does a
     // small run (a few points need a round or two, and the device planner submits at least two
     // chunks of rounds: one point through the host loop takes about a third of the time)
+    // (the small-run rule looks at the points the first phase leaves)
+    int rc;
+    const int seed = seed_limit(t);
+    if (t->n_tets == 1 && t->inserted == 0 && t->npend == 0 && seed > 0 && t->group == 0 && !tf.f && (rc = run_seed(t, seed)))
+        return rc;
     const int64_t todo = t->n_pts - t->head + t->npend;
     const bool host_loop = !t->pipelined || tf.f || t->xcd || t->compact_ratio > 0 || todo <= t->small_run;
-    int rc = host_loop ? run_host_planned(t, tf.f) : run_device_planned(t);
-    if (rc) return rc;
+    if (todo > 0 && (rc = host_loop ? run_host_planned(t, tf.f) : run_device_planned(t))) return rc;
     VO_HIP(hipEventRecord(t->ev[1], t->s));
     VO_HIP(hipEventSynchronize(t->ev[1]));
     float ms = 0;
