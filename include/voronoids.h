@@ -310,6 +310,9 @@ int vo_batch_triangulate(vo_engine* e, const double* pts, const int64_t* set_off
                          uint64_t seed, vo_set_result* results);
 /* canonical T / E (as vo_tri_canonical) of a result's simplices; arrays released with vo_free */
 int vo_result_canonical(const vo_set_result* r, int32_t** T, int64_t* n_T, int32_t** E, int64_t* n_E);
+/* the same, sorted on the engine's device where that is faster (r may come from any engine; n_points
+ * bounds its point indices).  A call of the handle like the others: one thread at a time. */
+int vo_engine_canonical(vo_engine* e, const vo_set_result* r, int32_t** T, int64_t* n_T, int32_t** E, int64_t* n_E);
 double vo_clock(void);
 
 /* served mode: requests of either dimension arrive from any thread; a driver thread admits

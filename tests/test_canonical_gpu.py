@@ -42,3 +42,20 @@ def test_small_trees_and_edited_ones(dim, n):
         T, E = t.canonical()
         Th, Eh = canonical_from_simplices(t.export()[0], dim)
         assert np.array_equal(T, Th) and np.array_equal(E, Eh)
+
+
+@pytest.mark.parametrize("dim,n", [(2, 30), (3, 100), (3, 150), (2, 700), (3, 4096)])
+def test_engine_results_sorted_on_the_device_equal_the_hosts(dim, n):
+    import voronoids_amd as vo
+    from voronoids_amd import datasets
+    from voronoids_amd.batch import canonical_from_simplices
+    e = vo.Engine(dim, max_points=1 << 16)
+    sets = [datasets.uniform(n, dim, seed=41), star(dim, 70), datasets.uniform(n + 1, dim, seed=42)]
+    res = e.batch(sets)
+    for closed in (False, True):                  # a closed engine's results are sorted on the host
+        if closed:
+            e.close()
+        for r in res:
+            T, E = r.canonical()
+            Th, Eh = canonical_from_simplices(r.simplices, dim)
+            assert np.array_equal(T, Th) and np.array_equal(E, Eh)

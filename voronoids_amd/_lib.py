@@ -26,7 +26,7 @@ EXPORTED = [
     "vo_last_error", "vo_version",
     "vo_engine_create", "vo_engine_destroy", "vo_engine_submit", "vo_engine_step", "vo_engine_launch",
     "vo_engine_finish", "vo_engine_results", "vo_engine_stats_get", "vo_engine_config", "vo_batch_triangulate",
-    "vo_result_canonical", "vo_clock",
+    "vo_result_canonical", "vo_engine_canonical", "vo_clock",
     "vo_server_create", "vo_server_submit", "vo_server_results", "vo_server_stats_get", "vo_server_destroy",
     "vo_predicates", "vo_bounding_sphere",
     "vo_tri_check_pairs", "vo_tri_set_vertex", "vo_tri_swap_simplex_vertices",
@@ -137,6 +137,7 @@ def lib() -> ctypes.CDLL:
         L.vo_engine_config.argtypes = [P, ctypes.c_char_p, ctypes.c_int64]
         L.vo_batch_triangulate.argtypes = [P, dp, i64p, ctypes.c_int64, ctypes.c_uint64, res_p]
         L.vo_result_canonical.argtypes = [res_p, ctypes.POINTER(i32p), i64p, ctypes.POINTER(i32p), i64p]
+        L.vo_engine_canonical.argtypes = [P, res_p, ctypes.POINTER(i32p), i64p, ctypes.POINTER(i32p), i64p]
         L.vo_clock.restype = ctypes.c_double
         L.vo_server_create.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.POINTER(P)]
         L.vo_server_submit.argtypes = [P, ctypes.c_int, dp, ctypes.c_int64, ctypes.c_uint64, ctypes.c_int64]

@@ -10,8 +10,10 @@ i = 2(d+1) + i).  There is no CPU fallback.
 from __future__ import annotations
 
 import ctypes
+import os
+import threading
 import weakref
-from dataclasses import dataclass
+from dataclasses import dataclass, field
 
 import numpy as np
 
@@ -34,6 +36,7 @@ class SetResult:
     t_admit: float
     t_done: float
     rounds: int
+    engine: object = field(default=None, repr=False, compare=False)    # weak reference to its Engine
 
     @property
     def latency(self) -> float:
@@ -41,22 +44,31 @@ class SetResult:
 
     def canonical(self) -> tuple[np.ndarray, np.ndarray]:
         """canonical T (all-real simplices as sorted input indices, lexicographic) and E
-        (real-real pairs, sorted, unique): the same form as DelaunayTree.canonical()"""
-        return canonical_from_simplices(self.simplices, self.dim)
+        (real-real pairs, sorted, unique): the same form as DelaunayTree.canonical().  Sorted on
+        the device of the engine it came from while that is open and free, else on the host."""
+        e = self.engine() if self.engine is not None else None
+        out = e._canonical(self) if e is not None else None
+        return canonical_from_simplices(self.simplices, self.dim) if out is None else out
+
+    def __getstate__(self):
+        return {**self.__dict__, "engine": None}
 
 
 def canonical_from_simplices(simplices: np.ndarray, dim: int) -> tuple[np.ndarray, np.ndarray]:
+    return _canonical(_lib.lib().vo_result_canonical, simplices, dim, 0)
+
+
+def _canonical(call, simplices, dim: int, n_points: int):
     M = dim + 1
     s = np.ascontiguousarray(simplices, dtype=np.int32).reshape(-1, M)
     r = _lib.VoSetResult()
     r.dim = dim
+    r.n_points = n_points
     r.n_simplices = s.shape[0]
     r.simplices = s.ctypes.data_as(_i32p)
     T, E = _i32p(), _i32p()
     nT, nE = ctypes.c_int64(), ctypes.c_int64()
-    L = _lib.lib()
-    _lib.check(L.vo_result_canonical(ctypes.byref(r), ctypes.byref(T), ctypes.byref(nT), ctypes.byref(E),
-                                     ctypes.byref(nE)))
+    _lib.check(call(ctypes.byref(r), ctypes.byref(T), ctypes.byref(nT), ctypes.byref(E), ctypes.byref(nE)))
     return _rows(T, nT.value, M), _rows(E, nE.value, 2)
 
 
@@ -162,13 +174,34 @@ class Engine:
         h = ctypes.c_void_p()
         _lib.check(_lib.lib().vo_engine_create(device, dim, int(max_points), int(max_simplices), ctypes.byref(h)))
         self._h = h
+        self._mu = threading.RLock()           # results may be sorted on the device from any thread
+        self._pid = os.getpid()
         for k, v in config.items():
             self.config(k, v)
 
     def close(self) -> None:
         if getattr(self, "_h", None):
-            _lib.lib().vo_engine_destroy(self._h)
-            self._h = None
+            with self._mu:
+                _lib.lib().vo_engine_destroy(self._h)
+                self._h = None
+
+    def _mine(self, out: list[SetResult]) -> list[SetResult]:
+        w = weakref.ref(self)
+        for r in out:
+            r.engine = w
+        return out
+
+    def _canonical(self, r: SetResult):
+        """canonical form on the engine's device (vo_engine_canonical), None when the engine is
+        closed, busy in another thread, or of another process"""
+        if os.getpid() != self._pid or not self._mu.acquire(blocking=False):
+            return None
+        try:
+            if not self._h:
+                return None
+            return _canonical(lambda *a: _lib.lib().vo_engine_canonical(self._h, *a), r.simplices, r.dim, r.n_points)
+        finally:
+            self._mu.release()
 
     def __del__(self):
         try:
@@ -181,11 +214,13 @@ class Engine:
 
     def submit(self, points, seed: int = 0, tag: int = 0) -> None:
         p = np.ascontiguousarray(points, dtype=np.float64).reshape(-1, self.dim)
-        _lib.check(_lib.lib().vo_engine_submit(self._h, p.ctypes.data_as(_dp), p.shape[0], seed, tag))
+        with self._mu:
+            _lib.check(_lib.lib().vo_engine_submit(self._h, p.ctypes.data_as(_dp), p.shape[0], seed, tag))
 
     def step(self) -> int:
         left = ctypes.c_int64()
-        _lib.check(_lib.lib().vo_engine_step(self._h, ctypes.byref(left)))
+        with self._mu:
+            _lib.check(_lib.lib().vo_engine_step(self._h, ctypes.byref(left)))
         return left.value
 
     def results(self) -> list[SetResult]:
@@ -193,10 +228,11 @@ class Engine:
         buf = (_lib.VoSetResult * 256)()
         n = ctypes.c_int64()
         while True:
-            _lib.check(_lib.lib().vo_engine_results(self._h, buf, 256, ctypes.byref(n)))
+            with self._mu:
+                _lib.check(_lib.lib().vo_engine_results(self._h, buf, 256, ctypes.byref(n)))
             out.extend(_take(buf[i]) for i in range(n.value))
             if n.value < 256:
-                return out
+                return self._mine(out)
 
     def run(self) -> list[SetResult]:
         """step until every submitted set is done; results in completion order"""
@@ -226,10 +262,13 @@ class Engine:
         offs = np.ascontiguousarray(offsets, dtype=np.int64)
         n_sets = offs.shape[0] - 1
         res = (_lib.VoSetResult * max(n_sets, 1))()
-        rc = _lib.lib().vo_batch_triangulate(self._h, pts.ctypes.data_as(_dp), offs.ctypes.data_as(_i64p), n_sets,
-                                             seed, res)
-        out = [_take(res[i]) for i in range(n_sets)]
-        _lib.check(rc)
+        with self._mu:
+            rc = _lib.lib().vo_batch_triangulate(self._h, pts.ctypes.data_as(_dp), offs.ctypes.data_as(_i64p), n_sets,
+                                                 seed, res)
+            msg = _lib.lib().vo_last_error()
+        out = self._mine([_take(res[i]) for i in range(n_sets)])
+        if rc != _lib.VO_OK:
+            raise _lib.VoError(rc, msg.decode() if msg else "")
         return out
 
 

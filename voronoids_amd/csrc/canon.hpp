@@ -162,6 +162,29 @@ __global__ void __launch_bounds__(256) k_canon_rows_tree(Ctx c, const int* vmap,
     }
 }
 
+// The same for a list of simplices in reference ids (first = the first point's) without adjacency:
+// every simplex answers for all its edges.  A point index of n or more is noted as a bucket too
+// large to sort here.
+template <int M>
+__global__ void __launch_bounds__(256) k_canon_rows_list(const int32_t* simp, int n_simp, int first, int n, int4* rows,
+                                                         int4* ranks, unsigned long long* cnt, CanonTot* tot) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) tot->rows = (unsigned)n_simp;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n_simp; i += gridDim.x * 256) {
+        int r[4] = {0, 0, 0, 0};
+        bool ok = true;
+        for (int k = 0; k < M; ++k) {
+            const int v = simp[(int64_t)i * M + k];
+            r[k] = v >= first ? v - first : kCanonNone;
+            ok &= r[k] < n || r[k] == kCanonNone;
+        }
+        int4 row = make_int4(kCanonNone, kCanonNone, kCanonNone, kCanonNone), rank = make_int4(0, 0, 0, 0);
+        if (ok) canon_row<M>(make_int4(r[0], r[1], r[2], r[3]), 15u, cnt, row, rank);
+        else atomicMax(&tot->max_bucket, 0xffffffffu);
+        rows[i] = row;
+        ranks[i] = rank;
+    }
+}
+
 // Exclusive scan of n 64-bit values, 4,096 per block: block sums, then each block adds the sums
 // before its own (n / 4096 of them) and scans its tile.  out[n] = the total.  With `big` (the
 // bucket counts): vertices with a bucket above kCanonSmall are listed and the largest noted.

@@ -305,4 +305,14 @@ int dev_alloc(T** p, size_t count) {
 int canonical_from_simplices(int M, const int32_t* s, int64_t nl, int32_t** T, int64_t* n_T, int32_t** E,
                              int64_t* n_E);
 
+// The same sorted on the device: simplices (host) over n points, on stream s of the current device,
+// with idle device memory of the caller as scratch.  *done = false, and nothing else, when the
+// scratch is too small, a point index is n or more, or a vertex has too many simplices.
+struct DeviceBlock {
+    void* p;
+    size_t bytes;
+};
+int canonical_rows_device(hipStream_t s, int M, const int32_t* simplices, int64_t nl, int64_t n, const DeviceBlock scratch[3],
+                          int32_t** T, int64_t* n_T, int32_t** E, int64_t* n_E, bool* done);
+
 }  // namespace vo_host

@@ -1768,6 +1768,9 @@ struct Scratch {
     char* base[3];
     size_t cap[3], used[3] = {0, 0, 0};
     std::vector<void*> own;
+    bool grow = true;                      // allocate what the idle buffers do not hold
+    explicit Scratch(const DeviceBlock b[3])
+        : base{(char*)b[0].p, (char*)b[1].p, (char*)b[2].p}, cap{b[0].bytes, b[1].bytes, b[2].bytes}, grow(false) {}
     explicit Scratch(const vo_tri* t)
         : base{(char*)t->cav, (char*)t->fac, (char*)t->fnb},
           cap{sizeof(int) * (size_t)t->win_cap * t->kcap, sizeof(int) * (size_t)t->win_cap * t->fcap,
@@ -1784,6 +1787,7 @@ struct Scratch {
                 used[i] += bytes;
                 return 0;
             }
+        if (!grow) return VO_ERR_OOM;
         const int rc = dev_alloc(p, n);
         if (!rc) own.push_back(*p);
         return rc;
@@ -2394,17 +2398,18 @@ int vo_tri_export(const vo_tri* t, int32_t* simplices, int32_t* neighbors) {
     return read_back(t->s, t->dev, const_cast<vo_tri*>(t)->ring, out);
 }
 
-// Canonical form by buckets (canon.hpp).  *done = false when a bucket outgrows LDS.  Every array
-// has its bound from the live simplices, so one readback of the sizes is all the host waits for.
+}  // extern "C"
+
+// Canonical form by buckets (canon.hpp) of at most cap simplices over n points; fill(rows, ranks, cnt,
+// tot) launches the kernel that writes their rows.  *done = false when a bucket outgrows LDS.
+// Every array has its bound from cap, so one readback of the sizes is all the host waits for.
 // Measured against the radix sorts with the export and scans they need: kernels at 3D n = 4M
 // 27 -> 7.2 ms (the record stream 4.5, scatter 1.1, sorts 1.3, edges 0.2); the whole call at
 // n = 40 0.60 -> 0.15 ms, at n = 10^5 8.7 -> 2.0 ms (the sorts waited for the device once a pass).
-static int canonical_buckets(const vo_tri* t, Scratch& mem, int32_t** T, int32_t** E, int64_t* n_T, int64_t* n_E,
-                             bool* done) {
-    const int M = t->M, P = M * (M - 1) / 2;
-    const int64_t n = t->n_pts;
-    const size_t cap = (size_t)t->n_live;
-    const hipStream_t s = t->s;
+template <class Fill>
+static int canonical_buckets(hipStream_t s, int M, int64_t n, size_t cap, Scratch& mem, Fill fill, int32_t** T, int32_t** E,
+                             int64_t* n_T, int64_t* n_E, bool* done) {
+    const int P = M * (M - 1) / 2;
     int4 *rows, *ranks, *tb;
     int *eb, *big;
     unsigned long long *cnt, *ofs, *bsum;
@@ -2418,17 +2423,11 @@ static int canonical_buckets(const vo_tri* t, Scratch& mem, int32_t** T, int32_t
         return rc;
     VO_HIP(hipMemsetAsync(tot, 0, sizeof(CanonTot), s));
     VO_HIP(hipMemsetAsync(cnt, 0, sizeof(unsigned long long) * (size_t)n, s));
-    const Ctx c = make_ctx(t);
     auto grid = [](int64_t items, int64_t per, int64_t most) {
         return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((items + per - 1) / per, most)));
     };
-    const dim3 rgrid = grid(t->n_tets, 1024, 8192), vgrid = grid(n, 16, 1 << 16), sgrid = grid((int64_t)cap, 256, 8192);
-    if (M == 4)
-        hipLaunchKernelGGL(k_canon_rows_tree<3>, rgrid, dim3(256), 0, s, c, t->vmap, t->n_tets, (int)t->edited, rows, ranks,
-                           (unsigned)cap, cnt, tot);
-    else
-        hipLaunchKernelGGL(k_canon_rows_tree<2>, rgrid, dim3(256), 0, s, c, t->vmap, t->n_tets, (int)t->edited, rows, ranks,
-                           (unsigned)cap, cnt, tot);
+    const dim3 vgrid = grid(n, 16, 1 << 16), sgrid = grid((int64_t)cap, 256, 8192);
+    fill(rows, ranks, cnt, tot);
     hipLaunchKernelGGL(k_scan64_sums, dim3((unsigned)nb), dim3(256), 0, s, cnt, bsum, n);
     hipLaunchKernelGGL(k_scan64_apply, dim3((unsigned)nb), dim3(256), 0, s, cnt, bsum, ofs, n, &tot->te, big, tot);
     hipLaunchKernelGGL(k_canon_scatter, sgrid, dim3(256), 0, s, rows, ranks, (unsigned)cap, tot, ofs, tb, eb);
@@ -2453,6 +2452,24 @@ static int canonical_buckets(const vo_tri* t, Scratch& mem, int32_t** T, int32_t
     *n_E = (int64_t)h.ne;
     return 0;
 }
+
+// Canonical form by buckets of a tree.
+static int canonical_tree(const vo_tri* t, Scratch& mem, int32_t** T, int32_t** E, int64_t* n_T, int64_t* n_E, bool* done) {
+    const size_t cap = (size_t)t->n_live;
+    const Ctx c = make_ctx(t);
+    auto fill = [&](int4* rows, int4* ranks, unsigned long long* cnt, CanonTot* tot) {
+        const dim3 g((unsigned)std::max(1, std::min((t->n_tets + 1023) / 1024, 8192)));
+        if (t->D == 3)
+            hipLaunchKernelGGL(k_canon_rows_tree<3>, g, dim3(256), 0, t->s, c, t->vmap, t->n_tets, (int)t->edited, rows, ranks,
+                               (unsigned)cap, cnt, tot);
+        else
+            hipLaunchKernelGGL(k_canon_rows_tree<2>, g, dim3(256), 0, t->s, c, t->vmap, t->n_tets, (int)t->edited, rows, ranks,
+                               (unsigned)cap, cnt, tot);
+    };
+    return canonical_buckets(t->s, t->M, t->n_pts, cap, mem, fill, T, E, n_T, n_E, done);
+}
+
+extern "C" {
 
 // Canonical form by radix sorts: real simplices as sorted tuples in lexicographic order (two
 // stable sorts: columns 2-3, then columns 0-1), real edges sorted and unique.
@@ -2541,7 +2558,7 @@ static int canonical_device(const vo_tri* t, int32_t** T, int64_t* n_T, int32_t*
     int64_t nt = 0, ne = 0;
     int rc;
     bool done = t->n_pts == 0;
-    if (!done && (rc = canonical_buckets(t, mem, &dT, &dE, &nt, &ne, &done))) return rc;
+    if (!done && (rc = canonical_tree(t, mem, &dT, &dE, &nt, &ne, &done))) return rc;
     if (!done) {
         if ((rc = canonical_radix(t, slow))) return rc;
         dT = slow.T.p;
@@ -2572,6 +2589,45 @@ int vo_tri_canonical(const vo_tri* t, int32_t** T, int64_t* n_T, int32_t** E, in
 }
 
 }  // extern "C"
+
+namespace vo_host {
+int canonical_rows_device(hipStream_t s, int M, const int32_t* simplices, int64_t nl, int64_t n, const DeviceBlock scratch[3],
+                          int32_t** T, int64_t* n_T, int32_t** E, int64_t* n_E, bool* done) {
+    *done = false;
+    if (nl <= 0 || n <= 0 || nl > INT32_MAX / 8 || n >= kCanonNone) return 0;
+    Scratch mem(scratch);
+    int32_t *in, *dT, *dE;
+    if (mem.get(&in, (size_t)nl * M)) return 0;
+    VO_HIP(hipMemcpyAsync(in, simplices, sizeof(int32_t) * (size_t)nl * M, hipMemcpyHostToDevice, s));
+    auto fill = [&](int4* rows, int4* ranks, unsigned long long* cnt, CanonTot* tot) {
+        const dim3 g((unsigned)std::min<int64_t>((nl + 255) / 256, 4096));
+        if (M == 4) hipLaunchKernelGGL(k_canon_rows_list<4>, g, dim3(256), 0, s, in, (int)nl, 2 * M, (int)n, rows, ranks, cnt, tot);
+        else hipLaunchKernelGGL(k_canon_rows_list<3>, g, dim3(256), 0, s, in, (int)nl, 2 * M, (int)n, rows, ranks, cnt, tot);
+    };
+    int64_t nt = 0, ne = 0;
+    bool ok = false;
+    int rc = canonical_buckets(s, M, n, (size_t)nl, mem, fill, &dT, &dE, &nt, &ne, &ok);
+    if (rc) {
+        VO_HIP(hipStreamSynchronize(s));
+        return rc == VO_ERR_OOM ? 0 : rc;
+    }
+    if (!ok) return 0;
+    const size_t bt = sizeof(int32_t) * (size_t)nt * M, be = sizeof(int32_t) * (size_t)ne * 2;
+    *T = (int32_t*)result_alloc(bt);
+    *E = (int32_t*)result_alloc(be);
+    rc = *T && *E ? read_back_plain(s, {{*T, dT, bt}, {*E, dE, be}}) : fail(VO_ERR_OOM, "host allocation");
+    if (rc) {
+        std::free(*T);
+        std::free(*E);
+        *T = *E = nullptr;
+        return rc;
+    }
+    *n_T = nt;
+    *n_E = ne;
+    *done = true;
+    return 0;
+}
+}  // namespace vo_host
 
 namespace {
 
