@@ -2746,23 +2746,28 @@ int vo_tri_locate(vo_tri* t, const double* p, int32_t* killed, int64_t killed_ca
     *n_facets = nf;
     if (nk > killed_cap || nf > facets_cap)
         return fail(VO_ERR_OVERFLOW, "output buffers too small: n_killed / n_facets hold the sizes needed");
-    DevBuf<int> pos;
-    DevBuf<int32_t> dk, df;
-    int64_t nl = 0;
+    // (the query's lists are in cav1 / fac1; the window's lists are idle)
+    Scratch mem(t);
+    const int64_t nb = (t->n_tets + kLiveTile - 1) / kLiveTile, nb2 = (nb + kScanTile - 1) / kScanTile;
+    unsigned long long *count, *before, *bsum, *total;
+    int32_t *dk, *df;
     int rc;
-    if ((rc = live_positions(t, pos, &nl)) || (rc = dev_alloc(&dk.p, (size_t)nk)) ||
-        (rc = dev_alloc(&df.p, (size_t)nf * (M + 1))))
+    if ((rc = mem.get(&count, (size_t)nb)) || (rc = mem.get(&before, (size_t)nb + 1)) || (rc = mem.get(&bsum, (size_t)nb2)) ||
+        (rc = mem.get(&total, 1)) || (rc = mem.get(&dk, (size_t)nk)) || (rc = mem.get(&df, (size_t)nf * (M + 1))))
         return rc;
-    const unsigned grid = (unsigned)((std::max(nk, nf) + 255) / 256);
+    const dim3 rows((unsigned)std::max(nk, nf));
+    if (D == 3) hipLaunchKernelGGL(k_live_counts<3>, dim3((unsigned)nb), dim3(256), 0, t->s, c, t->n_tets, count);
+    else hipLaunchKernelGGL(k_live_counts<2>, dim3((unsigned)nb), dim3(256), 0, t->s, c, t->n_tets, count);
+    hipLaunchKernelGGL(k_scan64_sums, dim3((unsigned)nb2), dim3(256), 0, t->s, count, bsum, nb);
+    hipLaunchKernelGGL(k_scan64_apply, dim3((unsigned)nb2), dim3(256), 0, t->s, count, bsum, before, nb, total, (int*)nullptr,
+                       (CanonTot*)nullptr);
     if (D == 3)
-        hipLaunchKernelGGL(k_locate_rows<3>, dim3(grid), dim3(256), 0, t->s, c, pos.p, t->vmap, t->cav1, nk, t->fac1, nf,
-                           dk.p, df.p);
+        hipLaunchKernelGGL(k_locate_rows<3>, rows, dim3(64), 0, t->s, c, before, t->vmap, t->cav1, nk, t->fac1, nf, dk, df);
     else
-        hipLaunchKernelGGL(k_locate_rows<2>, dim3(grid), dim3(256), 0, t->s, c, pos.p, t->vmap, t->cav1, nk, t->fac1, nf,
-                           dk.p, df.p);
+        hipLaunchKernelGGL(k_locate_rows<2>, rows, dim3(64), 0, t->s, c, before, t->vmap, t->cav1, nk, t->fac1, nf, dk, df);
     VO_HIP(hipGetLastError());
-    VO_HIP(hipMemcpyAsync(killed, dk.p, sizeof(int32_t) * (size_t)nk, hipMemcpyDeviceToHost, t->s));
-    VO_HIP(hipMemcpyAsync(facets, df.p, sizeof(int32_t) * (size_t)nf * (M + 1), hipMemcpyDeviceToHost, t->s));
+    VO_HIP(hipMemcpyAsync(killed, dk, sizeof(int32_t) * (size_t)nk, hipMemcpyDeviceToHost, t->s));
+    VO_HIP(hipMemcpyAsync(facets, df, sizeof(int32_t) * (size_t)nf * (M + 1), hipMemcpyDeviceToHost, t->s));
     VO_HIP(hipStreamSynchronize(t->s));
     std::sort(killed, killed + nk);           // the reference sorts and dedups (src/delaunay_tree.rs:55-56)
     return 0;
