@@ -110,8 +110,7 @@ struct BatchCtl {
     int min_window;        // least fresh window of a set per round
     int big_window;        // windows at least this large aim at a higher winning fraction
     int slots;             // set slots that may be in use: one past the highest (host, before each replay)
-    int ahead;             // fresh points after the window that may be walked ahead (one set; see
-                           // kAheadWaves)
+    int ahead;             // fresh points after the window that may be walked ahead (one set)
     int virt, vhead;       // virt = 1: the window is not written out: slots below npend are the
                            // pending list (Ctx::win), slot i >= npend is point vhead + i - npend
 };

@@ -108,9 +108,12 @@ __device__ __forceinline__ int lds_find(const int* list, int n, int x) {
 // lanes or fewer (a table per point would take 8 KB and more of LDS per wavefront, and with it a
 // third of the wavefronts) the list is scanned.
 template <int D, int G> constexpr bool kCavityHash = D == 3 && G >= 16;
-template <int D, int G> constexpr int kHashSize = kCavityHash<D, G> ? 256 : 4;
-static_assert(VO_GROUP_KC3 + 64 <= 256, "a full killed list and one pass's finds fit the table");
-__device__ __forceinline__ int hash_slot(int n) { return (int)((unsigned)n * 0x9E3779B1u >> 24); }
+constexpr int pow2_from(int n) { return n <= 1 ? 1 : 2 * pow2_from((n + 1) / 2); }
+// (a full killed list and one pass's finds fit the table)
+template <int D, int G> constexpr int kHashSize = kCavityHash<D, G> ? pow2_from(kGroupKC<D> + 64) : 4;
+template <int SIZE> __device__ __forceinline__ int hash_slot(int n) {
+    return (int)((unsigned)n * 0x9E3779B1u >> 16) & (SIZE - 1);
+}
 
 // LDS of one wavefront of the lane-group cavity search
 template <int D, int G> struct alignas(16) CavityLds {
@@ -121,26 +124,96 @@ template <int D, int G> struct alignas(16) CavityLds {
     int tmp[kCavityHash<D, G> ? 4 : 64];
 };
 
-// Walking ahead.  A small round takes as long as its slowest point, and that is one whose walk
-// started far away: of some hundred fresh points a few walk 30 to 70 steps of 1 us each, where the
-// median walks 3 and its search takes 10 us.  A device-planned window is therefore followed by
-// slots of the fresh points that come after it, up to twice as many as the window has: they walk at
-// most kAheadSteps from where they are, write only their conflict pointer (and the hint of a walk
-// that ended) and search nothing.  When their round comes they are a step or two away.  The tree
-// does not change while this kernel runs, and a point's walk has no part in which points win, so
-// rounds and windows are the same with and without.  Only as many as make
-// up kAheadWaves wavefronts with the window's: a window that fills the chip is bound by its work,
-// and a walk split in two costs a few loads more.  Run at 3D n = 10^4 8.1 -> 6.8 ms, 10^5
-// 12.8 -> 11.1, 4M 63.8 -> 62.4, clustered 10^6 50.6 -> 47.6, 2D n = 10^6 6.9 -> 6.6.  (Steps 8 or
-// 24: 1% slower at 10^5.  Wavefronts: 3,072 in 3D leave clustered points at 48.5, 8,192 in 2D cost
-// 1%.  Four times the window instead of twice: the same.)
-template <int D> constexpr int kAheadWaves = D == 3 ? 8192 : 3072;
-constexpr int kAheadSteps = 12;
+// Walking ahead.  A point's walk keeps D + 1 lanes busy, its search all G: with 32 lanes per point a
+// wavefront walks two points where it could walk 16, and a walk step is 300 instructions.  And a
+// small round takes as long as its slowest point, one whose walk started far away: of some hundred
+// fresh points a few walk 30 to 70 steps of 1 us each, where the median walks 3 and its search takes
+// 10 us.  So the cavity launch of a device-planned round has further blocks that walk the fresh
+// points of the coming windows, up to twice as many as the window has, 4 lanes a point: at most
+// kAheadSteps (kAheadFar from windows of kAheadBig on, where the launch lasts longer) from where
+// they are; they write only the conflict pointer, and the hint of a walk that ended.  When their
+// round comes they are a step or two away.  The tree does not change while this kernel runs, and a
+// point's walk has no part in which points win, so rounds and windows are the same with and
+// without.  Run at 3D n = 10^4 8.1 -> 6.8 ms and 10^5 12.8 -> 11.1 when the points ahead walked with
+// the window's lanes and only beside small windows; with 4 lanes and beside all of them also
+// clustered 10^6 46.0 -> 41.4 and 4M 59.0 -> 57.1.  (kAheadSteps 8 or 24: 1% slower at 10^5;
+// kAheadFar 48 from 8,192 on: 58.5 at 4M; as many points ahead as the window, not twice: clustered
+// 44.0.)  With 4 lanes a point in the search itself (2D windows past 16,384) there is nothing to
+// gain and the second look at the walk's end costs 20%.
+constexpr int kAheadSteps = 12, kAheadFar = 24, kAheadBig = 2048;
+template <int D, int G> constexpr bool kWalksAhead = G >= 8;
+
+template <int D>
+__device__ __forceinline__ void walk_ahead_pass(const Ctx& c, int first, int count, int wb, int nwb, int budget) {
+    using F = typename VT<D>::F;
+    constexpr int M = D + 1, PER = 16;
+    const Group<4> g;
+    const bool lead = g.gl == 0;
+    LocalCnt lc = {};
+    for (int b = wb * PER; b < count; b += nwb * PER) {
+        bool walking = b + g.gid < count, there = false;
+        int p = 0, pv = 0, t = 0, came = -1;
+        F pf{}, a[4];
+        int4 aa = make_int4(-1, -1, -1, -1);
+        if (walking) {
+            p = first + b + g.gid;
+            pv = c.M + p;
+            pf = VT<D>::ld(c.X32, pv);
+            t = c.cp[p];
+            if (t < 0) t = hint_lookup<D>(hint_view(c, p), pf);
+            int2 tt = ld_v01<D>(c, t);
+            for (int hops = 0; tt.x < 0; ++hops) {
+                if (hops > kChainLimit) {
+                    walking = false;           // (its own round reports it)
+                    break;
+                }
+                t = tt.y;
+                tt = ld_v01<D>(c, t);
+                if (lead) lc.chain++;
+            }
+            if (walking) ld_ax<D>(c, t, aa, a);
+        }
+        const bool write = walking;
+        uint32_t rng = mix32((uint32_t)p * 0x9E3779B9u + 0x632BE5ABu);
+        for (int step = 0; __any(walking); ++step) {
+            int s = 1, nb = -1;
+            bool test = false;
+            if (walking) {
+                rng = rng * 1664525u + 1013904223u;
+                int k = (int)((rng >> 16) % M) + g.gl;
+                if (k >= M) k -= M;
+                if (g.gl < M) {
+                    nb = comp(aa, k);
+                    test = !(nb >= 0 && (nb >> 2) == came);
+                    if (test) s = orient_at<D>(c, a, t, k, pv, pf, lc, false);
+                }
+            }
+            const unsigned long long und = g.ballot(test && s == SIGN_UNDECIDED);
+            const unsigned long long neg = g.ballot(test && s != SIGN_UNDECIDED && s < 0);
+            const int nb_sel = g.bcast(nb, neg ? __ffsll(neg) - 1 : 0);
+            if (walking) {
+                if (lead) lc.walk++;
+                if (!und && !neg) there = true;
+                if (und || !neg || nb_sel < 0 || step >= budget) {
+                    walking = false;           // there, or left to its own round
+                } else {
+                    came = t;
+                    t = nb_sel >> 2;
+                    ld_ax<D>(c, t, aa, a);
+                }
+            }
+        }
+        if (write && lead) {
+            c.cp[p] = t;
+            if (there) hint_store<D>(hint_view(c, p), pf, a, t);
+        }
+    }
+    flush_counters(c.cnt, lc);
+}
 
 // One wavefront's share of a round's cavity searches: window slots it.off + kb + lane group for
-// kb = it.base, it.base + it.stride, ... below it.lim; slots from nwin on walk ahead.  Run by
-// k_cavity_g (one wavefront per block) and by the one-workgroup early-round kernel (one share per
-// wavefront).
+// kb = it.base, it.base + it.stride, ... below it.lim.  Run by k_cavity_g (one wavefront per
+// block) and by the one-workgroup kernels (one share per wavefront).
 template <int D, int G>
 __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long long key_hi, const SlotIter it,
                                             CavityLds<D, G>& L) {
@@ -161,7 +234,6 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
     const WinView wv = win_view(c);
     for (int kb = it.base; kb < it.lim; kb += it.stride) {
     const int slot = it.off + kb + g.gid;
-    const bool pre = slot >= nwin;         // (with XCD regions slots are below nwin, too)
     const bool valid = kb + g.gid < it.lim;
     int st = valid ? ST_OK : ST_IDLE;
     int p = 0, pv = 0, t = 0;
@@ -216,7 +288,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
     // resumes from there next round (only in windows of 64 or more, whose other points progress)
     bool walking = st == ST_OK;
     bool paused = false;
-    const int budget = pre ? kAheadSteps : (c.walk_budget > 0 && nwin >= 64) ? c.walk_budget : 0x7fffffff;
+    const int budget = (c.walk_budget > 0 && nwin >= 64) ? c.walk_budget : 0x7fffffff;
     int came = -1;
     uint32_t rng = mix32((uint32_t)p * 0x9E3779B9u + 0x632BE5ABu);
     F a[4];
@@ -242,7 +314,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             if (g.gl < M) {
                 nb = comp(aa, k);
                 test = !(nb >= 0 && (nb >> 2) == came);
-                if (test) s = orient_at<D>(c, a, t, k, pv, pf, lc, !pre);
+                if (test) s = orient_at<D>(c, a, t, k, pv, pf, lc);
             }
         }
         const unsigned long long und = g.ballot(test && s == SIGN_UNDECIDED);
@@ -260,7 +332,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             } else if (!neg) {
                 walking = false;
             } else if (nb_sel < 0 || step > kWalkLimit) {
-                if (lead && !pre) atomicOr(&c.st->err, nb_sel < 0 ? ERR_HULL : ERR_WALK);
+                if (lead) atomicOr(&c.st->err, nb_sel < 0 ? ERR_HULL : ERR_WALK);
                 st = ST_BROKEN;
                 walking = false;
             } else {
@@ -275,15 +347,14 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             }
         }
     }
-    if (st == ST_OK || (st == ST_DEFER && !pre)) {
+    if (st == ST_OK || st == ST_DEFER) {
         if (lead) {
             c.cp[p] = t;
             hint_store<D>(hint_view(c, p), pf, a, t);
         }
-    } else if ((paused || (st == ST_DEFER && pre)) && lead) {
+    } else if (paused && lead) {
         c.cp[p] = t;          // no hint: t need not be near p
     }
-    if (pre) st = ST_IDLE;
 #ifdef VO_POINT_PROBE
     pr_tw = (unsigned)(wall_clock64() - pr_t0);
 #endif
@@ -315,7 +386,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
     if (bfs) {
         if (lead) {
             s_cav[g.gid][0] = t << 2;
-            if constexpr (HASH) L.tab[g.gid][hash_slot(t)] = t;
+            if constexpr (HASH) L.tab[g.gid][hash_slot<HS>(t)] = t;
             if (c.abort_early) kold = atomicMin(kres_p<D>(c, t), key);
         }
         nk = 1;
@@ -343,7 +414,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             if (!hull) {
                 n = nb >> 2;
                 if constexpr (HASH) {
-                    hs = hash_slot(n);
+                    hs = hash_slot<HS>(n);
                     int x = L.tab[g.gid][hs];
                     while (x != -1 && x != n) {
                         hs = (hs + 1) & (HS - 1);
@@ -424,7 +495,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
             c.cav[(size_t)slot * c.kcap + (j)] = x;
         }
     }
-    if (valid && lead && !pre) {
+    if (valid && lead) {
         c.nk[slot] = nk;
         c.nf[slot] = nf;
         c.status[slot] = st;
@@ -454,9 +525,18 @@ __global__ void __launch_bounds__(64, D == 3 ? VO_CAVITY_WAVES : VO_CAVITY_WAVES
         c.st->flag_n = c.pflag ? nwin : 0;
         if (nwin > 0) c.st->n_compact = 0;
     }
-    int slots = nwin;
-    if (c.ctl && c.ctl->virt) slots += max(0, min(c.ctl->ahead, kAheadWaves<D> * Group<G>::NG - nwin));
-    cavity_pass<D, G>(c, nwin, key_hi, slot_iter(c, slots, Group<G>::NG), L);
+    SlotIter it = slot_iter(c, nwin, Group<G>::NG);
+    if (kWalksAhead<D, G> && c.ctl && c.ctl->virt && c.ctl->ahead > 0) {
+        // the blocks past the window's walk ahead (none when the grid was sized too small)
+        const int need = (nwin + Group<G>::NG - 1) / Group<G>::NG;
+        if ((int)blockIdx.x >= need) {
+            walk_ahead_pass<D>(c, c.ctl->vhead + nwin - c.ctl->npend, c.ctl->ahead, blockIdx.x - need, gridDim.x - need,
+                               nwin >= kAheadBig ? kAheadFar : kAheadSteps);
+            return;
+        }
+        it.stride = min((int)gridDim.x, need) * Group<G>::NG;
+    }
+    cavity_pass<D, G>(c, nwin, key_hi, it, L);
 }
 
 // Partners of the ridges of a winner's cavity boundary (fv: the new simplices' vertex tuples in
@@ -614,7 +694,7 @@ __device__ __forceinline__ bool outside_next_star(const Ctx& c, int t, int i, in
 template <int D, int G> struct alignas(16) CommitLds {
     static constexpr int DW = (kGroupFC<D> * D + 31) / 32;   // one bit per (facet, ridge): internal face linked
     // ridges by hash: a facet has 1.5 of them, so at most three quarters of the table fill
-    static constexpr int HS = D == 3 && kGroupMC<D, G> > 0 ? 2 * kGroupMC<D, G> : 4;
+    static constexpr int HS = D == 3 && kGroupMC<D, G> > 0 ? pow2_from(2 * kGroupMC<D, G>) : 4;
     int tab[Group<G>::NG][HS];
     int fac[Group<G>::NG][kGroupFC<D>];                     // facet list, then the new simplices
     typename FacetTuple<D>::T fv[Group<G>::NG][kGroupMC<D, G> > 0 ? kGroupMC<D, G> : 1];   // facet tuples

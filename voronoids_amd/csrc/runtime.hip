@@ -1638,9 +1638,8 @@ int run_device_planned(vo_tri* t) {
                     hipLaunchKernelGGL(k_plan_one<2>, dim3(1 + fixb), dim3(256), 0, t->s, t->plan, c, t->cnt, t->pend[cur]);
                 hipEvent_t* e = &t->rev[(size_t)(slot * R + r) * 3];
                 if (t->round_timing) VO_HIP(hipEventRecord(e[0], t->s));
-                // (the cavity search's blocks cover the points walked ahead, too)
-                const int per_wave = 64 / std::max(Gc, 4), most = (D == 3 ? kAheadWaves<3> : kAheadWaves<2>) * per_wave;
-                const int slots = std::max(est_hi, std::min(3 * est_hi, most));
+                // (with blocks for the points walked ahead, 16 a block and twice the window)
+                const int slots = Gc < 8 ? est_hi : est_hi + (2 * est_hi + 15) / 16 * (64 / Gc);
                 if ((rc = launch_round(t, c, slots, 0, 0, Gc))) return rc;
                 if (t->round_timing) VO_HIP(hipEventRecord(e[1], t->s));
                 if ((rc = launch_round(t, c, est_hi, 0, 1, Gm, false))) return rc;
