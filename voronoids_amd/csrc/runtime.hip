@@ -628,8 +628,13 @@ __device__ void plan_step(RunPlan& p, RoundState* st, bool s_absorb) {
 // beyond the LDS lists, queued exact predicates, an error) halts the planner for the host, as in
 // k_plan_one without in-stream exact evaluation.  The loop is bounded by max_rounds.
 constexpr int kBootMaxRounds = 4096;
-template <int D> constexpr int kBootWaves = D == 3 ? 8 : 12;
 template <int D> constexpr int kBootLanes = 8;      // lanes per point in both passes
+constexpr size_t kLdsBytes = (size_t)160 << 10;     // LDS of one CU
+template <int D> constexpr size_t kBootWaveLds =
+    std::max(sizeof(CavityLds<D, kBootLanes<D>>), sizeof(CommitLds<D, kBootLanes<D>>));
+// (fewer where the lists are built larger)
+template <int D> constexpr int kBootWaves =
+    (int)std::min<size_t>(D == 3 ? 8 : 12, (kLdsBytes - 2048) / kBootWaveLds<D>);
 
 template <int D>
 __global__ void __launch_bounds__(64 * kBootWaves<D>) k_boot(Ctx c, RunPlan* P, int* pend0, int* pend1, int max_rounds) {
@@ -705,11 +710,10 @@ template <> struct Seed<2> {
     static constexpr int G = 16, NW = 8, CAP = 512, LIM = 128, KC = 64, FC = 96, NEW = 2, ALL = 128, FIRST = 0;
 };
 
-template <int D> struct SeedLds {
+template <int D> struct SeedState {
     static constexpr int G = Seed<D>::G, NW = Seed<D>::NW, SLOTS = NW * (64 / G), NV = D + 1 + Seed<D>::LIM;
     RoundState st;
     Counters cnt;
-    alignas(16) char rec[(size_t)Seed<D>::CAP * Rec<D>::B];
     union {
         CavityLds<D, G> cav[NW];
         CommitLds<D, G> com[NW];
@@ -721,11 +725,17 @@ template <int D> struct SeedLds {
     int nk[SLOTS], nf[SLOTS], status[SLOTS], flag[SLOTS], win[SLOTS];
     int nwin, hint;
 };
-static_assert(sizeof(SeedLds<3>) <= 160 * 1024 && sizeof(SeedLds<2>) <= 160 * 1024, "LDS of one CU");
+template <int D> struct SeedLds : SeedState<D> {
+    // (fewer records where the lists are built larger)
+    static constexpr int CAP =
+        (int)std::min<size_t>(Seed<D>::CAP, (kLdsBytes - 512 - sizeof(SeedState<D>)) / Rec<D>::B);
+    alignas(16) char rec[(size_t)CAP * Rec<D>::B];
+};
+static_assert(sizeof(SeedLds<3>) <= kLdsBytes && sizeof(SeedLds<2>) <= kLdsBytes, "LDS of one CU");
 
 template <int D>
 __global__ void __launch_bounds__(64 * Seed<D>::NW) k_seed(Ctx g, RunPlan p, RunPlan* out, int* pend_out, int limit, int max_rounds) {
-    constexpr int G = Seed<D>::G, NW = Seed<D>::NW, CAP = Seed<D>::CAP, B = Rec<D>::B;
+    constexpr int G = Seed<D>::G, NW = Seed<D>::NW, CAP = SeedLds<D>::CAP, B = Rec<D>::B;
     constexpr int SLOTS = SeedLds<D>::SLOTS, LIM = Seed<D>::LIM, M = D + 1, S = VT<D>::S;
     __shared__ SeedLds<D> L;
     const int tid = threadIdx.x, w = tid >> 6;
