@@ -402,11 +402,28 @@ __global__ void __launch_bounds__(256) k_input_coords(const double* X64, const i
         for (int k = 0; k < D; ++k) out[(int64_t)(vmap[i] - id0) * D + k] = X64[i * S + k];
 }
 
-// next window = pending losers followed by fresh points head .. head + nfresh - 1
-__global__ void k_window(int* win, const int* pend, int npend, int head, int nfresh) {
+// a host-planned round: cleared round state, and the window = pending losers followed by fresh points
+// head .. head + nfresh - 1
+__global__ void k_open_round(RoundState* st, int* win, const int* pend, int npend, int head, int nfresh) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < npend) win[i] = pend[i];
     else if (i < npend + nfresh) win[i] = head + (i - npend);
+    if (i == 0) {
+        st->n_next_pending = 0;
+        st->n_winners = 0;
+        st->n_q = 0;
+        st->n_fix = 0;
+        st->n_live_delta = 0;
+        st->n_big = 0;
+    }
+}
+// ... and its end: block 0 adds up the statistics, the others link the shared facets
+template <int D> __global__ void __launch_bounds__(256) k_close_round(Ctx c) {
+    if (blockIdx.x == 0) {
+        round_totals(c.cnt, c.st);
+        return;
+    }
+    if (shared_facets(c)) fix_shared_pass<D>(c, (blockIdx.x - 1) * 256 + threadIdx.x, (gridDim.x - 1) * 256);
 }
 
 // region of point p: the top three bits of its Morton code over the hint grid's box (3D: the
@@ -1160,7 +1177,7 @@ int auto_group(const vo_tri* t, int nwin, int which) {
 
 // nwin sizes the grid (the kernels read the exact window from c.ctl when it is set); G = 0:
 // lanes per point chosen from nwin
-int launch_round(vo_tri* t, const Ctx& c, int nwin, unsigned long long key_hi, int which, int G = 0, bool fix = true) {
+int launch_round(vo_tri* t, const Ctx& c, int nwin, unsigned long long key_hi, int which, int G = 0) {
     if (!G) G = auto_group(t, nwin, which);
     // with regions, a multiple of 8 blocks and slack for unequal region sizes
     auto blocks = [&](int per_block) {
@@ -1194,14 +1211,6 @@ int launch_round(vo_tri* t, const Ctx& c, int nwin, unsigned long long key_hi, i
         }
     }
     VO_HIP(hipGetLastError());
-    // links across the facets two winners share (only without reuse; the thread commit keeps to
-    // disjoint, non-adjacent cavities)
-    if (fix && which && G != 1 && shared_facets(c)) {
-        const int fb = std::max(1, std::min(1024, nwin / 64 + 1));
-        if (t->D == 3) hipLaunchKernelGGL(k_fix_shared<3>, dim3(fb), dim3(256), 0, t->s, c);
-        else hipLaunchKernelGGL(k_fix_shared<2>, dim3(fb), dim3(256), 0, t->s, c);
-        VO_HIP(hipGetLastError());
-    }
     return 0;
 }
 #undef VO_LAUNCH_G
@@ -1309,34 +1318,40 @@ int64_t round_records(const vo_tri* t, int64_t nwin) {
 // The host's side of a finished round whose state is in st_host: errors, points re-run alone,
 // the exact queue, then the counters and the window factor (k_plan_one applies the same rule
 // on the device).
-int finish_round(vo_tri* t, int nwin, int nfresh, FILE* trace, float ms_cav, float ms_com, bool exact_done = false) {
+int finish_round(vo_tri* t, int nwin, int nfresh, FILE* trace, float ms_cav, float ms_com, bool totals, bool exact_done = false) {
     int rc;
     if ((rc = check_err(t))) return rc;
     const int n_big = t->st_host->n_big;
+    int winners = totals ? t->st_host->n_winners : 0, live = totals ? t->st_host->n_live_delta : 0;
     if (n_big > 0 && (rc = run_solo(t, n_big))) return rc;
     const RoundState& r = *t->st_host;
     if (r.n_q > 0 && !exact_done) {      // (exact_done: evaluated in the stream after the commit)
         if ((rc = run_exact(t, r.n_q))) return rc;
         if ((rc = sync_state(t)) || (rc = check_err(t))) return rc;
     }
-    // the round's winners (solo runs included) from the statistics
-    hipLaunchKernelGGL(k_round_totals, dim3(1), dim3(kCntStripes), 0, t->s, t->cnt, t->st);
-    if ((rc = sync_state(t))) return rc;
+    // the round's winners from the statistics (totals: added up at the round's end, but for the
+    // points re-run alone since)
+    if (!totals || n_big > 0) {
+        hipLaunchKernelGGL(k_round_totals, dim3(1), dim3(kCntStripes), 0, t->s, t->cnt, t->st);
+        if ((rc = sync_state(t))) return rc;
+        winners += r.n_winners;
+        live += r.n_live_delta;
+    }
     t->n_tets = r.n_tets;
-    t->n_live += r.n_live_delta;
-    t->inserted += r.n_winners;
+    t->n_live += live;
+    t->inserted += winners;
     t->windows_total += nwin;
     if (trace) {
         std::vector<Counters> hs(kCntStripes);
         hipMemcpy(hs.data(), t->cnt, sizeof(Counters) * kCntStripes, hipMemcpyDeviceToHost);
         const Counters h = sum_counters(hs.data());
         std::fprintf(trace, "%lld %d %d %d %d %.4f %.4f %d %lld %d %d %llu %llu %llu %llu\n", (long long)t->rounds, nwin,
-                     t->npend, nfresh, r.n_winners, ms_cav, ms_com, r.n_q, (long long)t->inserted, n_big,
+                     t->npend, nfresh, winners, ms_cav, ms_com, r.n_q, (long long)t->inserted, n_big,
                      r.n_next_pending, h.walk_steps, h.chain_hops, h.killed, h.created);
     }
-    const int64_t consumed = (int64_t)nwin - r.n_next_pending - r.n_winners;   // duplicates
+    const int64_t consumed = (int64_t)nwin - r.n_next_pending - winners;       // duplicates
     t->dups += consumed;
-    const double frac = nwin ? (double)r.n_winners / nwin : 1.0;
+    const double frac = nwin ? (double)winners / nwin : 1.0;
     // keep about half of the window winning; windows past big_window are throughput-bound
     // (a loser's cavity is wasted work, a round costs little beyond its points), so there
     // the target winning fraction is higher
@@ -1345,7 +1360,7 @@ int finish_round(vo_tri* t, int nwin, int nfresh, FILE* trace, float ms_cav, flo
     if (frac > hi) t->gamma = std::min(t->gamma * 1.5, 4.0);
     else if (frac < lo) t->gamma = std::max(t->gamma * 0.7, 0.002);
     // every round either inserts, drops a duplicate, or resolves queued predicates
-    t->stalled = (r.n_winners == 0 && consumed == 0 && r.n_q == 0) ? t->stalled + 1 : 0;
+    t->stalled = (winners == 0 && consumed == 0 && r.n_q == 0) ? t->stalled + 1 : 0;
     if (t->stalled > 64) return fail(VO_ERR_INTERNAL, "no progress for 64 rounds");
     t->npend = r.n_next_pending;
     t->cur ^= 1;
@@ -1372,9 +1387,8 @@ int run_host_planned(vo_tri* t, FILE* trace) {
         const auto [nwin, nfresh] = host_window(t);
         if ((rc = ensure_records(t, (int64_t)t->n_tets + (int64_t)nwin * window_records(D) + 1024))) return rc;
         const int grid = (nwin + 255) / 256;
-        hipLaunchKernelGGL(k_window, dim3(grid), dim3(256), 0, t->s, t->win, t->pend[t->cur], t->npend, (int)t->head,
-                           nfresh);
-        hipLaunchKernelGGL(k_reset_round, dim3(1), dim3(1), 0, t->s, t->st);
+        hipLaunchKernelGGL(k_open_round, dim3(grid), dim3(256), 0, t->s, t->st, t->win, t->pend[t->cur], t->npend,
+                           (int)t->head, nfresh);
         const unsigned long long key_hi = (unsigned long long)(0xFFFFFFFFu - (uint32_t)t->rounds) << 32;
         Ctx c = make_ctx(t);
 #ifdef VO_POINT_PROBE
@@ -1405,6 +1419,11 @@ int run_host_planned(vo_tri* t, FILE* trace) {
         VO_HIP(hipEventRecord(t->ev[3], t->s));
         if ((rc = launch_round(t, c, nwin, key_hi, 1))) return rc;
         VO_HIP(hipEventRecord(t->ev[1], t->s));
+        // (the thread kernels, one lane per point, share no facets)
+        const int fixb = shared_facets(c) && auto_group(t, nwin, 1) != 1 ? std::max(1, std::min(1024, nwin / 64 + 1)) : 0;
+        if (D == 3) hipLaunchKernelGGL(k_close_round<3>, dim3(1 + fixb), dim3(256), 0, t->s, c);
+        else hipLaunchKernelGGL(k_close_round<2>, dim3(1 + fixb), dim3(256), 0, t->s, c);
+        VO_HIP(hipGetLastError());
         if ((rc = sync_state(t))) return rc;
         float a = 0, b = 0;
         hipEventElapsedTime(&a, t->ev[2], t->ev[3]);
@@ -1423,7 +1442,7 @@ int run_host_planned(vo_tri* t, FILE* trace) {
             std::fwrite(h.data(), sizeof(uint4), h.size(), t->probe_f);
         }
 #endif
-        if ((rc = finish_round(t, nwin, nfresh, trace, a, b))) return rc;
+        if ((rc = finish_round(t, nwin, nfresh, trace, a, b, true))) return rc;
         if (t->compact_ratio > 0 && t->n_tets >= t->compact_min && (double)t->n_tets > t->compact_ratio * (double)t->n_live &&
             (rc = compact(t)))
             return rc;
@@ -1513,7 +1532,7 @@ int absorb_halted_plan(vo_tri* t, const RunPlan& P, bool flags = false) {
     if (exact_done && P.nq_done > 0) t->st_host->n_q = P.nq_done;
     if (P.launched && t->st_host->n_q > 0) t->exact_dev = 1;
     if (t->exact_dev) t->cache_used = true;
-    if (P.launched && (rc = finish_round(t, P.nwin, P.nfresh, nullptr, 0.f, 0.f, exact_done))) return rc;
+    if (P.launched && (rc = finish_round(t, P.nwin, P.nfresh, nullptr, 0.f, 0.f, false, exact_done))) return rc;
     if ((rc = check_err(t))) return rc;
     if (P.halt & HALT_STALL) return fail(VO_ERR_INTERNAL, "no progress for 64 rounds");
     return 0;
@@ -1561,7 +1580,7 @@ int run_device_planned(vo_tri* t) {
     int rc;
     bool booted = false;
     if ((rc = ensure_plan(t))) return rc;
-    while ((int)t->rev.size() < 2 * R * 3) {
+    while (t->round_timing && (int)t->rev.size() < 2 * R * 3) {
         hipEvent_t e;
         VO_HIP(hipEventCreate(&e));
         t->rev.push_back(e);
@@ -1646,13 +1665,13 @@ int run_device_planned(vo_tri* t) {
                     hipLaunchKernelGGL(k_plan_one<3>, dim3(1 + fixb), dim3(256), 0, t->s, t->plan, c, t->cnt, t->pend[cur]);
                 else
                     hipLaunchKernelGGL(k_plan_one<2>, dim3(1 + fixb), dim3(256), 0, t->s, t->plan, c, t->cnt, t->pend[cur]);
-                hipEvent_t* e = &t->rev[(size_t)(slot * R + r) * 3];
+                hipEvent_t* e = t->round_timing ? &t->rev[(size_t)(slot * R + r) * 3] : nullptr;
                 if (t->round_timing) VO_HIP(hipEventRecord(e[0], t->s));
                 // (with blocks for the points walked ahead, 16 a block and twice the window)
                 const int slots = Gc < 8 ? est_hi : est_hi + (2 * est_hi + 15) / 16 * (64 / Gc);
                 if ((rc = launch_round(t, c, slots, 0, 0, Gc))) return rc;
                 if (t->round_timing) VO_HIP(hipEventRecord(e[1], t->s));
-                if ((rc = launch_round(t, c, est_hi, 0, 1, Gm, false))) return rc;
+                if ((rc = launch_round(t, c, est_hi, 0, 1, Gm))) return rc;
                 if (t->round_timing) VO_HIP(hipEventRecord(e[2], t->s));
                 if (t->exact_dev) {
                     // the round's queued predicates (count read from the round state; none: the
