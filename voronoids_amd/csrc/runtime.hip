@@ -96,6 +96,7 @@ struct RunPlan {
     int chunk_rate_milli;      // records reserved per window point x 1000 across the allocation
                                // stripes of a round (0: no stripes)
     int chunk;                 // the planned round's chunk per stripe
+    double frac;               // winners per window point of the last round absorbed (1 before)
     int rounds0, n_tets;       // k_seed: rounds before it; records after it
 };
 
@@ -194,6 +195,7 @@ struct vo_tri {
     int64_t small_run = 64;            // runs of at most this many points use the host loop
     int exact_dev = 0;                 // this run has queued exact predicates: evaluate them in the stream
     int64_t stalled = 0;
+    double win_frac = 1.0;             // winners per window point of the last device-planned round
     double gamma = 0.25;
     int filters = 3;
     int64_t big_window = 0;            // windows at least this large target big_frac_lo..hi winners (0: off)
@@ -583,6 +585,7 @@ __device__ void plan_step(RunPlan& p, RoundState* st, bool s_absorb) {
         p.n_live += st->n_live_delta;
         p.windows += nwin;
         const double frac = nwin ? (double)w / nwin : 1.0;
+        if (nwin) p.frac = frac;
         const bool big = p.big_window > 0 && nwin >= p.big_window;
         const double hi = big ? p.big_frac_hi : p.small_frac_hi, lo = big ? p.big_frac_lo : p.small_frac_lo;
         if (frac > hi) p.gamma = fmin(p.gamma * 1.5, 4.0);
@@ -609,8 +612,14 @@ __device__ void plan_step(RunPlan& p, RoundState* st, bool s_absorb) {
         p.halt |= HALT_BOOT;
         return;
     }
+    // by the last round's share of winners, which changes little from round to round (a stripe that
+    // runs out takes the shared count).  Every record reserved is a line that the export, the
+    // checks, a query and a reset stream over: by the window alone the records were 39 per point at
+    // 3D n = 4M and 54 at 10^5, now 29.8 and 32.8, of which 27 hold simplices
     const long long chunk =
-        p.chunk_rate_milli > 0 ? ((long long)nwin * p.chunk_rate_milli / 1000 + kAllocStripes - 1) / kAllocStripes + 16 : 0;
+        p.chunk_rate_milli > 0
+            ? ((long long)(nwin * fmin(1.0, 1.1 * p.frac) * p.chunk_rate_milli / 1000) + kAllocStripes - 1) / kAllocStripes + 16
+            : 0;
     if ((long long)st->n_tets + (long long)nwin * p.per_point + chunk * kAllocStripes + 1024 > p.tet_cap) {
         p.halt |= HALT_SPACE;
         return;
@@ -1296,19 +1305,19 @@ void choose_reuse(vo_tri* t, int64_t to_insert) {
     t->reuse_on = t->reuse == 1 || (t->reuse < 0 && append_only > ((int64_t)1 << 29));
 }
 
-// records reserved per point to insert: a winner creates about 27 (3D) / 6 (2D) simplices; with
-// reuse all but about 7 (3D) / 2 (2D) of them take the winner's killed records
-int64_t records_per_point(const vo_tri* t) {
-    if (t->reuse_on) return t->D == 3 ? 12 : 4;
-    // allocation stripes leave the unused part of each round's chunks behind (measured: 35-39
-    // records per point in 3D, uniform and clustered; 8.5 in 2D)
-    if (t->alloc_stripes) return t->D == 3 ? 44 : 12;
-    return t->D == 3 ? 30 : 8;
+// Records reserved for `left` points to insert: a winner creates about 27 (3D) / 6 (2D) simplices;
+// with reuse all but about 7 (3D) / 2 (2D) of them take the winner's killed records.  Allocation
+// stripes leave the unused part of each round's chunks behind (29.8 records per point in all at 3D
+// n = 4M, 32.8 at 10^5; 6.6 in 2D), and 64 x 16 records a round, which a few hundred rounds of a small set make more than its own.
+int64_t reserve_records(const vo_tri* t, int64_t left) {
+    if (t->reuse_on) return left * (t->D == 3 ? 12 : 4) + 4096;
+    if (!t->alloc_stripes || left <= t->small_run) return left * (t->D == 3 ? 30 : 8) + 4096;
+    return left * (t->D == 3 ? 44 : 12) + std::min<int64_t>((int64_t)1 << 18, 256 * left) + 4096;
 }
 
 // records a planned round may claim: per_point for each window point, plus the stripes' chunks
 // (the planner's space check, plan_step)
-int chunk_rate_milli(const vo_tri* t) { return (t->alloc_stripes && !t->reuse_on) ? (t->D == 3 ? 25000 : 5400) : 0; }
+int chunk_rate_milli(const vo_tri* t) { return (t->alloc_stripes && !t->reuse_on) ? (t->D == 3 ? 27000 : 6000) : 0; }
 int64_t round_records(const vo_tri* t, int64_t nwin) {
     const int64_t rate = chunk_rate_milli(t);
     const int64_t chunk = rate ? (nwin * rate / 1000 + kAllocStripes - 1) / kAllocStripes + 16 : 0;
@@ -1475,6 +1484,7 @@ RunPlan plan_from_host(const vo_tri* t) {
     p.exact_dev = t->exact_dev;
     p.min_window = t->min_window;
     p.chunk_rate_milli = chunk_rate_milli(t);
+    p.frac = t->win_frac;
     return p;
 }
 
@@ -1489,6 +1499,7 @@ void plan_to_host(vo_tri* t, const RunPlan& p) {
     t->rounds = p.rounds;
     t->stalled = p.stalled;
     t->cur = p.cur;
+    t->win_frac = p.frac;
 }
 
 // cavity and commit kernel time of the R rounds of chunk slot `slot`
@@ -1590,7 +1601,7 @@ int run_device_planned(vo_tri* t) {
     {
         const int64_t left = t->n_pts - t->head + t->npend;
         const int64_t want =
-            std::min<int64_t>((int64_t)t->n_tets + left * records_per_point(t) + 4096, (int64_t)1 << 29);
+            std::min<int64_t>((int64_t)t->n_tets + reserve_records(t, left), (int64_t)1 << 29);
         if ((rc = ensure_records(t, want))) return rc;
     }
     // the lane-group commit of device-planned rounds writes outcome flags (the planning launch's
@@ -2189,6 +2200,7 @@ int vo_tri_reset(vo_tri* t, const double* pts, int64_t n) {
     t->stalled = 0;
     t->exact_dev = 0;
     t->gamma = dim == 3 ? 0.2 : 0.6;
+    t->win_frac = 1.0;
     t->ms_run = t->ms_cav = t->ms_com = t->ms_ex = t->ms_other = t->ms_compact = 0;
     t->n_cav = t->n_com = t->n_solo = t->n_compact = 0;
     t->dirty_dup = false;
@@ -2293,8 +2305,9 @@ int vo_tri_stage(vo_tri* t, const double* pts, int64_t n, uint64_t seed) {
     }
     // simplex capacity for everything staged (uniform data creates ~27 (3D) / 6 (2D) per point)
     choose_reuse(t, n_after - t->inserted - t->dups);
-    const int64_t want = (int64_t)t->n_tets + records_per_point(t) * (n_after - t->inserted - t->dups) + 4096;
-    if ((rc = grow_tets(t, want))) return rc;
+    const int64_t want = (int64_t)t->n_tets + reserve_records(t, n_after - t->inserted - t->dups);
+    // (a tree that grows call by call moves to half as much again, not to the last record needed)
+    if ((rc = t->n_tets > 1 ? ensure_records(t, want) : grow_tets(t, want))) return rc;
     t->n_pts = n_after;
     return 0;
 }
