@@ -1285,7 +1285,13 @@ namespace {
 int ensure_records(vo_tri* t, int64_t need) {
     if (need <= t->tcap) return 0;
     const int64_t cap_max = (int64_t)1 << 29;
-    return grow_tets(t, std::max(need, std::min(t->tcap * 3 / 2, cap_max)));
+    const int64_t half = std::min(t->tcap * 3 / 2, cap_max);
+    // (where half as much again does not fit beside the old records, the records asked for may)
+    if (half > need) {
+        if (grow_tets(t, half) == 0) return 0;
+        (void)hipGetLastError();
+    }
+    return grow_tets(t, need);
 }
 
 // records a window point may create at most, as the planners reserve them
@@ -1297,9 +1303,10 @@ int64_t window_records(int D) { return D == 3 ? 64 : 16; }
 // measured 3D n = 4M 147 -> 154 ms, 2D n = 10M 99 -> 114 ms) and needs the stricter round rule.
 void choose_reuse(vo_tri* t, int64_t to_insert) {
     // append-only growth per point: about 27 (3D) / 6 (2D) live simplices, with allocation
-    // stripes the unused chunk tails (measured up to 39 / 8.5 records per point in all), and
-    // the reservation of the run's last rounds (64 / 16 records per window point, plus their
-    // chunks: about 5 per input point), which must fit below the cap as well
+    // stripes the unused chunk tails (up to 39 / 8.5 records per point in all where a round's
+    // share of winners drops sharply; 32.8 / 6.6 measured), and the reservation of the run's last
+    // rounds (64 / 16 records per window point, plus their chunks: about 5 per input point),
+    // which must fit below the cap as well
     const int64_t per = t->alloc_stripes ? (t->D == 3 ? 46 : 14) : (t->D == 3 ? 34 : 10);
     const int64_t append_only = (int64_t)t->n_tets + per * to_insert + 4096;
     t->reuse_on = t->reuse == 1 || (t->reuse < 0 && append_only > ((int64_t)1 << 29));
@@ -1308,11 +1315,14 @@ void choose_reuse(vo_tri* t, int64_t to_insert) {
 // Records reserved for `left` points to insert: a winner creates about 27 (3D) / 6 (2D) simplices;
 // with reuse all but about 7 (3D) / 2 (2D) of them take the winner's killed records.  Allocation
 // stripes leave the unused part of each round's chunks behind (29.8 records per point in all at 3D
-// n = 4M, 32.8 at 10^5; 6.6 in 2D), and 64 x 16 records a round, which a few hundred rounds of a small set make more than its own.
+// n = 4M, 32.8 at 10^5; 6.6 in 2D), and 64 x 16 records a round, which a few hundred rounds of a
+// small set make more than its own; those are reserved only as far as the 2^29 records allow.
 int64_t reserve_records(const vo_tri* t, int64_t left) {
     if (t->reuse_on) return left * (t->D == 3 ? 12 : 4) + 4096;
     if (!t->alloc_stripes || left <= t->small_run) return left * (t->D == 3 ? 30 : 8) + 4096;
-    return left * (t->D == 3 ? 44 : 12) + std::min<int64_t>((int64_t)1 << 18, 256 * left) + 4096;
+    const int64_t own = left * (t->D == 3 ? 44 : 12) + 4096;
+    const int64_t room = std::max<int64_t>(0, ((int64_t)1 << 29) - t->n_tets - own);
+    return own + std::min({(int64_t)1 << 18, 256 * left, room});
 }
 
 // records a planned round may claim: per_point for each window point, plus the stripes' chunks
