@@ -1446,6 +1446,7 @@ __global__ void __launch_bounds__(64) k_locate_query(Ctx c, QueryPoint<D> q, int
         if (ovf) status = 4;
         else if (s0 <= 0) status = 1;
     }
+    int lo = t;                            // the first of the cavity's records and their neighbors
     if (status == 0) {
         if (lane == 0) {
             s_k[0] = t;
@@ -1464,6 +1465,7 @@ __global__ void __launch_bounds__(64) k_locate_query(Ctx c, QueryPoint<D> q, int
                 hull = nb < 0;
                 n = nb >> 2;
                 test = !hull;
+                if (test) lo = min(lo, n);
             }
             for (int j = 0; j < nk; ++j) {
                 const int x = j < KL ? s_k[j] : out_k[j];
@@ -1506,21 +1508,27 @@ __global__ void __launch_bounds__(64) k_locate_query(Ctx c, QueryPoint<D> q, int
             __syncthreads();
         }
     }
+    for (int o = 32; o; o >>= 1) lo = min(lo, __shfl_xor(lo, o, 64));
     if (lane == 0) {
         res[0] = nk;
         res[1] = nf;
         res[2] = status;
+        res[3] = lo;
     }
 }
 
 // Live records of each 1,024: the numbering of vo_tri_export is the rank among the live records,
 // and a query needs the rank of a few only.  One stream over the records (a line each), four loads
 // in flight per lane; nothing is written but the counts (3D n = 500,000, 17.9 M records: 0.49 ms,
-// 4.7 TB/s; flags, their scan over all records and its sums on the host took 0.8).
+// 4.7 TB/s; flags, their scan over all records and its sums on the host took 0.8).  The stream
+// starts at the tile of the first record that the query asks for, since the number of live records
+// from there on, taken from all, is the number before it.  Of the records made early few are left, so
+// a query asks for late ones: half of the records on average, counts 0.35 -> 0.19 ms at 15 M records,
+// a query 0.45 -> 0.31 ms (with the loads of live_rank in flight together).
 constexpr int kLiveTile = 1024;
-template <int D> __global__ void __launch_bounds__(256) k_live_counts(Ctx c, int n, unsigned long long* count) {
+template <int D> __global__ void __launch_bounds__(256) k_live_counts(Ctx c, int first, int n, unsigned long long* count) {
     __shared__ int s_w[4];
-    const int b0 = blockIdx.x * kLiveTile;
+    const int b0 = (first + (int)blockIdx.x) * kLiveTile;
     int v[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -1532,11 +1540,26 @@ template <int D> __global__ void __launch_bounds__(256) k_live_counts(Ctx c, int
     __syncthreads();
     if (threadIdx.x == 0) count[blockIdx.x] = (unsigned long long)(s_w[0] + s_w[1] + s_w[2] + s_w[3]);
 }
-// rank of record t among the live ones (before: exclusive sums of the counts); the whole wavefront
-template <int D> __device__ __forceinline__ int live_rank(const Ctx& c, const unsigned long long* before, int t) {
+// counts of the tiles from `first` on, as exclusive sums with their total at [tiles]
+struct LiveSums {
+    const unsigned long long* before;
+    int first, tiles;
+    long long n_live;
+};
+// rank of record t among the live ones; the whole wavefront, its 16 loads in flight together
+template <int D> __device__ __forceinline__ int live_rank(const Ctx& c, const LiveSums& p, int t) {
+    const int b0 = t & ~(kLiveTile - 1);
+    int v[kLiveTile / 64];
+#pragma unroll
+    for (int j = 0; j < kLiveTile / 64; ++j) {
+        const int r = b0 + j * 64 + (int)__lane_id();
+        v[j] = r < t ? *v_ptr<D>(c, r, 0) : -1;
+    }
     int k = 0;
-    for (int r = (t & ~(kLiveTile - 1)) + (int)__lane_id(); r < t; r += 64) k += *v_ptr<D>(c, r, 0) >= 0;
-    return (int)before[t / kLiveTile] + wave_total(k);
+#pragma unroll
+    for (int j = 0; j < kLiveTile / 64; ++j) k += v[j] >= 0;
+    const long long from = (long long)(p.before[p.tiles] - p.before[t / kLiveTile - p.first]);
+    return (int)(p.n_live - from) + wave_total(k);
 }
 
 // rows of a located cavity in the export's numbering: killed records -> export positions;
@@ -1544,13 +1567,13 @@ template <int D> __device__ __forceinline__ int live_rank(const Ctx& c, const un
 // reference id space, in the order replace_first gives the new simplex after q).  One wavefront
 // per row.
 template <int D>
-__global__ void __launch_bounds__(64) k_locate_rows(Ctx c, const unsigned long long* before, const int* vmap, const int* in_k,
-                                                    int nk, const int* in_f, int nf, int32_t* out_k, int32_t* out_f) {
+__global__ void __launch_bounds__(64) k_locate_rows(Ctx c, LiveSums live, const int* vmap, const int* in_k, int nk,
+                                                    const int* in_f, int nf, int32_t* out_k, int32_t* out_f) {
     constexpr int M = D + 1;
     const int i = blockIdx.x;
     const bool lead = threadIdx.x == 0;
     if (i < nk) {
-        const int r = live_rank<D>(c, before, in_k[i]);
+        const int r = live_rank<D>(c, live, in_k[i]);
         if (lead) out_k[i] = r;
     }
     if (i < nf) {
@@ -1559,8 +1582,8 @@ __global__ void __launch_bounds__(64) k_locate_rows(Ctx c, const unsigned long l
         const int nb = *a_ptr<D>(c, t, face);
         const int4 nv = replace_first<D>(ld_v<D>(c, t), face, -1);
         int32_t* row = out_f + (size_t)i * (M + 1);
-        const int rt = live_rank<D>(c, before, t);
-        const int ro = nb < 0 ? -1 : live_rank<D>(c, before, nb >> 2);
+        const int rt = live_rank<D>(c, live, t);
+        const int ro = nb < 0 ? -1 : live_rank<D>(c, live, nb >> 2);
         if (lead) {
             row[0] = rt;
             row[1] = ro;

@@ -148,7 +148,7 @@ struct vo_tri {
     int* big = nullptr;
     int* cav1 = nullptr;
     int* fac1 = nullptr;
-    int* misc1 = nullptr;              // nk, nf, status of the single point
+    int* misc1 = nullptr;              // nk, nf, status of the single point; a query's first record
     int big_cap = 1 << 20;
     // hints
     int* hint = nullptr;               // kept over resets while it is large enough
@@ -2784,7 +2784,7 @@ int vo_tri_locate(vo_tri* t, const double* p, int32_t* killed, int64_t killed_ca
                            t->big_cap, t->misc1);
     }
     VO_HIP(hipGetLastError());
-    int res[3] = {0, 0, 0};
+    int res[4] = {0, 0, 0, 0};
     VO_HIP(hipMemcpyAsync(res, t->misc1, sizeof(res), hipMemcpyDeviceToHost, t->s));
     VO_HIP(hipStreamSynchronize(t->s));
     if (res[2] == 1)
@@ -2799,7 +2799,8 @@ int vo_tri_locate(vo_tri* t, const double* p, int32_t* killed, int64_t killed_ca
         return fail(VO_ERR_OVERFLOW, "output buffers too small: n_killed / n_facets hold the sizes needed");
     // (the query's lists are in cav1 / fac1; the window's lists are idle)
     Scratch mem(t);
-    const int64_t nb = (t->n_tets + kLiveTile - 1) / kLiveTile, nb2 = (nb + kScanTile - 1) / kScanTile;
+    const int first = res[3] / kLiveTile;
+    const int64_t nb = (t->n_tets + kLiveTile - 1) / kLiveTile - first, nb2 = (nb + kScanTile - 1) / kScanTile;
     unsigned long long *count, *before, *bsum, *total;
     int32_t *dk, *df;
     int rc;
@@ -2807,15 +2808,16 @@ int vo_tri_locate(vo_tri* t, const double* p, int32_t* killed, int64_t killed_ca
         (rc = mem.get(&total, 1)) || (rc = mem.get(&dk, (size_t)nk)) || (rc = mem.get(&df, (size_t)nf * (M + 1))))
         return rc;
     const dim3 rows((unsigned)std::max(nk, nf));
-    if (D == 3) hipLaunchKernelGGL(k_live_counts<3>, dim3((unsigned)nb), dim3(256), 0, t->s, c, t->n_tets, count);
-    else hipLaunchKernelGGL(k_live_counts<2>, dim3((unsigned)nb), dim3(256), 0, t->s, c, t->n_tets, count);
+    if (D == 3) hipLaunchKernelGGL(k_live_counts<3>, dim3((unsigned)nb), dim3(256), 0, t->s, c, first, t->n_tets, count);
+    else hipLaunchKernelGGL(k_live_counts<2>, dim3((unsigned)nb), dim3(256), 0, t->s, c, first, t->n_tets, count);
     hipLaunchKernelGGL(k_scan64_sums, dim3((unsigned)nb2), dim3(256), 0, t->s, count, bsum, nb);
     hipLaunchKernelGGL(k_scan64_apply, dim3((unsigned)nb2), dim3(256), 0, t->s, count, bsum, before, nb, total, (int*)nullptr,
                        (CanonTot*)nullptr);
+    const LiveSums live{before, first, (int)nb, t->n_live};
     if (D == 3)
-        hipLaunchKernelGGL(k_locate_rows<3>, rows, dim3(64), 0, t->s, c, before, t->vmap, t->cav1, nk, t->fac1, nf, dk, df);
+        hipLaunchKernelGGL(k_locate_rows<3>, rows, dim3(64), 0, t->s, c, live, t->vmap, t->cav1, nk, t->fac1, nf, dk, df);
     else
-        hipLaunchKernelGGL(k_locate_rows<2>, rows, dim3(64), 0, t->s, c, before, t->vmap, t->cav1, nk, t->fac1, nf, dk, df);
+        hipLaunchKernelGGL(k_locate_rows<2>, rows, dim3(64), 0, t->s, c, live, t->vmap, t->cav1, nk, t->fac1, nf, dk, df);
     VO_HIP(hipGetLastError());
     VO_HIP(hipMemcpyAsync(killed, dk, sizeof(int32_t) * (size_t)nk, hipMemcpyDeviceToHost, t->s));
     VO_HIP(hipMemcpyAsync(facets, df, sizeof(int32_t) * (size_t)nf * (M + 1), hipMemcpyDeviceToHost, t->s));
