@@ -11,6 +11,7 @@
 //            rotates around the ridge and finds the neighboring facet by an LDS scan.
 #pragma once
 #include "kernels.hpp"
+#include "ridges.hpp"
 
 namespace vo {
 
@@ -539,32 +540,7 @@ __global__ void __launch_bounds__(64, D == 3 ? VO_CAVITY_WAVES : VO_CAVITY_WAVES
     cavity_pass<D, G>(c, nwin, key_hi, it, L);
 }
 
-// Partners of the ridges of a winner's cavity boundary (fv: the new simplices' vertex tuples in
-// LDS, p first, then the facet's D vertices): ridge k of facet j is the facet's vertices other than
-// fv[j][k].  The boundary of a cavity is a closed manifold, so exactly one other facet holds all of
-// the ridge; its new simplex shares the face across the ridge.
-//
-// 3D: by a hash table of ridges (two entries per facet tuple, -1 = free; an entry is j * 3 + k - 1
-// of the ridge that came first).  Returns the entry of the ridge with the same two vertices, or -1
-// for the first of the two to come.  A scan of the facets reads up to nf tuples per ridge, 3 nf
-// ridges, 30 facets on average and up to 100: run at n = 4M 74.6 -> 66.8 ms, 10^5 16.6 -> 13.6 ms.
-template <int SIZE> __device__ __forceinline__ int match_ridge(const int4* fv, int* tab, int q) {
-    static_assert((SIZE & (SIZE - 1)) == 0, "a power of two");
-    const int4 a = fv[q / 3];
-    const int k = q % 3;
-    const int u = k == 0 ? a.z : a.y, w = k == 2 ? a.z : a.w;
-    const int lo = u < w ? u : w, hi = u < w ? w : u;
-    int h = (int)((((unsigned)lo * 0x9E3779B1u) ^ ((unsigned)hi * 0x85EBCA77u)) >> 16) & (SIZE - 1);
-    for (;;) {
-        const int o = atomicCAS(&tab[h], -1, q);
-        if (o == -1) return -1;
-        const int4 b = fv[o / 3];
-        const int m = o % 3;
-        const int bu = m == 0 ? b.z : b.y, bw = m == 2 ? b.z : b.w;
-        if ((bu == u && bw == w) || (bu == w && bw == u)) return o;
-        h = (h + 1) & (SIZE - 1);
-    }
-}
+// Partners of the ridges of a winner's cavity boundary.  3D: match_ridge of ridges.hpp.
 // 2D (the facet (f1, f2), the ridge one vertex, about 6 facets): a scan, four tuples per step
 // (indices clamped to the list, so every read is in it) before comparing, one LDS round trip per
 // four facets.  Returns the partner facet and, in kk, the index (1..2) of its vertex off the
@@ -878,17 +854,31 @@ __device__ __forceinline__ void commit_pass(const Ctx c, int nwin, unsigned long
                 for (int w = g.gl; w < HS / 4; w += G)
                     reinterpret_cast<int4*>(L.tab[g.gid])[w] = make_int4(-1, -1, -1, -1);
                 __builtin_amdgcn_wave_barrier();
-                for (int q = g.gl; q < nf * D; q += G) {
-                    const int o = match_ridge<HS>(s_fv[g.gid], L.tab[g.gid], q);
+                for (int q0 = 0; q0 < nf * D; q0 += G) {
+                    const int q = q0 + g.gl;
+                    const int o = q < nf * D ? match_ridge<HS>(s_fv[g.gid], L.tab[g.gid], q) : kRidgeFirst;
                     found += __popcll(g.ballot(o >= 0));
-                    if (o < 0) continue;
-                    const int j = q / D, k = 1 + q % D, jj = o / D, kk = 1 + o % D;
-                    const int Nj = reuse ? s_fac[g.gid][j] : base + j, Njj = reuse ? s_fac[g.gid][jj] : base + jj;
+                    if (o == kRidgeFirst) continue;
+                    const int j = q / D, k = 1 + q % D;
+                    const int Nj = reuse ? s_fac[g.gid][j] : base + j;
+                    if (o == kRidgeNoRoom) {
+                        *a_ptr<D>(c, Nj, k) = -1;
+                        continue;
+                    }
+                    const int jj = o / D, kk = 1 + o % D;
+                    const int Njj = reuse ? s_fac[g.gid][jj] : base + jj;
                     *a_ptr<D>(c, Nj, k) = (Njj << 2) | kk;
                     *a_ptr<D>(c, Njj, kk) = (Nj << 2) | k;
                 }
-                // (the lead took part in every step)
-                if (lead && 2 * found != nf * D) atomicOr(&c.st->err, ERR_WALK);
+                // an open boundary: the ridges still without a partner lead nowhere
+                if (2 * found != nf * D) {
+                    __builtin_amdgcn_wave_barrier();
+                    for (int w = g.gl; w < HS; w += G) {
+                        const int o = L.tab[g.gid][w];
+                        if (o >= 0) *a_ptr<D>(c, reuse ? s_fac[g.gid][o / D] : base + o / D, 1 + o % D) = -1;
+                    }
+                    if (lead) atomicOr(&c.st->err, ERR_WALK);
+                }
             }
         } else {
             for (int w = g.gl; w < DW; w += G) s_done[g.gid][w] = 0u;
