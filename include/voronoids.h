@@ -168,7 +168,8 @@ int vo_tri_stats(const vo_tri* t, vo_stats* out);
  * in 2D instead of 0.22 ms through the device planner, which submits at least two chunks of rounds).
  * "walk_budget" (default per the autotuner's table, else 0 = off): in windows of 64 or more points, a
  * point whose walk has moved this many times stops there and resumes next round, so that one long
- * walk does not hold a whole round.  Like abort_early, a budget makes the winners of a round depend
+ * walk does not hold a whole round; while most of a round's walks stop so, the next round's may go
+ * twice as far.  Like abort_early, a budget makes the winners of a round depend
  * on timing (a walk's length depends on which concurrent write a hint cell kept); 0 with
  * abort_early 0 gives the same rounds on every run.
  * "boot_window" (default 0 in 3D, 256 in 2D; 0..65536, 0 = off): a vo_tri_run whose first windows hold at

@@ -46,7 +46,7 @@ constexpr int kChainLimit = 1 << 20;
 constexpr int kCntStripes = 128;
 struct alignas(256) Counters {
     unsigned long long t1[2], t2[2], t3[2], def[2];
-    unsigned long long walk_steps, chain_hops, killed, created, winners, dups, exact_evaluated;
+    unsigned long long walk_steps, chain_hops, killed, created, winners, dups, exact_evaluated, paused;
     unsigned long long max_killed, max_facets;
     unsigned long long pend;       // points sent on to the next window
 };
@@ -68,7 +68,8 @@ struct RoundState {
     int n_live_delta;                 // sum over its winners of (created - killed) (round_totals)
     unsigned long long acc_winners;   // statistics totals at the last round_totals call
     long long acc_live;
-    unsigned long long acc_pend;
+    unsigned long long acc_pend;      // (with paused walks << 32)
+    int n_paused;                     // walks of the round that its budget stopped (round_totals)
     int flag_n;                       // window slots of the last round whose outcomes are in Ctx::pflag
     alignas(256) int n_compact;       // pending points the planning launch placed from Ctx::pflag
 };
@@ -111,6 +112,7 @@ struct BatchCtl {
     int big_window;        // windows at least this large aim at a higher winning fraction
     int slots;             // set slots that may be in use: one past the highest (host, before each replay)
     int ahead;             // fresh points after the window that may be walked ahead (one set)
+    int walk_shift;        // doublings of the walk budget (one set, next_walk_shift)
     int virt, vhead;       // virt = 1: the window is not written out: slots below npend are the
                            // pending list (Ctx::win), slot i >= npend is point vhead + i - npend
 };
@@ -172,7 +174,8 @@ struct Ctx {
     int abort_early;       // lane-group cavity search: reserve each member as it is found and stop
                            // once a reservation shows a higher-priority point of the round
     int walk_budget;       // lane-group cavity walk in windows of at least 64 points: a point that
-                           // has moved this many times stops and resumes there next round (0 = off)
+                           // has moved this many times stops and resumes there next round (0 = off;
+                           // x 2^BatchCtl::walk_shift)
     int M;                 // vertex id of point p is M + p
     int win_cap, kcap, fcap;
     int tet_cap;
@@ -210,6 +213,22 @@ __device__ __forceinline__ void round_params(const Ctx& c, int& nwin, unsigned l
         nwin = c.ctl->nwin;
         key_hi = c.ctl->key_hi;
     }
+}
+
+// Doublings of the walk budget for the next round, from the share of the round's walks that it
+// stopped: one more while it stops most of them, one less once it stops few.  Points far from every
+// hint (thousands of simplices away: points along a line in 3D, whose hint cells hold thousands each,
+// or a grid sized by a small first load) then get there in a logarithm of rounds, and a round that
+// only walked is no lack of progress.  The last budget is above kWalkLimit for any first one.
+constexpr int kWalkShiftMax = 17;
+__host__ __device__ inline bool mostly_paused(int nwin, int paused) { return paused > nwin / 2; }
+__host__ __device__ inline int next_walk_shift(int shift, int nwin, int paused) {
+    if (mostly_paused(nwin, paused)) return shift < kWalkShiftMax ? shift + 1 : shift;
+    return shift > 0 && paused <= nwin / 8 ? shift - 1 : shift;
+}
+__host__ __device__ inline int shifted_budget(int budget, int shift) {
+    const long long b = (long long)budget << shift;
+    return b < 0x7fffffff ? (int)b : 0x7fffffff;
 }
 
 // the round's window: point of slot i
@@ -359,7 +378,7 @@ template <int D> __device__ __forceinline__ int4 replace_first(int4 v, int i, in
 
 struct LocalCnt {
     unsigned t1[2], t2[2], t3[2], def[2];
-    unsigned walk, chain, killed, created, wins, dups, pend;
+    unsigned walk, chain, killed, created, wins, dups, pend, paused;
     unsigned maxk, maxf;
 };
 
@@ -395,6 +414,7 @@ inline Counters sum_counters(const Counters* stripes) {
         r.dups += x.dups;
         r.pend += x.pend;
         r.exact_evaluated += x.exact_evaluated;
+        r.paused += x.paused;
         r.max_killed = x.max_killed > r.max_killed ? x.max_killed : r.max_killed;
         r.max_facets = x.max_facets > r.max_facets ? x.max_facets : r.max_facets;
     }
@@ -434,6 +454,7 @@ __device__ inline void flush_counters(Counters* c, const LocalCnt& l) {
     VO_FLUSH(t3[0], l.t3[0]) VO_FLUSH(t3[1], l.t3[1]) VO_FLUSH(def[0], l.def[0]) VO_FLUSH(def[1], l.def[1])
     VO_FLUSH(walk_steps, l.walk) VO_FLUSH(chain_hops, l.chain) VO_FLUSH(killed, l.killed)
     VO_FLUSH(created, l.created) VO_FLUSH(winners, l.wins) VO_FLUSH(dups, l.dups) VO_FLUSH(pend, l.pend)
+    VO_FLUSH(paused, l.paused)
 #undef VO_FLUSH
     if (__any(l.maxk != 0u)) {
         const unsigned mk = wave_max(l.maxk), mf = wave_max(l.maxf);
@@ -446,17 +467,18 @@ __device__ inline void flush_counters(Counters* c, const LocalCnt& l) {
 
 // Winners and the change in live simplices since the last call, from the striped statistics
 // (each commit wavefront adds its winners, created and killed simplices there), into
-// st->n_winners / st->n_live_delta, and with pend_count the points sent on to the next window
+// st->n_winners / st->n_live_delta, the walks paused into st->n_paused, and with pend_count the points sent on to the next window
 // into st->n_next_pending (rounds whose commit wrote Ctx::pflag instead of appending).  Called
 // by every thread of one block (block-uniform).
 __device__ inline void round_totals(const Counters* cnt, RoundState* st, bool pend_count = false) {
     __shared__ unsigned long long s_w[16], s_p[16];
     __shared__ long long s_l[16];
+    // (pn: points sent on plus paused walks << 32; a round's share of both is below 2^31 each)
     unsigned long long w = 0, pn = 0;
     long long l = 0;
     for (int k = threadIdx.x; k < kCntStripes; k += blockDim.x) {
         w += cnt[k].winners;
-        pn += cnt[k].pend;
+        pn += cnt[k].pend + (cnt[k].paused << 32);
         l += (long long)cnt[k].created - (long long)cnt[k].killed;
     }
     w = wave_sum(w);
@@ -479,7 +501,9 @@ __device__ inline void round_totals(const Counters* cnt, RoundState* st, bool pe
         }
         st->n_winners = (int)(W - st->acc_winners);
         st->n_live_delta = (int)(L - st->acc_live);
-        if (pend_count) st->n_next_pending = (int)(P - st->acc_pend);
+        const unsigned long long sent = P - st->acc_pend;
+        if (pend_count) st->n_next_pending = (int)(unsigned)sent;
+        st->n_paused = (int)(sent >> 32);
         st->acc_winners = W;
         st->acc_live = L;
         st->acc_pend = P;

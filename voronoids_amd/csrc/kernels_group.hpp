@@ -355,6 +355,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
         }
     } else if (paused && lead) {
         c.cp[p] = t;          // no hint: t need not be near p
+        lc.paused++;
     }
 #ifdef VO_POINT_PROBE
     pr_tw = (unsigned)(wall_clock64() - pr_t0);
@@ -518,6 +519,7 @@ template <int D, int G>
 __global__ void __launch_bounds__(64, D == 3 ? VO_CAVITY_WAVES : VO_CAVITY_WAVES2) k_cavity_g(Ctx c, int nwin, unsigned long long key_hi) {
     __shared__ CavityLds<D, G> L;
     round_params(c, nwin, key_hi);
+    if (c.ctl) c.walk_budget = shifted_budget(c.walk_budget, c.ctl->walk_shift);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         // the slots whose shared facets the launch after this round's commit links
         c.st->n_fix = shared_facets(c) ? nwin : 0;

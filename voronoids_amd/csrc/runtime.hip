@@ -195,6 +195,7 @@ struct vo_tri {
     int64_t small_run = 64;            // runs of at most this many points use the host loop
     int exact_dev = 0;                 // this run has queued exact predicates: evaluate them in the stream
     int64_t stalled = 0;
+    int walk_shift = 0;                // doublings of walk_budget (next_walk_shift)
     double win_frac = 1.0;             // winners per window point of the last device-planned round
     double gamma = 0.25;
     int filters = 3;
@@ -245,7 +246,7 @@ Ctx make_ctx(const vo_tri* t) {
     c.filters = t->filters;
     c.solo = 0;
     c.abort_early = t->abort_early;
-    c.walk_budget = t->walk_budget;
+    c.walk_budget = t->walk_budget;      // (host-planned rounds: x 2^walk_shift there)
     c.reuse = t->reuse_on;
     c.shared = t->shared_facets;
     c.win_cap = t->win_cap;
@@ -578,25 +579,31 @@ __device__ void plan_step(RunPlan& p, RoundState* st, bool s_absorb) {
             p.halt |= HALT_HOST;
             return;
         }
-        const int nwin = p.nwin, w = st->n_winners, nx = st->n_next_pending;
+        // (loaded together: every trip of this one thread to memory is a part of each round's time)
+        const int nwin = p.nwin, w = st->n_winners, nx = st->n_next_pending, nq = st->n_q, paused = st->n_paused;
+        const int shift = p.ctl.walk_shift, stalled = p.stalled;
         const int consumed = nwin - nx - w;
         p.dups += consumed;
         p.inserted += w;
         p.n_live += st->n_live_delta;
         p.windows += nwin;
         const double frac = nwin ? (double)w / nwin : 1.0;
-        if (nwin) p.frac = frac;
+        const bool walked = mostly_paused(nwin, paused);     // (says nothing about conflicts)
+        if (nwin && !walked) p.frac = frac;
         const bool big = p.big_window > 0 && nwin >= p.big_window;
         const double hi = big ? p.big_frac_hi : p.small_frac_hi, lo = big ? p.big_frac_lo : p.small_frac_lo;
         if (frac > hi) p.gamma = fmin(p.gamma * 1.5, 4.0);
-        else if (frac < lo) p.gamma = fmax(p.gamma * 0.7, 0.002);
-        p.stalled = (w == 0 && consumed == 0 && st->n_q == 0) ? p.stalled + 1 : 0;
+        else if (frac < lo && !walked) p.gamma = fmax(p.gamma * 0.7, 0.002);
+        // (a round that only walked is followed by longer walks)
+        const int idle = stalled + (!walked || shift == kWalkShiftMax);
+        p.stalled = w || consumed || nq ? 0 : idle;
+        p.ctl.walk_shift = next_walk_shift(shift, nwin, paused);
         p.npend = nx;
         p.cur ^= 1;
         p.head += p.nfresh;
         p.rounds++;
         p.launched = 0;
-        if (p.stalled > 64) p.halt |= HALT_STALL;
+        if (idle > 64 && !(w || consumed || nq)) p.halt |= HALT_STALL;
     }
     if (p.halt) return;
     if (p.head >= p.n_pts && p.npend == 0) {
@@ -671,6 +678,7 @@ __global__ void __launch_bounds__(64 * kBootWaves<D>) k_boot(Ctx c, RunPlan* P, 
         CommitLds<D, G> com[NW];
     } U;
     __shared__ int s_absorb, s_go;     // two flags: a wave may still read one while thread 0 sets the other
+    const int budget = c.walk_budget;
     const int w = threadIdx.x >> 6;
     RunPlan& p = *P;
     for (int r = 0; r <= max_rounds; ++r) {
@@ -688,6 +696,7 @@ __global__ void __launch_bounds__(64 * kBootWaves<D>) k_boot(Ctx c, RunPlan* P, 
         if (!s_go) break;
         const int nwin = p.ctl.nwin;
         const unsigned long long key_hi = p.ctl.key_hi;
+        c.walk_budget = shifted_budget(budget, p.ctl.walk_shift);
         c.win = p.cur ? pend1 : pend0;
         c.pend_next = p.cur ? pend0 : pend1;
         cavity_pass<D, G>(c, nwin, key_hi, SlotIter{w * Group<G>::NG, NW * Group<G>::NG, nwin, 0}, U.cav[w]);
@@ -1342,6 +1351,7 @@ int finish_round(vo_tri* t, int nwin, int nfresh, FILE* trace, float ms_cav, flo
     if ((rc = check_err(t))) return rc;
     const int n_big = t->st_host->n_big;
     int winners = totals ? t->st_host->n_winners : 0, live = totals ? t->st_host->n_live_delta : 0;
+    int paused = totals ? t->st_host->n_paused : 0;
     if (n_big > 0 && (rc = run_solo(t, n_big))) return rc;
     const RoundState& r = *t->st_host;
     if (r.n_q > 0 && !exact_done) {      // (exact_done: evaluated in the stream after the commit)
@@ -1355,6 +1365,7 @@ int finish_round(vo_tri* t, int nwin, int nfresh, FILE* trace, float ms_cav, flo
         if ((rc = sync_state(t))) return rc;
         winners += r.n_winners;
         live += r.n_live_delta;
+        paused += r.n_paused;
     }
     t->n_tets = r.n_tets;
     t->n_live += live;
@@ -1376,10 +1387,14 @@ int finish_round(vo_tri* t, int nwin, int nfresh, FILE* trace, float ms_cav, flo
     // the target winning fraction is higher
     const bool big = t->big_window > 0 && nwin >= t->big_window;
     const double hi = big ? t->big_frac_hi : t->small_frac_hi, lo = big ? t->big_frac_lo : t->small_frac_lo;
+    const bool walked = mostly_paused(nwin, paused);     // (says nothing about conflicts)
     if (frac > hi) t->gamma = std::min(t->gamma * 1.5, 4.0);
-    else if (frac < lo) t->gamma = std::max(t->gamma * 0.7, 0.002);
-    // every round either inserts, drops a duplicate, or resolves queued predicates
-    t->stalled = (winners == 0 && consumed == 0 && r.n_q == 0) ? t->stalled + 1 : 0;
+    else if (frac < lo && !walked) t->gamma = std::max(t->gamma * 0.7, 0.002);
+    // every round either inserts, drops a duplicate, resolves queued predicates, or is followed by
+    // longer walks
+    if (winners || consumed || r.n_q) t->stalled = 0;
+    else if (!walked || t->walk_shift == kWalkShiftMax) t->stalled++;
+    t->walk_shift = next_walk_shift(t->walk_shift, nwin, paused);
     if (t->stalled > 64) return fail(VO_ERR_INTERNAL, "no progress for 64 rounds");
     t->npend = r.n_next_pending;
     t->cur ^= 1;
@@ -1410,6 +1425,7 @@ int run_host_planned(vo_tri* t, FILE* trace) {
                            (int)t->head, nfresh);
         const unsigned long long key_hi = (unsigned long long)(0xFFFFFFFFu - (uint32_t)t->rounds) << 32;
         Ctx c = make_ctx(t);
+        c.walk_budget = shifted_budget(t->walk_budget, t->walk_shift);
 #ifdef VO_POINT_PROBE
         // VO_PROBE=<path>: per round a header (round, nwin, 0, 0), three uint4 per window slot from
         // the cavity kernel and two from the commit kernel
@@ -1487,6 +1503,7 @@ RunPlan plan_from_host(const vo_tri* t) {
     p.npend = t->npend;
     p.rounds = (int)t->rounds;
     p.stalled = (int)t->stalled;
+    p.ctl.walk_shift = t->walk_shift;
     p.cur = t->cur;
     p.win_cap = t->win_cap;
     p.big_window = (int)t->big_window;
@@ -1508,6 +1525,7 @@ void plan_to_host(vo_tri* t, const RunPlan& p) {
     t->npend = p.npend;
     t->rounds = p.rounds;
     t->stalled = p.stalled;
+    t->walk_shift = p.ctl.walk_shift;
     t->cur = p.cur;
     t->win_frac = p.frac;
 }
@@ -2329,6 +2347,7 @@ int vo_tri_run(vo_tri* t) {
     t->ms_cav = t->ms_com = t->ms_ex = t->ms_other = 0;
     t->n_cav = t->n_com = 0;
     t->stalled = 0;
+    t->walk_shift = 0;
     t->exact_dev = 0;
     const int64_t dups0 = t->dups;
     VO_HIP(hipEventRecord(t->ev[0], t->s));
