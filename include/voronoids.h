@@ -6,8 +6,9 @@
  * code and never aborts; vo_last_error() gives a thread-local message for the last failure.
  * Ownership: the caller owns every host buffer (copied during the call, never retained);
  * the library owns all device memory behind a vo_tri handle.  A vo_tri is single-writer
- * (the reference mutates through &mut self); distinct handles may be used from different
- * threads.
+ * (the reference mutates through &mut self).  It serves one call at a time of those that work on
+ * the device, reading calls (const vo_tri*) among them: one made while another thread's runs
+ * waits for it.  Distinct handles may be used from different threads.
  *
  * Ids in exported views follow the reference: super vertices 0..d, ghost vertices d+1..2d+1
  * (never referenced here: the hull is -1), input point i is vertex 2(d+1)+i.

@@ -101,6 +101,10 @@ struct RunPlan {
 };
 
 struct vo_tri {
+    // one call at a time of those that work on the device, whether they change the tree or read it:
+    // readers too use the round's lists as scratch and send large results through the ring
+    // (recursive: an insert is a stage and a run)
+    mutable std::recursive_mutex mu;
     int dev = 0, D = 3, M = 4, S = 4;
     hipStream_t s = nullptr;
     double c[3] = {0, 0, 0}, r = 0, R = 0;
@@ -216,6 +220,8 @@ struct vo_tri {
 };
 
 namespace {
+
+using OneCall = std::lock_guard<std::recursive_mutex>;
 
 Ctx make_ctx(const vo_tri* t) {
     Ctx c;
@@ -2199,6 +2205,7 @@ void vo_tri_destroy(vo_tri* t) {
 
 int vo_tri_reset(vo_tri* t, const double* pts, int64_t n) {
     if (!t) return fail(VO_ERR_INVALID, "null handle");
+    const OneCall one(t->mu);
     if (n < 0 || (n > 0 && !pts)) return fail(VO_ERR_INVALID, "bad point buffer");
     const int dim = t->D;
     VO_HIP(hipSetDevice(t->dev));
@@ -2252,6 +2259,7 @@ int vo_tri_root_sphere(const vo_tri* t, double* center, double* radius) {
 
 int vo_tri_stage(vo_tri* t, const double* pts, int64_t n, uint64_t seed) {
     if (!t) return fail(VO_ERR_INVALID, "null handle");
+    const OneCall one(t->mu);
     if (n < 0 || (n > 0 && !pts)) return fail(VO_ERR_INVALID, "bad point buffer");
     if (n == 0) return 0;
     const int D = t->D, S = t->S, M = t->M;
@@ -2342,6 +2350,7 @@ int vo_tri_stage(vo_tri* t, const double* pts, int64_t n, uint64_t seed) {
 
 int vo_tri_run(vo_tri* t) {
     if (!t) return fail(VO_ERR_INVALID, "null handle");
+    const OneCall one(t->mu);
     VO_HIP(hipSetDevice(t->dev));
     choose_reuse(t, t->n_pts - t->head + t->npend);
     t->ms_cav = t->ms_com = t->ms_ex = t->ms_other = 0;
@@ -2379,6 +2388,8 @@ int vo_tri_run(vo_tri* t) {
 }
 
 int vo_tri_insert(vo_tri* t, const double* pts, int64_t n, uint64_t seed) {
+    if (!t) return fail(VO_ERR_INVALID, "null handle");
+    const OneCall one(t->mu);
     int rc = vo_tri_stage(t, pts, n, seed);
     return rc ? rc : vo_tri_run(t);
 }
@@ -2454,6 +2465,7 @@ static int export_device(const vo_tri* tc, DevBuf<int32_t>& simp, DevBuf<int32_t
 
 int vo_tri_export(const vo_tri* t, int32_t* simplices, int32_t* neighbors) {
     if (!t) return fail(VO_ERR_INVALID, "null handle");
+    const OneCall one(t->mu);
     VO_HIP(hipSetDevice(t->dev));
     DevBuf<int32_t> ds, dn;
     int64_t nl;
@@ -2654,6 +2666,7 @@ static int canonical_device(const vo_tri* t, int32_t** T, int64_t* n_T, int32_t*
 
 int vo_tri_canonical(const vo_tri* t, int32_t** T, int64_t* n_T, int32_t** E, int64_t* n_E) {
     if (!t || !T || !n_T || !E || !n_E) return fail(VO_ERR_INVALID, "null argument");
+    const OneCall one(t->mu);
     VO_HIP(hipSetDevice(t->dev));
     return canonical_device(t, T, n_T, E, n_E);
 }
@@ -2762,12 +2775,14 @@ extern "C" {
 
 int vo_tri_check(vo_tri* t, int64_t* n_violations) {
     if (!t || !n_violations) return fail(VO_ERR_INVALID, "null argument");
+    const OneCall one(t->mu);
     VO_HIP(hipSetDevice(t->dev));
     return run_check(t, 0, n_violations);
 }
 
 int vo_tri_check_pairs(vo_tri* t, int64_t* n_pairs) {
     if (!t || !n_pairs) return fail(VO_ERR_INVALID, "null argument");
+    const OneCall one(t->mu);
     const double work = (double)t->n_live * (double)(t->M + t->n_pts);
     if (work > (double)((int64_t)1 << 36))
         return fail(VO_ERR_INVALID, "vo_tri_check_pairs is O(simplices x vertices), limited to 2^36 pairs; "
@@ -2779,6 +2794,7 @@ int vo_tri_check_pairs(vo_tri* t, int64_t* n_pairs) {
 int vo_tri_locate(vo_tri* t, const double* p, int32_t* killed, int64_t killed_cap, int64_t* n_killed,
                   int32_t* facets, int64_t facets_cap, int64_t* n_facets) {
     if (!t || !p || !n_killed || !n_facets) return fail(VO_ERR_INVALID, "null argument");
+    const OneCall one(t->mu);
     if (killed_cap < 0 || facets_cap < 0 || (killed_cap > 0 && !killed) || (facets_cap > 0 && !facets))
         return fail(VO_ERR_INVALID, "bad output buffer");
     const int D = t->D, M = t->M;
@@ -2847,6 +2863,7 @@ int vo_tri_locate(vo_tri* t, const double* p, int32_t* killed, int64_t killed_ca
 
 int vo_tri_set_vertex(vo_tri* t, int64_t id, const double* coords, int records) {
     if (!t || !coords) return fail(VO_ERR_INVALID, "null argument");
+    const OneCall one(t->mu);
     const int D = t->D, S = t->S;
     for (int k = 0; k < D; ++k)
         if (!std::isfinite(coords[k])) return fail(VO_ERR_INVALID, "non-finite coordinate");
@@ -2880,6 +2897,7 @@ int vo_tri_set_vertex(vo_tri* t, int64_t id, const double* coords, int records) 
 
 int vo_tri_swap_simplex_vertices(vo_tri* t, int64_t simplex, int i, int j) {
     if (!t) return fail(VO_ERR_INVALID, "null handle");
+    const OneCall one(t->mu);
     if (i < 0 || j < 0 || i > t->D || j > t->D || i == j) return fail(VO_ERR_INVALID, "i, j must be distinct in 0..dim");
     if (simplex < 0 || simplex >= t->n_live) return fail(VO_ERR_INVALID, "no live simplex at that export index");
     VO_HIP(hipSetDevice(t->dev));
@@ -3023,6 +3041,7 @@ int vo_tri_config(vo_tri* t, const char* key, int64_t value) {
 
 int vo_tri_vertices(const vo_tri* t, double* coords) {
     if (!t || !coords) return fail(VO_ERR_INVALID, "null argument");
+    const OneCall one(t->mu);
     VO_HIP(hipSetDevice(t->dev));
     const int D = t->D, M = t->M, S = t->S;
     for (int v = 0; v < 2 * M; ++v) {
