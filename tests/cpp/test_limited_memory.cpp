@@ -1,0 +1,92 @@
+// A tree whose device memory runs out: this program's hipMalloc and hipFree stand before the HIP
+// library's and refuse what would pass a limit, and the calls have to do with what there is or
+// leave the tree as it was.
+//
+//   test_limited_memory points    tables of a growing tree
+#include <dlfcn.h>
+#include <hip/hip_runtime_api.h>
+
+#include <cstdint>
+#include <cstdio>
+#include <cstring>
+#include <map>
+#include <random>
+#include <vector>
+
+#include "voronoids.h"
+
+static std::map<void*, size_t> g_sizes;
+static size_t g_used = 0, g_limit = SIZE_MAX;
+
+extern "C" hipError_t hipMalloc(void** p, size_t bytes) {
+    using Fn = hipError_t (*)(void**, size_t);
+    static const Fn real = (Fn)dlsym(RTLD_NEXT, "hipMalloc");
+    if (bytes > g_limit || g_used > g_limit - bytes) return hipErrorOutOfMemory;
+    const hipError_t e = real(p, bytes);
+    if (e == hipSuccess) {
+        g_sizes[*p] = bytes;
+        g_used += bytes;
+    }
+    return e;
+}
+extern "C" hipError_t hipFree(void* p) {
+    using Fn = hipError_t (*)(void*);
+    static const Fn real = (Fn)dlsym(RTLD_NEXT, "hipFree");
+    const auto it = g_sizes.find(p);
+    if (it != g_sizes.end()) {
+        g_used -= it->second;
+        g_sizes.erase(it);
+    }
+    return real(p);
+}
+
+#define CHECK(x)                                                                                     \
+    do {                                                                                             \
+        if (!(x)) {                                                                                  \
+            std::printf("line %d: %s (%s)\n", __LINE__, #x, vo_last_error() ? vo_last_error() : ""); \
+            return 1;                                                                                \
+        }                                                                                            \
+    } while (0)
+
+static std::vector<double> points(int dim, int64_t n, unsigned seed) {
+    std::mt19937_64 g(seed);
+    std::uniform_real_distribution<double> u(0.0, 1.0);
+    std::vector<double> p((size_t)n * dim);
+    for (double& x : p) x = u(g);
+    return p;
+}
+
+static int run_points() {
+    const int64_t n = 200000;
+    const std::vector<double> p = points(2, n, 1), more = points(2, 20, 2);
+    vo_tri* t = nullptr;
+    CHECK(vo_tri_create(0, 2, p.data(), n, &t) == VO_OK);
+    CHECK(vo_tri_insert(t, p.data(), n, 0) == VO_OK);
+    // records enough for a few points more: what is left to ask for are the point tables, 32 bytes a
+    // point: 6.4 MB as needed, 9.6 MB with half as many points again
+    CHECK(vo_tri_config(t, "reuse", 1) == VO_OK);
+    const size_t used = g_used;
+    g_limit = used + 5000000;                // neither
+    for (int k = 0; k < 3; ++k) {
+        CHECK(vo_tri_stage(t, more.data(), 10, 0) == VO_ERR_OOM);
+        CHECK(g_used == used);
+    }
+    g_limit = used + 8500000;                // the tables needed
+    CHECK(vo_tri_insert(t, more.data(), 10, 0) == VO_OK);
+    g_limit = SIZE_MAX;
+    CHECK(vo_tri_insert(t, more.data() + 20, 10, 0) == VO_OK);
+    int64_t bad = -1, nv = 0;
+    CHECK(vo_tri_check(t, &bad) == VO_OK && bad == 0);
+    CHECK(vo_tri_counts(t, &nv, nullptr, nullptr) == VO_OK && nv == n + 20 + 3);
+    vo_tri_destroy(t);
+    CHECK(g_used == 0);
+    return 0;
+}
+
+int main(int argc, char** argv) {
+    const char* what = argc > 1 ? argv[1] : "";
+    int failed = 1;
+    if (!std::strcmp(what, "points")) failed = run_points();
+    if (!failed) std::printf("%s: ok\n", what);
+    return failed;
+}

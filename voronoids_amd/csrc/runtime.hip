@@ -929,14 +929,17 @@ int grow_tets(vo_tri* t, int64_t cap) {
 int grow_points(vo_tri* t, int64_t cap) {
     if (cap <= t->vcap) return 0;
     if (t->M + cap > INT32_MAX / 2) return fail(VO_ERR_INVALID, "too many points");
-    double* X64;
-    float* X32;
-    int *cp, *vmap;
+    double* X64 = nullptr;
+    float* X32 = nullptr;
+    int *cp = nullptr, *vmap = nullptr;
     int rc;
     const int64_t nv = t->M + cap;
     if ((rc = dev_alloc(&X64, nv * t->S)) || (rc = dev_alloc(&X32, nv * t->S)) || (rc = dev_alloc(&cp, cap)) ||
-        (rc = dev_alloc(&vmap, nv)))
+        (rc = dev_alloc(&vmap, nv))) {
+        hipFree(X64); hipFree(X32); hipFree(cp); hipFree(vmap);
+        (void)hipGetLastError();       // (not for the next launch to report)
         return rc;
+    }
     if (t->X64) {
         const int64_t old = t->M + t->n_pts;
         VO_HIP(hipMemcpyAsync(X64, t->X64, sizeof(double) * old * t->S, hipMemcpyDeviceToDevice, t->s));
@@ -949,6 +952,16 @@ int grow_points(vo_tri* t, int64_t cap) {
     t->X64 = X64; t->X32 = X32; t->cp = cp; t->vmap = vmap;
     t->vcap = cap;
     return 0;
+}
+
+// room for `need` points, and in a tree that has some for half as many again, so that points added
+// one at a time do not move the tables each time (where that does not fit beside the old tables,
+// the rows asked for may)
+int ensure_points(vo_tri* t, int64_t need) {
+    if (need <= t->vcap) return 0;
+    const int64_t half = t->n_pts > 0 ? std::min(t->vcap * 3 / 2, (int64_t)INT32_MAX / 2 - t->M) : 0;
+    if (half > need && grow_points(t, half) == 0) return 0;
+    return grow_points(t, need);
 }
 
 // An empty tree: the super vertices, the first simplex's record, the round state and cleared
@@ -2268,10 +2281,7 @@ int vo_tri_stage(vo_tri* t, const double* pts, int64_t n, uint64_t seed) {
     if (!dev_check && !all_finite(pts, n * D)) return fail(VO_ERR_INVALID, "non-finite coordinate");
     VO_HIP(hipSetDevice(t->dev));
     int rc;
-    // (room for half as many points again, so that points added one at a time do not move the tables each time)
-    if (t->n_pts + n > t->vcap &&
-        (rc = grow_points(t, std::max(t->n_pts + n, t->n_pts > 0 ? std::min(t->vcap * 3 / 2, (int64_t)INT32_MAX / 2 - M) : 0))))
-        return rc;
+    if ((rc = ensure_points(t, t->n_pts + n))) return rc;
     // vertex ids are committed (n_pts) only once every upload and allocation has succeeded, so
     // that a failed stage leaves the handle as it was
     const int64_t v0 = M + t->n_pts, n_after = t->n_pts + n;
