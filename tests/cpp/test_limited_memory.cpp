@@ -3,6 +3,7 @@
 // leave the tree as it was.
 //
 //   test_limited_memory points    tables of a growing tree
+//   test_limited_memory compact   a run that ends for lack of records, taken up again with compaction
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 
@@ -83,10 +84,44 @@ static int run_points() {
     return 0;
 }
 
+static int run_compact() {
+    const int64_t n = 30000;
+    for (const int dim : {3, 2}) {
+        const std::vector<double> p = points(dim, n, 3);
+        vo_tri* t = nullptr;
+        CHECK(vo_tri_create(0, dim, p.data(), n, &t) == VO_OK);
+        // reserved at the stage: 30 (2D: 8) records a point, while windows as large as the tree reserve
+        // 64 (16) for each of their points: that fails with about a third of the points inserted,
+        // when points beyond the window have walked ahead
+        CHECK(vo_tri_config(t, "alloc_stripes", 0) == VO_OK);
+        CHECK(vo_tri_config(t, "window_gamma_milli", 1000) == VO_OK);
+        CHECK(vo_tri_config(t, "small_frac_lo_milli", 1) == VO_OK);
+        CHECK(vo_tri_config(t, "small_frac_hi_milli", 999) == VO_OK);
+        CHECK(vo_tri_stage(t, p.data(), n, 0) == VO_OK);
+        g_limit = g_used + 1000000;
+        CHECK(vo_tri_run(t) == VO_ERR_OOM);
+        g_limit = SIZE_MAX;
+        int64_t nv = 0, bad = -1;
+        CHECK(vo_tri_counts(t, &nv, nullptr, nullptr) == VO_OK);
+        std::printf("%dD: %lld of %lld points in when the records ran out\n", dim, (long long)nv, (long long)n);
+        std::fflush(stdout);
+        CHECK(nv > n / 10 && nv < n / 2);
+        CHECK(vo_tri_config(t, "compact_min", 16) == VO_OK);
+        CHECK(vo_tri_config(t, "compact_ratio_milli", 1500) == VO_OK);
+        CHECK(vo_tri_run(t) == VO_OK);
+        CHECK(vo_tri_check(t, &bad) == VO_OK && bad == 0);
+        CHECK(vo_tri_counts(t, &nv, nullptr, nullptr) == VO_OK && nv == n + dim + 1);
+        vo_tri_destroy(t);
+    }
+    CHECK(g_used == 0);
+    return 0;
+}
+
 int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     int failed = 1;
     if (!std::strcmp(what, "points")) failed = run_points();
+    if (!std::strcmp(what, "compact")) failed = run_compact();
     if (!failed) std::printf("%s: ok\n", what);
     return failed;
 }

@@ -1111,7 +1111,7 @@ int run_solo(vo_tri* t, int n_big) {
 
 // Live records to a fresh array in spatial order (compact.hpp), between rounds: the pending
 // points' conflict pointers and the walk hints are first moved to live simplices, then
-// renumbered with the records.
+// renumbered with the records; those of points to come are dropped.
 int compact(vo_tri* t) {
     const int D = t->D;
     const int n = t->n_tets;
@@ -1164,6 +1164,10 @@ int compact(vo_tri* t) {
         hipLaunchKernelGGL(k_move<2>, dim3(blocks), dim3(256), 0, t->s, c, t->rec_spare, t->cmap, n);
     }
     if (t->npend) hipLaunchKernelGGL(k_remap_points, dim3(256), dim3(256), 0, t->s, t->cp, pend, t->npend, t->cmap);
+    // points not yet in a window have no pointer, but for those that a device-planned run walked ahead
+    // before it ended early: they start from the hints
+    if (t->n_pts > t->head)
+        VO_HIP(hipMemsetAsync(t->cp + t->head, 0xFF, sizeof(int) * (size_t)(t->n_pts - t->head), t->s));
     hipLaunchKernelGGL(k_remap_hints, dim3(1024), dim3(256), 0, t->s, t->hint, cells, t->cmap);
     VO_HIP(hipGetLastError());
     VO_HIP(hipMemcpyAsync(&t->st->n_tets, &live, sizeof(int), hipMemcpyHostToDevice, t->s));
