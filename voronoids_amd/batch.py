@@ -141,11 +141,11 @@ def simplex_set_hash(simplices) -> int:
 
 def _rows(p, n: int, width: int) -> np.ndarray:
     """the n rows of a C result's buffer as a numpy array without copying; vo_free runs when the
-    array is collected"""
+    array is collected (at exit it is left to the system: exit handlers may still read it)"""
     addr = ctypes.cast(p, ctypes.c_void_p).value if p else None
     if n > 0 and addr:
         buf = (ctypes.c_int32 * (n * width)).from_address(addr)
-        weakref.finalize(buf, _lib.lib().vo_free, ctypes.c_void_p(addr))
+        weakref.finalize(buf, _lib.lib().vo_free, ctypes.c_void_p(addr)).atexit = False
         return np.frombuffer(buf, dtype=np.int32).reshape(n, width)
     if addr:
         _lib.lib().vo_free(ctypes.c_void_p(addr))
