@@ -13,7 +13,7 @@ import ctypes
 import os
 import threading
 import weakref
-from dataclasses import dataclass, field
+from dataclasses import dataclass
 
 import numpy as np
 
@@ -36,7 +36,8 @@ class SetResult:
     t_admit: float
     t_done: float
     rounds: int
-    engine: object = field(default=None, repr=False, compare=False)    # weak reference to its Engine
+
+    _engine = None                 # weak reference to its Engine (no field: not a part of the record)
 
     @property
     def latency(self) -> float:
@@ -46,12 +47,12 @@ class SetResult:
         """canonical T (all-real simplices as sorted input indices, lexicographic) and E
         (real-real pairs, sorted, unique): the same form as DelaunayTree.canonical().  Sorted on
         the device of the engine it came from while that is open and free, else on the host."""
-        e = self.engine() if self.engine is not None else None
+        e = self._engine() if self._engine is not None else None
         out = e._canonical(self) if e is not None else None
         return canonical_from_simplices(self.simplices, self.dim) if out is None else out
 
     def __getstate__(self):
-        return {**self.__dict__, "engine": None}
+        return {k: v for k, v in self.__dict__.items() if k != "_engine"}
 
 
 def canonical_from_simplices(simplices: np.ndarray, dim: int) -> tuple[np.ndarray, np.ndarray]:
@@ -188,7 +189,7 @@ class Engine:
     def _mine(self, out: list[SetResult]) -> list[SetResult]:
         w = weakref.ref(self)
         for r in out:
-            r.engine = w
+            r._engine = w
         return out
 
     def _canonical(self, r: SetResult):
