@@ -302,7 +302,9 @@ __global__ void __launch_bounds__(256) k_canon_sort(const unsigned long long* of
                                                     unsigned cap) {
     if (!canon_ok(tot, cap)) return;
     constexpr int L = 16, V = 256 / L;
-    __shared__ int4 s_t[V][kCanonSmall];
+    // a row as its entries in order and its place: equal rows (a list given by the caller may hold
+    // some) differ by the last, and two comparisons of 64 bits order any two
+    __shared__ ulonglong2 s_t[V][kCanonSmall];
     __shared__ int s_e[V][kCanonSmall];
     __shared__ int s_u[V];
     const int g = threadIdx.x / L, l = threadIdx.x % L;
@@ -317,15 +319,22 @@ __global__ void __launch_bounds__(256) k_canon_sort(const unsigned long long* of
         int nt = (int)((unsigned)b - (unsigned)a), ne = (int)((unsigned)(b >> 32) - (unsigned)(a >> 32));
         const bool small = nt <= kCanonSmall && ne <= kCanonSmall;
         if (!small) nt = ne = 0;
-        for (int i = l; i < nt; i += L) s_t[g][i] = tb[t0 + i];
+        for (int i = l; i < nt; i += L) {
+            const int4 q = tb[t0 + i];
+            s_t[g][i] = make_ulonglong2((unsigned long long)(unsigned)q.x << 32 | (unsigned)q.y,
+                                        (unsigned long long)(unsigned)(M == 4 ? q.z : 0) << 32 | (unsigned)i);
+        }
         for (int i = l; i < ne; i += L) s_e[g][i] = eb[e0 + i];
         if (l == 0) s_u[g] = 0;
         __syncthreads();
         for (int i = l; i < nt; i += L) {
-            const int4 x = s_t[g][i];
+            const ulonglong2 x = s_t[g][i];
             int rank = 0;
-            for (int j = 0; j < nt; ++j) rank += canon_less<M>(s_t[g][j], x);
-            canon_put<M>(T, t0 + rank, (int)v, x);
+            for (int j = 0; j < nt; ++j) {
+                const ulonglong2 y = s_t[g][j];
+                rank += (y.x < x.x) | ((y.x == x.x) & (y.y < x.y));
+            }
+            canon_put<M>(T, t0 + rank, (int)v, make_int4((int)(x.x >> 32), (int)x.x, (int)(x.y >> 32), 0));
         }
         // entries repeated by a later one are dropped: the last of equal entries stays
         bool keep[kCanonSmall / L];
