@@ -34,7 +34,9 @@ static Result match(const std::vector<int4>& fv) {
     std::vector<int> tab(SIZE, -1);
     Result r;
     for (int q = 0; q < 3 * (int)fv.size(); ++q) {
-        r.o.push_back(vo::match_ridge<SIZE>(fv.data(), tab.data(), q));
+        int h = -1;
+        r.o.push_back(vo::match_ridge<SIZE>(fv.data(), tab.data(), q, h));
+        if (r.o.back() >= 0) CHECK(vo::take_ridge(tab.data(), h, r.o.back()) == r.o.back());
         (r.o.back() >= 0 ? r.pairs : r.o.back() == vo::kRidgeFirst ? r.first : r.none)++;
     }
     return r;
@@ -66,6 +68,15 @@ int main() {
         for (int i = 0; i < MC; ++i) fv.push_back({9, 3 * i, 3 * i + 1, 3 * i + 2});
         const Result r = match(fv);
         CHECK(r.pairs == 0 && r.first == SIZE && r.none == 3 * MC - SIZE);
+    }
+    // two lanes that matched one entry in one step: one of them gets it
+    {
+        std::vector<int> tab(SIZE, -1);
+        const std::vector<int4> fv = {{9, 0, 1, 2}, {9, 0, 1, 3}, {9, 0, 1, 4}};
+        int h0 = -1, h1 = -1, h2 = -1;
+        CHECK(vo::match_ridge<SIZE>(fv.data(), tab.data(), 2, h0) == vo::kRidgeFirst);
+        CHECK(vo::match_ridge<SIZE>(fv.data(), tab.data(), 5, h1) == 2 && vo::match_ridge<SIZE>(fv.data(), tab.data(), 8, h2) == 2);
+        CHECK(h1 == h0 && h2 == h0 && vo::take_ridge(tab.data(), h1, 2) == 2 && vo::take_ridge(tab.data(), h2, 2) != 2);
     }
     // three facets on one ridge, and ridges alone: the third is nobody's partner
     {

@@ -858,19 +858,19 @@ __device__ __forceinline__ void commit_pass(const Ctx c, int nwin, unsigned long
                 __builtin_amdgcn_wave_barrier();
                 for (int q0 = 0; q0 < nf * D; q0 += G) {
                     const int q = q0 + g.gl;
-                    const int o = q < nf * D ? match_ridge<HS>(s_fv[g.gid], L.tab[g.gid], q) : kRidgeFirst;
-                    found += __popcll(g.ballot(o >= 0));
-                    if (o == kRidgeFirst) continue;
+                    int h = 0;
+                    const int o = q < nf * D ? match_ridge<HS>(s_fv[g.gid], L.tab[g.gid], q, h) : kRidgeFirst;
+                    const int took = take_ridge(L.tab[g.gid], h, o);
                     const int j = q / D, k = 1 + q % D;
-                    const int Nj = reuse ? s_fac[g.gid][j] : base + j;
-                    if (o == kRidgeNoRoom) {
-                        *a_ptr<D>(c, Nj, k) = -1;
-                        continue;
+                    if (o >= 0) {
+                        const int jj = o / D, kk = 1 + o % D;
+                        const int Nj = reuse ? s_fac[g.gid][j] : base + j, Njj = reuse ? s_fac[g.gid][jj] : base + jj;
+                        *a_ptr<D>(c, Nj, k) = (Njj << 2) | kk;
+                        *a_ptr<D>(c, Njj, kk) = (Nj << 2) | k;
+                    } else if (o == kRidgeNoRoom) {
+                        *a_ptr<D>(c, reuse ? s_fac[g.gid][j] : base + j, k) = -1;
                     }
-                    const int jj = o / D, kk = 1 + o % D;
-                    const int Njj = reuse ? s_fac[g.gid][jj] : base + jj;
-                    *a_ptr<D>(c, Nj, k) = (Njj << 2) | kk;
-                    *a_ptr<D>(c, Njj, kk) = (Nj << 2) | k;
+                    found += __popcll(g.ballot(took == o));
                 }
                 // an open boundary: the ridges still without a partner lead nowhere
                 if (2 * found != nf * D) {
