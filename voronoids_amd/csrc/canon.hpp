@@ -8,9 +8,9 @@
 //    vertex, whose few entries are then sorted in LDS.  A vertex has about 7 simplices and 13 edge
 //    entries, so one scatter and one short sort take the place of a radix sort's 14 to 18 passes
 //    over all of them;
-//  * a stable least-significant-digit radix sort of 64-bit keys (8-bit digits, optional 32-bit
-//    payload), for trees with a vertex whose bucket outgrows LDS (kCanonBig).  Each sort pass is
-//    three kernels: per-tile digit histograms (tile = 4,096 elements, one block), a scan of the
+//  * where a vertex's bucket outgrows LDS (kCanonBig), the same rows and edge entries by a stable
+//    least-significant-digit radix sort of 64-bit keys (8-bit digits, optional 32-bit payload).  Each
+//    sort pass is per-tile digit histograms (tile = 4,096 elements, one block), a scan of the
 //    histograms in digit-major order (tile offsets of every digit), and a stable scatter in which
 //    each wavefront ranks its 64 elements per digit with ballots.
 #pragma once
@@ -248,11 +248,11 @@ __device__ __forceinline__ bool canon_ok(const CanonTot* tot, unsigned cap) {
     return tot->rows <= cap && tot->max_bucket <= (unsigned)kCanonBig;
 }
 
-// rows to their buckets: a simplex's other vertices (16 B) and the edges' other ends (4 B)
-__global__ void __launch_bounds__(256) k_canon_scatter(const int4* rows, const int4* ranks, unsigned cap, const CanonTot* tot,
-                                                       const unsigned long long* ofs, int4* tb, int* eb) {
-    if (!canon_ok(tot, cap)) return;
-    const unsigned n = tot->rows;
+// every row and edge entry with its place in the buckets: row(place, r0, r1, r2, r3), edge(place,
+// least, other)
+template <class Row, class Edge>
+__device__ __forceinline__ void canon_places(const int4* rows, const int4* ranks, unsigned n, const unsigned long long* ofs,
+                                             Row row, Edge edge) {
     for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
         const int4 q = rows[i], k = ranks[i];
         constexpr int low = 0x3fffffff;
@@ -262,19 +262,27 @@ __global__ void __launch_bounds__(256) k_canon_scatter(const int4* rows, const i
         const bool real = r3 != kCanonNone;
         if (real || e01 || e02 || e03) {
             const unsigned long long o = ofs[r0];
-            if (real) tb[(size_t)(unsigned)o + (unsigned)k.x] = make_int4(r1, r2, r3, 0);
+            if (real) row((size_t)(unsigned)o + (unsigned)k.x, r0, r1, r2, r3);
             size_t e = (size_t)(unsigned)(o >> 32) + (unsigned)k.y;
-            if (e01) eb[e++] = r1;
-            if (e02) eb[e++] = r2;
-            if (e03) eb[e] = r3;
+            if (e01) edge(e++, r0, r1);
+            if (e02) edge(e++, r0, r2);
+            if (e03) edge(e, r0, r3);
         }
         if (e12 || e13) {
             size_t e = (size_t)(unsigned)(ofs[r1] >> 32) + (unsigned)k.z;
-            if (e12) eb[e++] = r2;
-            if (e13) eb[e] = r3;
+            if (e12) edge(e++, r1, r2);
+            if (e13) edge(e, r1, r3);
         }
-        if (e23) eb[(size_t)(unsigned)(ofs[r2] >> 32) + (unsigned)k.w] = r3;
+        if (e23) edge((size_t)(unsigned)(ofs[r2] >> 32) + (unsigned)k.w, r2, r3);
     }
+}
+
+// rows to their buckets: a simplex's other vertices (16 B) and the edges' other ends (4 B)
+__global__ void __launch_bounds__(256) k_canon_scatter(const int4* rows, const int4* ranks, unsigned cap, const CanonTot* tot,
+                                                       const unsigned long long* ofs, int4* tb, int* eb) {
+    if (!canon_ok(tot, cap)) return;
+    canon_places(rows, ranks, tot->rows, ofs, [&](size_t o, int, int r1, int r2, int r3) { tb[o] = make_int4(r1, r2, r3, 0); },
+                 [&](size_t e, int, int y) { eb[e] = y; });
 }
 
 template <int M> __device__ __forceinline__ bool canon_less(int4 a, int4 b) {
@@ -475,31 +483,9 @@ constexpr int kRadixTile = 4096;                         // 16 elements per thre
 constexpr int kRadixWaves = kRadixThreads / 64;
 constexpr int kRadixPerWave = kRadixTile / kRadixWaves;  // contiguous elements per wavefront
 
-// exclusive scan inside 256-element blocks, block totals to bsum
-__global__ void __launch_bounds__(256) k_scan_blocks(const int* in, int* out, int* bsum, int64_t n) {
-    __shared__ int s[256];
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const int v = i < n ? in[i] : 0;
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = 1; o < 256; o <<= 1) {
-        const int add = threadIdx.x >= (unsigned)o ? s[threadIdx.x - o] : 0;
-        __syncthreads();
-        s[threadIdx.x] += add;
-        __syncthreads();
-    }
-    if (i < n) out[i] = s[threadIdx.x] - v;
-    if (threadIdx.x == 255) bsum[blockIdx.x] = s[255];
-}
-
-__global__ void __launch_bounds__(256) k_scan_add(int* out, const int* boff, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i < n) out[i] += boff[blockIdx.x];
-}
-
 // per-tile histogram of the digit at `shift`: hist[d * ntiles + tile]
 __global__ void __launch_bounds__(kRadixThreads) k_radix_hist(const unsigned long long* keys, int64_t n, int shift,
-                                                             int* hist, int ntiles) {
+                                                             unsigned long long* hist, int ntiles) {
     __shared__ int h[256];
     h[threadIdx.x] = 0;
     __syncthreads();
@@ -509,7 +495,7 @@ __global__ void __launch_bounds__(kRadixThreads) k_radix_hist(const unsigned lon
         if (j < n) atomicAdd(&h[(int)((keys[j] >> shift) & 255ull)], 1);
     }
     __syncthreads();
-    hist[(int64_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    hist[(int64_t)threadIdx.x * ntiles + blockIdx.x] = (unsigned long long)h[threadIdx.x];
 }
 
 // Stable scatter of one tile: wavefront w owns elements [w * kRadixPerWave, (w + 1) * ...) of
@@ -518,22 +504,22 @@ __global__ void __launch_bounds__(kRadixThreads) k_radix_hist(const unsigned lon
 // in order, ranking equal digits among its 64 lanes with ballots.
 __global__ void __launch_bounds__(kRadixThreads) k_radix_scatter(const unsigned long long* keys, const uint32_t* vals,
                                                                 unsigned long long* okeys, uint32_t* ovals, int64_t n,
-                                                                int shift, const int* off, int ntiles) {
-    __shared__ int cnt[kRadixWaves][256];
+                                                                int shift, const unsigned long long* off, int ntiles) {
+    __shared__ unsigned cnt[kRadixWaves][256];
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     for (int d = lane; d < 256; d += 64) cnt[w][d] = 0;
     __syncthreads();
     const int64_t base = (int64_t)blockIdx.x * kRadixTile + (int64_t)w * kRadixPerWave;
     for (int i = lane; i < kRadixPerWave; i += 64) {
         const int64_t j = base + i;
-        if (j < n) atomicAdd(&cnt[w][(int)((keys[j] >> shift) & 255ull)], 1);
+        if (j < n) atomicAdd(&cnt[w][(int)((keys[j] >> shift) & 255ull)], 1u);
     }
     __syncthreads();
     // per-wavefront starting positions: tile offset of the digit + counts of earlier wavefronts
     for (int d = threadIdx.x; d < 256; d += kRadixThreads) {
-        int acc = off[(int64_t)d * ntiles + blockIdx.x];
+        unsigned acc = (unsigned)off[(int64_t)d * ntiles + blockIdx.x];
         for (int v = 0; v < kRadixWaves; ++v) {
-            const int c = cnt[v][d];
+            const unsigned c = cnt[v][d];
             cnt[v][d] = acc;
             acc += c;
         }
@@ -557,9 +543,9 @@ __global__ void __launch_bounds__(kRadixThreads) k_radix_scatter(const unsigned 
             same &= ((d >> b) & 1) ? bb : ~bb;
         }
         const int rank = __popcll(same & below);
-        const int start = valid ? cnt[w][d] : 0;
+        const unsigned start = valid ? cnt[w][d] : 0u;
         if (valid) {
-            const int pos = start + rank;
+            const unsigned pos = start + rank;
             okeys[pos] = k;
             if (vals) ovals[pos] = v;
         }
@@ -574,44 +560,20 @@ __global__ void k_iota_u32(uint32_t* v, int64_t n) {
         v[i] = (uint32_t)i;
 }
 
-// Real simplices (every vertex a point: reference id >= first) as sorted tuples of point
-// indices (id - first); flag[i] = 1 for them.  Rows of the output have stride 4 (2D: w = -1).
+// The rows and their two 64-bit sort keys, lo = columns (2, 3) (2D: column 2) and hi = columns (0, 1),
+// and the edge entries' keys (least, other), each column `nb` bits wide, at their places in the buckets.
 template <int M>
-__global__ void k_canon_rows(const int32_t* simp, int64_t n, int first, int4* rows, int* flag) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        int r[4] = {0, 0, 0, 0x7fffffff};
-        bool real = true;
-        for (int k = 0; k < M; ++k) {
-            const int v = simp[i * M + k];
-            real &= v >= first;
-            r[k] = v - first;
-        }
-        // sorting network on M <= 4 values
-        auto cs = [&](int a, int b) {
-            const int lo = r[a] < r[b] ? r[a] : r[b], hi = r[a] < r[b] ? r[b] : r[a];
-            r[a] = lo;
-            r[b] = hi;
-        };
-        if (M == 4) { cs(0, 1); cs(2, 3); cs(0, 2); cs(1, 3); cs(1, 2); }
-        else { cs(0, 1); cs(1, 2); cs(0, 1); }
-        rows[i] = make_int4(r[0], r[1], r[2], M == 4 ? r[3] : -1);
-        flag[i] = real;
-    }
-}
-
-// compacted rows and their two 64-bit sort keys: lo = columns (2, 3) (2D: column 2), hi =
-// columns (0, 1), each column `nb` bits wide
-template <int M>
-__global__ void k_canon_keys(const int4* rows, const int* flag, const int* pos, int64_t n, int nb, int4* crow,
-                             unsigned long long* klo, unsigned long long* khi) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        if (!flag[i]) continue;
-        const int4 r = rows[i];
-        const int64_t o = pos[i];
-        crow[o] = r;
-        klo[o] = M == 4 ? (((unsigned long long)r.z << nb) | (unsigned long long)r.w) : (unsigned long long)r.z;
-        khi[o] = ((unsigned long long)r.x << nb) | (unsigned long long)r.y;
-    }
+__global__ void __launch_bounds__(256) k_canon_keys(const int4* rows, const int4* ranks, unsigned n, const unsigned long long* ofs,
+                                                    int nb, int4* crow, unsigned long long* klo, unsigned long long* khi,
+                                                    unsigned long long* ekeys) {
+    auto two = [&](int a, int b) { return ((unsigned long long)a << nb) | (unsigned long long)b; };
+    canon_places(rows, ranks, n, ofs,
+                 [&](size_t o, int r0, int r1, int r2, int r3) {
+                     crow[o] = make_int4(r0, r1, r2, r3);
+                     klo[o] = M == 4 ? two(r2, r3) : (unsigned long long)r2;
+                     khi[o] = two(r0, r1);
+                 },
+                 [&](size_t e, int x, int y) { ekeys[e] = two(x, y); });
 }
 
 // key of every row in the permutation's order: dst[i] = khi[perm[i]]
@@ -632,39 +594,18 @@ __global__ void k_canon_out_rows(const int4* crow, const uint32_t* perm, int64_t
     }
 }
 
-// every vertex pair of every simplex as a key (min << nb | max); pairs with a super vertex get
-// the largest key, which sorts last
-template <int M>
-__global__ void k_canon_edge_keys(const int32_t* simp, int64_t n, int first, int nb, unsigned long long* keys) {
-    constexpr int P = M * (M - 1) / 2;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        int v[4];
-        for (int k = 0; k < M; ++k) v[k] = simp[i * M + k];
-        int e = 0;
-        for (int a = 0; a < M; ++a)
-            for (int b = a + 1; b < M; ++b) {
-                unsigned long long key = ~0ull;
-                if (v[a] >= first && v[b] >= first) {
-                    const int x = v[a] - first, y = v[b] - first;
-                    key = ((unsigned long long)(x < y ? x : y) << nb) | (unsigned long long)(x < y ? y : x);
-                }
-                keys[i * P + e++] = key;
-            }
-    }
-}
-
-// first occurrence of each real edge key in the sorted list
-__global__ void k_canon_edge_flags(const unsigned long long* keys, int64_t n, int* flag) {
+// first occurrence of each edge key in the sorted list
+__global__ void k_canon_edge_flags(const unsigned long long* keys, int64_t n, unsigned long long* flag) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        flag[i] = keys[i] != ~0ull && (i == 0 || keys[i] != keys[i - 1]);
+        flag[i] = i == 0 || keys[i] != keys[i - 1];
 }
 
-__global__ void k_canon_edge_out(const unsigned long long* keys, const int* flag, const int* pos, int64_t n, int nb,
+__global__ void k_canon_edge_out(const unsigned long long* keys, const unsigned long long* pos, int64_t n, int nb,
                                  int32_t* out) {
     const unsigned long long mask = (1ull << nb) - 1ull;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        if (!flag[i]) continue;
-        const int64_t o = pos[i];
+        const int64_t o = (int64_t)pos[i];
+        if ((int64_t)pos[i + 1] == o) continue;
         out[2 * o] = (int32_t)(keys[i] >> nb);
         out[2 * o + 1] = (int32_t)(keys[i] & mask);
     }

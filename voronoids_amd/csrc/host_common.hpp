@@ -307,7 +307,7 @@ int canonical_from_simplices(int M, const int32_t* s, int64_t nl, int32_t** T, i
 
 // The same sorted on the device: simplices (host) over n points, on stream s of the current device,
 // with idle device memory of the caller as scratch.  *done = false, and nothing else, when the
-// scratch is too small, a point index is n or more, or a vertex has too many simplices.
+// scratch is too small or a point index is n or more.
 struct DeviceBlock {
     void* p;
     size_t bytes;

@@ -1801,63 +1801,6 @@ template <class T> int idle_or_alloc(DevBuf<T>& b, void* idle, size_t idle_bytes
     return dev_alloc(&b.p, n);
 }
 
-// exclusive scan of n ints (device), total of the inputs to *total
-int device_excl_scan(hipStream_t s, const int* in, int* out, int64_t n, int64_t* total) {
-    if (n <= 0) {
-        *total = 0;
-        return 0;
-    }
-    const int64_t nb = (n + 255) / 256;
-    DevBuf<int> bsum, boff;
-    int rc;
-    if ((rc = dev_alloc(&bsum.p, (size_t)nb)) || (rc = dev_alloc(&boff.p, (size_t)nb))) return rc;
-    hipLaunchKernelGGL(k_scan_blocks, dim3((unsigned)nb), dim3(256), 0, s, in, out, bsum.p, n);
-    VO_HIP(hipGetLastError());
-    int64_t t2 = 0;
-    if (nb > 1) {
-        if ((rc = device_excl_scan(s, bsum.p, boff.p, nb, &t2))) return rc;
-        hipLaunchKernelGGL(k_scan_add, dim3((unsigned)nb), dim3(256), 0, s, out, boff.p, n);
-        VO_HIP(hipGetLastError());
-    }
-    int last_in = 0, last_out = 0;
-    VO_HIP(hipMemcpyAsync(&last_out, out + n - 1, sizeof(int), hipMemcpyDeviceToHost, s));
-    VO_HIP(hipMemcpyAsync(&last_in, in + n - 1, sizeof(int), hipMemcpyDeviceToHost, s));
-    VO_HIP(hipStreamSynchronize(s));
-    *total = (int64_t)last_out + last_in;
-    return 0;
-}
-
-// stable LSD radix sort of n 64-bit keys (only the low `bits` bits are compared) with an
-// optional 32-bit payload; keys/vals and the temporaries swap roles each pass, so the result is
-// in keys/vals on return
-int radix_sort(hipStream_t s, unsigned long long*& keys, uint32_t*& vals, unsigned long long*& ktmp, uint32_t*& vtmp,
-               int64_t n, int bits) {
-    if (n <= 1) return 0;
-    const int64_t ntiles = (n + kRadixTile - 1) / kRadixTile;
-    DevBuf<int> hist, off;
-    int rc;
-    if ((rc = dev_alloc(&hist.p, (size_t)(256 * ntiles))) || (rc = dev_alloc(&off.p, (size_t)(256 * ntiles)))) return rc;
-    for (int shift = 0; shift < bits; shift += 8) {
-        hipLaunchKernelGGL(k_radix_hist, dim3((unsigned)ntiles), dim3(kRadixThreads), 0, s, keys, n, shift, hist.p, (int)ntiles);
-        VO_HIP(hipGetLastError());
-        int64_t tot = 0;
-        if ((rc = device_excl_scan(s, hist.p, off.p, 256 * ntiles, &tot))) return rc;
-        if (tot != n) return fail(VO_ERR_INTERNAL, "radix sort: histogram total differs from the key count");
-        hipLaunchKernelGGL(k_radix_scatter, dim3((unsigned)ntiles), dim3(kRadixThreads), 0, s, keys, vals, ktmp, vtmp, n,
-                           shift, off.p, (int)ntiles);
-        VO_HIP(hipGetLastError());
-        std::swap(keys, ktmp);
-        std::swap(vals, vtmp);
-    }
-    return 0;
-}
-
-// device arrays of the canonical form, with their sizes
-struct CanonOut {
-    DevBuf<int32_t> T, E;
-    int64_t nt = 0, ne = 0;
-};
-
 // Scratch of one call: cut from the handle's idle buffers (free between runs; every call of the
 // handle waits for its stream before it returns) while they last, then allocated
 struct Scratch {
@@ -1889,6 +1832,32 @@ struct Scratch {
         return rc;
     }
 };
+
+// exclusive scan of n values into out, their total to out[n] and *total
+void scan64(hipStream_t s, const unsigned long long* in, unsigned long long* out, unsigned long long* bsum, int64_t n,
+            unsigned long long* total) {
+    const unsigned nb = (unsigned)((n + kScanTile - 1) / kScanTile);
+    hipLaunchKernelGGL(k_scan64_sums, dim3(nb), dim3(256), 0, s, in, bsum, n);
+    hipLaunchKernelGGL(k_scan64_apply, dim3(nb), dim3(256), 0, s, in, bsum, out, n, total, (int*)nullptr, (CanonTot*)nullptr);
+}
+
+// Stable LSD radix sort of n 64-bit keys (only the low `bits` bits are compared) with an optional
+// 32-bit payload; keys/vals and the temporaries swap roles each pass, so the result is in keys/vals
+// on return.  hist, off, bsum: the tiles' histograms (radix_tiles(n) x 256), their scan (one more) and
+// its block sums.
+int64_t radix_tiles(int64_t n) { return (n + kRadixTile - 1) / kRadixTile; }
+void radix_sort(hipStream_t s, unsigned long long*& keys, uint32_t*& vals, unsigned long long*& ktmp, uint32_t*& vtmp,
+                int64_t n, int bits, unsigned long long* hist, unsigned long long* off, unsigned long long* bsum) {
+    const int64_t tiles = radix_tiles(n);
+    for (int shift = 0; n > 1 && shift < bits; shift += 8) {
+        hipLaunchKernelGGL(k_radix_hist, dim3((unsigned)tiles), dim3(kRadixThreads), 0, s, keys, n, shift, hist, (int)tiles);
+        scan64(s, hist, off, bsum, 256 * tiles, off + 256 * tiles);
+        hipLaunchKernelGGL(k_radix_scatter, dim3((unsigned)tiles), dim3(kRadixThreads), 0, s, keys, vals, ktmp, vtmp, n,
+                           shift, off, (int)tiles);
+        std::swap(keys, ktmp);
+        std::swap(vals, vtmp);
+    }
+}
 
 // From this many points on the bounding sphere (and the check for non-finite coordinates) is
 // folded on the device: the upload, two kernels and two readbacks take about 45 us, the host
@@ -2502,9 +2471,54 @@ int vo_tri_export(const vo_tri* t, int32_t* simplices, int32_t* neighbors) {
 
 }  // extern "C"
 
+// Canonical form by radix sorts of the rows and edge entries that the buckets were to hold, where one
+// of these outgrows LDS: simplices by two stable sorts (columns 2-3, then columns 0-1), edges by one,
+// then their first occurrences.  nt, ne: simplices and edge entries.  Only the readback of the edges'
+// number waits for the device.  From an export and all edges of every simplex, with allocations and
+// a wait in each pass, the sorts took the whole call for 3D points around a hub of 2,862 / 8,639 /
+// 18,227 neighbors 1.32 / 1.69 / 3.25 ms, and 1.36 / 1.97 / 3.60 after buckets tried in vain; now
+// 0.74 / 0.94 / 1.53.
+static int canonical_radix(hipStream_t s, int M, int64_t n, unsigned n_rows, int64_t nt, int64_t ne, const int4* rows,
+                           const int4* ranks, const unsigned long long* ofs, CanonTot* tot, int4* crow, Scratch& mem,
+                           int32_t* T, int32_t* E, int64_t* n_E) {
+    const int nb = std::max(1, bit_length(n - 1));
+    const int64_t most = std::max(nt, ne), slots = 256 * radix_tiles(most);
+    unsigned long long *klo, *khi, *ktmp, *ekeys, *etmp, *pos, *hist, *off, *bsum;
+    uint32_t *perm, *ptmp, *none = nullptr;
+    int rc;
+    if ((rc = mem.get(&klo, (size_t)nt)) || (rc = mem.get(&khi, (size_t)nt)) || (rc = mem.get(&ktmp, (size_t)nt)) ||
+        (rc = mem.get(&perm, (size_t)nt)) || (rc = mem.get(&ptmp, (size_t)nt)) || (rc = mem.get(&ekeys, (size_t)ne)) ||
+        (rc = mem.get(&etmp, (size_t)ne)) || (rc = mem.get(&pos, (size_t)ne + 1)) || (rc = mem.get(&hist, (size_t)slots)) ||
+        (rc = mem.get(&off, (size_t)slots + 1)) || (rc = mem.get(&bsum, (size_t)(std::max(slots, ne) / kScanTile + 1))))
+        return rc;
+    auto grid = [](int64_t items) { return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((items + 255) / 256, 8192))); };
+    if (M == 4) hipLaunchKernelGGL(k_canon_keys<4>, grid(n_rows), dim3(256), 0, s, rows, ranks, n_rows, ofs, nb, crow, klo, khi, ekeys);
+    else hipLaunchKernelGGL(k_canon_keys<3>, grid(n_rows), dim3(256), 0, s, rows, ranks, n_rows, ofs, nb, crow, klo, khi, ekeys);
+    // least significant columns first, then the leading two (stable): lexicographic order
+    hipLaunchKernelGGL(k_iota_u32, grid(nt), dim3(256), 0, s, perm, nt);
+    radix_sort(s, klo, perm, ktmp, ptmp, nt, M == 4 ? 2 * nb : nb, hist, off, bsum);
+    hipLaunchKernelGGL(k_gather_u64, grid(nt), dim3(256), 0, s, khi, perm, klo, nt);
+    radix_sort(s, klo, perm, ktmp, ptmp, nt, 2 * nb, hist, off, bsum);
+    if (M == 4) hipLaunchKernelGGL(k_canon_out_rows<4>, grid(nt), dim3(256), 0, s, crow, perm, nt, T);
+    else hipLaunchKernelGGL(k_canon_out_rows<3>, grid(nt), dim3(256), 0, s, crow, perm, nt, T);
+    *n_E = 0;
+    if (ne == 0) return 0;
+    radix_sort(s, ekeys, none, etmp, none, ne, 2 * nb, hist, off, bsum);
+    hipLaunchKernelGGL(k_canon_edge_flags, grid(ne), dim3(256), 0, s, ekeys, ne, etmp);
+    scan64(s, etmp, pos, bsum, ne, &tot->ne);
+    hipLaunchKernelGGL(k_canon_edge_out, grid(ne), dim3(256), 0, s, ekeys, pos, ne, nb, E);
+    VO_HIP(hipGetLastError());
+    unsigned long long unique = 0;
+    VO_HIP(hipMemcpyAsync(&unique, &tot->ne, sizeof(unique), hipMemcpyDeviceToHost, s));
+    VO_HIP(hipStreamSynchronize(s));
+    *n_E = (int64_t)unique;
+    return 0;
+}
+
 // Canonical form by buckets (canon.hpp) of at most cap simplices over n points; fill(rows, ranks, cnt,
-// tot) launches the kernel that writes their rows.  *done = false when a bucket outgrows LDS.
-// Every array has its bound from cap, so one readback of the sizes is all the host waits for.
+// tot) launches the kernel that writes their rows.  *done = false where the list named a point of n or
+// more (k_canon_rows_list).  Every array has its bound from cap, so one readback of the sizes is all
+// the host waits for.
 // Measured against the radix sorts with the export and scans they need: kernels at 3D n = 4M
 // 27 -> 7.2 ms (the record stream 4.5, scatter 1.1, sorts 1.3, edges 0.2); the whole call at
 // n = 40 0.60 -> 0.15 ms, at n = 10^5 8.7 -> 2.0 ms (the sorts waited for the device once a pass).
@@ -2549,14 +2563,15 @@ static int canonical_buckets(hipStream_t s, int M, int64_t n, size_t cap, Scratc
     VO_HIP(hipMemcpyAsync(&h, tot, sizeof(h), hipMemcpyDeviceToHost, s));
     VO_HIP(hipStreamSynchronize(s));
     if (h.rows > cap) return fail(VO_ERR_INTERNAL, "live records differ from the live simplex count");
-    *done = h.max_bucket <= (unsigned)kCanonBig;
+    *done = h.max_bucket != ~0u;
     *n_T = (int64_t)(uint32_t)h.te;
     *n_E = (int64_t)h.ne;
-    return 0;
+    if (!*done || h.max_bucket <= (unsigned)kCanonBig) return 0;
+    return canonical_radix(s, M, n, h.rows, *n_T, (int64_t)(h.te >> 32), rows, ranks, ofs, tot, tb, mem, *T, *E, n_E);
 }
 
 // Canonical form by buckets of a tree.
-static int canonical_tree(const vo_tri* t, Scratch& mem, int32_t** T, int32_t** E, int64_t* n_T, int64_t* n_E, bool* done) {
+static int canonical_tree(const vo_tri* t, Scratch& mem, int32_t** T, int32_t** E, int64_t* n_T, int64_t* n_E) {
     const size_t cap = (size_t)t->n_live;
     const Ctx c = make_ctx(t);
     auto fill = [&](int4* rows, int4* ranks, unsigned long long* cnt, CanonTot* tot) {
@@ -2568,106 +2583,21 @@ static int canonical_tree(const vo_tri* t, Scratch& mem, int32_t** T, int32_t** 
             hipLaunchKernelGGL(k_canon_rows_tree<2>, g, dim3(256), 0, t->s, c, t->vmap, t->n_tets, (int)t->edited, rows, ranks,
                                (unsigned)cap, cnt, tot);
     };
-    return canonical_buckets(t->s, t->M, t->n_pts, cap, mem, fill, T, E, n_T, n_E, done);
+    bool done = false;                 // (always: a tree names its own points)
+    return canonical_buckets(t->s, t->M, t->n_pts, cap, mem, fill, T, E, n_T, n_E, &done);
 }
 
 extern "C" {
-
-// Canonical form by radix sorts: real simplices as sorted tuples in lexicographic order (two
-// stable sorts: columns 2-3, then columns 0-1), real edges sorted and unique.
-static int canonical_radix(const vo_tri* t, CanonOut& out) {
-    const int M = t->M;
-    const hipStream_t s = t->s;
-    DevBuf<int32_t> ds, dn;
-    int64_t nl = 0;
-    int rc = export_device(t, ds, dn, &nl);
-    if (rc) return rc;
-    if (dn.own) hipFree(dn.p);
-    dn.p = nullptr;
-    const int first = 2 * M;
-    const int nb = std::max(1, bit_length(t->n_pts - 1));
-    const unsigned grid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(4096, (nl + 255) / 256));
-    // ---- simplices
-    int64_t& nt = out.nt;
-    DevBuf<int32_t>& dT = out.T;
-    {
-        DevBuf<int4> rows, crow;
-        DevBuf<int> flag, pos;
-        if ((rc = dev_alloc(&rows.p, (size_t)std::max<int64_t>(nl, 1))) || (rc = dev_alloc(&flag.p, (size_t)std::max<int64_t>(nl, 1))) ||
-            (rc = dev_alloc(&pos.p, (size_t)std::max<int64_t>(nl, 1))))
-            return rc;
-        if (M == 4) hipLaunchKernelGGL(k_canon_rows<4>, dim3(grid), dim3(256), 0, s, ds.p, nl, first, rows.p, flag.p);
-        else hipLaunchKernelGGL(k_canon_rows<3>, dim3(grid), dim3(256), 0, s, ds.p, nl, first, rows.p, flag.p);
-        VO_HIP(hipGetLastError());
-        if ((rc = device_excl_scan(s, flag.p, pos.p, nl, &nt))) return rc;
-        const size_t nt1 = (size_t)std::max<int64_t>(nt, 1);
-        DevBuf<unsigned long long> klo, khi, ktmp;
-        DevBuf<uint32_t> perm, ptmp;
-        if ((rc = dev_alloc(&crow.p, nt1)) || (rc = dev_alloc(&klo.p, nt1)) || (rc = dev_alloc(&khi.p, nt1)) ||
-            (rc = dev_alloc(&ktmp.p, nt1)) || (rc = dev_alloc(&perm.p, nt1)) || (rc = dev_alloc(&ptmp.p, nt1)) ||
-            (rc = dev_alloc(&dT.p, nt1 * M)))
-            return rc;
-        if (M == 4) hipLaunchKernelGGL(k_canon_keys<4>, dim3(grid), dim3(256), 0, s, rows.p, flag.p, pos.p, nl, nb, crow.p, klo.p, khi.p);
-        else hipLaunchKernelGGL(k_canon_keys<3>, dim3(grid), dim3(256), 0, s, rows.p, flag.p, pos.p, nl, nb, crow.p, klo.p, khi.p);
-        hipLaunchKernelGGL(k_iota_u32, dim3(grid), dim3(256), 0, s, perm.p, nt);
-        VO_HIP(hipGetLastError());
-        // least significant columns first, then the leading two (stable): lexicographic order
-        if ((rc = radix_sort(s, klo.p, perm.p, ktmp.p, ptmp.p, nt, M == 4 ? 2 * nb : nb))) return rc;
-        hipLaunchKernelGGL(k_gather_u64, dim3(grid), dim3(256), 0, s, khi.p, perm.p, klo.p, nt);
-        VO_HIP(hipGetLastError());
-        if ((rc = radix_sort(s, klo.p, perm.p, ktmp.p, ptmp.p, nt, 2 * nb))) return rc;
-        if (M == 4) hipLaunchKernelGGL(k_canon_out_rows<4>, dim3(grid), dim3(256), 0, s, crow.p, perm.p, nt, dT.p);
-        else hipLaunchKernelGGL(k_canon_out_rows<3>, dim3(grid), dim3(256), 0, s, crow.p, perm.p, nt, dT.p);
-        VO_HIP(hipGetLastError());
-    }
-    // ---- edges
-    int64_t& ne = out.ne;
-    DevBuf<int32_t>& dE = out.E;
-    {
-        const int P = M * (M - 1) / 2;
-        const int64_t nk = nl * P;
-        const size_t nk1 = (size_t)std::max<int64_t>(nk, 1);
-        DevBuf<unsigned long long> keys, ktmp;
-        DevBuf<int> flag, pos;
-        uint32_t* nov = nullptr;
-        uint32_t* novt = nullptr;
-        if ((rc = dev_alloc(&keys.p, nk1)) || (rc = dev_alloc(&ktmp.p, nk1)) || (rc = dev_alloc(&flag.p, nk1)) ||
-            (rc = dev_alloc(&pos.p, nk1)))
-            return rc;
-        if (M == 4) hipLaunchKernelGGL(k_canon_edge_keys<4>, dim3(grid), dim3(256), 0, s, ds.p, nl, first, nb, keys.p);
-        else hipLaunchKernelGGL(k_canon_edge_keys<3>, dim3(grid), dim3(256), 0, s, ds.p, nl, first, nb, keys.p);
-        VO_HIP(hipGetLastError());
-        if ((rc = radix_sort(s, keys.p, nov, ktmp.p, novt, nk, 2 * nb))) return rc;
-        const unsigned egrid = (unsigned)std::max<int64_t>(1, std::min<int64_t>(8192, (nk + 255) / 256));
-        hipLaunchKernelGGL(k_canon_edge_flags, dim3(egrid), dim3(256), 0, s, keys.p, nk, flag.p);
-        VO_HIP(hipGetLastError());
-        if ((rc = device_excl_scan(s, flag.p, pos.p, nk, &ne))) return rc;
-        if ((rc = dev_alloc(&dE.p, (size_t)std::max<int64_t>(ne, 1) * 2))) return rc;
-        hipLaunchKernelGGL(k_canon_edge_out, dim3(egrid), dim3(256), 0, s, keys.p, flag.p, pos.p, nk, nb, dE.p);
-        VO_HIP(hipGetLastError());
-    }
-    VO_HIP(hipStreamSynchronize(s));        // before the temporaries are freed
-    return 0;
-}
 
 // Canonical form on the device, copied to malloc'd arrays.  The same output as
 // canonical_from_simplices on the host, which the engine's results use.
 static int canonical_device(const vo_tri* t, int32_t** T, int64_t* n_T, int32_t** E, int64_t* n_E) {
     const int M = t->M;
     Scratch mem(t);
-    CanonOut slow;
     int32_t *dT = nullptr, *dE = nullptr;
     int64_t nt = 0, ne = 0;
     int rc;
-    bool done = t->n_pts == 0;
-    if (!done && (rc = canonical_tree(t, mem, &dT, &dE, &nt, &ne, &done))) return rc;
-    if (!done) {
-        if ((rc = canonical_radix(t, slow))) return rc;
-        dT = slow.T.p;
-        dE = slow.E.p;
-        nt = slow.nt;
-        ne = slow.ne;
-    }
+    if (t->n_pts > 0 && (rc = canonical_tree(t, mem, &dT, &dE, &nt, &ne))) return rc;
     const size_t bt = sizeof(int32_t) * (size_t)nt * M, be = sizeof(int32_t) * (size_t)ne * 2;
     *T = (int32_t*)result_alloc(bt);
     *E = (int32_t*)result_alloc(be);
