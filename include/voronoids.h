@@ -225,6 +225,10 @@ int vo_tri_vertices(const vo_tri* t, double* coords);
 
 const char* vo_last_error(void);
 int vo_version(void);
+/* how this thread's last canonical form (vo_tri_canonical, vo_result_canonical, vo_engine_canonical)
+ * was sorted: 0 none yet or nothing to sort, 1 on the device by buckets, 2 on the device by radix
+ * sorts, 3 on the host */
+int vo_canonical_route(void);
 
 /* geometry::bounding_sphere (src/geometry.rs:99-141), host only: center[dim] and radius of the sphere
  * DelaunayTree::new builds its super simplex around (per-axis min/max midpoint, then the radius x 1.5

@@ -23,7 +23,7 @@ VO_ERR_INTERNAL = -7
 EXPORTED = [
     "vo_tri_create", "vo_tri_destroy", "vo_tri_insert", "vo_tri_stage", "vo_tri_run", "vo_tri_counts",
     "vo_tri_export", "vo_tri_canonical", "vo_free", "vo_tri_check", "vo_tri_stats", "vo_tri_config", "vo_tri_vertices",
-    "vo_last_error", "vo_version",
+    "vo_last_error", "vo_version", "vo_canonical_route",
     "vo_engine_create", "vo_engine_destroy", "vo_engine_submit", "vo_engine_step", "vo_engine_launch",
     "vo_engine_finish", "vo_engine_results", "vo_engine_stats_get", "vo_engine_config", "vo_batch_triangulate",
     "vo_result_canonical", "vo_engine_canonical", "vo_clock",

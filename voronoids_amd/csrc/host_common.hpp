@@ -17,6 +17,7 @@
 namespace vo_host {
 
 inline thread_local std::string g_err;
+inline thread_local int g_canonical_route = 0;       // vo_canonical_route
 
 inline int fail(int code, const std::string& msg) {
     g_err = msg;

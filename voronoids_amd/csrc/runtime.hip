@@ -36,6 +36,7 @@ using namespace vo_host;
 namespace vo_host {
 int canonical_from_simplices(int M, const int32_t* s, int64_t nl, int32_t** T, int64_t* n_T, int32_t** E,
                              int64_t* n_E) {
+    g_canonical_route = 3;
     const int32_t first = 2 * M;
     std::vector<std::array<int32_t, 4>> tris;
     std::vector<std::array<int32_t, 2>> edges;
@@ -2075,6 +2076,7 @@ int vo_predicates_noalloc(int hip_device, int type, const double* pts, int64_t n
 
 const char* vo_last_error(void) { return vo_host::g_err.c_str(); }
 int vo_version(void) { return 1; }
+int vo_canonical_route(void) { return vo_host::g_canonical_route; }
 
 int vo_bounding_sphere(int dim, const double* pts, int64_t n, double* center, double* radius) {
     if (dim != 2 && dim != 3) return fail(VO_ERR_INVALID, "dim must be 2 or 3");
@@ -2566,7 +2568,8 @@ static int canonical_buckets(hipStream_t s, int M, int64_t n, size_t cap, Scratc
     *done = h.max_bucket != ~0u;
     *n_T = (int64_t)(uint32_t)h.te;
     *n_E = (int64_t)h.ne;
-    if (!*done || h.max_bucket <= (unsigned)kCanonBig) return 0;
+    g_canonical_route = !*done ? 0 : h.max_bucket <= (unsigned)kCanonBig ? 1 : 2;
+    if (g_canonical_route != 2) return 0;
     return canonical_radix(s, M, n, h.rows, *n_T, (int64_t)(h.te >> 32), rows, ranks, ofs, tot, tb, mem, *T, *E, n_E);
 }
 
@@ -2597,6 +2600,7 @@ static int canonical_device(const vo_tri* t, int32_t** T, int64_t* n_T, int32_t*
     int32_t *dT = nullptr, *dE = nullptr;
     int64_t nt = 0, ne = 0;
     int rc;
+    g_canonical_route = 0;
     if (t->n_pts > 0 && (rc = canonical_tree(t, mem, &dT, &dE, &nt, &ne))) return rc;
     const size_t bt = sizeof(int32_t) * (size_t)nt * M, be = sizeof(int32_t) * (size_t)ne * 2;
     *T = (int32_t*)result_alloc(bt);
