@@ -593,8 +593,7 @@ __device__ void plan_step(RunPlan& p, RoundState* st, bool s_absorb) {
             return;
         }
         // (loaded together: every trip of this one thread to memory is a part of each round's time)
-        const int nwin = p.nwin, w = st->n_winners, nx = st->n_next_pending, nq = st->n_q, paused = st->n_paused;
-        const int shift = p.ctl.walk_shift, stalled = p.stalled;
+        const int nwin = p.nwin, w = st->n_winners, nx = st->n_next_pending, paused = st->n_paused, shift = p.ctl.walk_shift;
         const int consumed = nwin - nx - w;
         p.dups += consumed;
         p.inserted += w;
@@ -608,15 +607,16 @@ __device__ void plan_step(RunPlan& p, RoundState* st, bool s_absorb) {
         if (frac > hi) p.gamma = fmin(p.gamma * 1.5, 4.0);
         else if (frac < lo && !walked) p.gamma = fmax(p.gamma * 0.7, 0.002);
         // (a round that only walked is followed by longer walks)
-        const int idle = stalled + (!walked || shift == kWalkShiftMax);
-        p.stalled = w || consumed || nq ? 0 : idle;
-        p.ctl.walk_shift = next_walk_shift(shift, nwin, paused);
+        const bool idle = w == 0 && consumed == 0 && st->n_q == 0;
+        p.stalled = idle ? p.stalled + (!walked || shift == kWalkShiftMax) : 0;
+        const int next = next_walk_shift(shift, nwin, paused);
+        if (next != shift) p.ctl.walk_shift = next;
         p.npend = nx;
         p.cur ^= 1;
         p.head += p.nfresh;
         p.rounds++;
         p.launched = 0;
-        if (idle > 64 && !(w || consumed || nq)) p.halt |= HALT_STALL;
+        if (p.stalled > 64) p.halt |= HALT_STALL;
     }
     if (p.halt) return;
     if (p.head >= p.n_pts && p.npend == 0) {
