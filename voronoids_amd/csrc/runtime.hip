@@ -2363,11 +2363,17 @@ int vo_tri_run(vo_tri* t) {
     // (the small-run rule looks at the points the first phase leaves)
     int rc;
     const int seed = seed_limit(t);
+    // a run that fails leaves records that the host may not have counted; a reset clears them
+    auto failed = [&](int code) {
+        const std::string why = g_err;
+        if (sync_state(t) == 0) t->n_tets = std::max(t->n_tets, t->st_host->n_tets);
+        return fail(code, why);
+    };
     if (t->n_tets == 1 && t->inserted == 0 && t->npend == 0 && seed > 0 && t->group == 0 && !tf.f && (rc = run_seed(t, seed)))
-        return rc;
+        return failed(rc);
     const int64_t todo = t->n_pts - t->head + t->npend;
     const bool host_loop = !t->pipelined || tf.f || t->xcd || t->compact_ratio > 0 || todo <= t->small_run;
-    if (todo > 0 && (rc = host_loop ? run_host_planned(t, tf.f) : run_device_planned(t))) return rc;
+    if (todo > 0 && (rc = host_loop ? run_host_planned(t, tf.f) : run_device_planned(t))) return failed(rc);
     VO_HIP(hipEventRecord(t->ev[1], t->s));
     VO_HIP(hipEventSynchronize(t->ev[1]));
     float ms = 0;
