@@ -3,6 +3,7 @@
 // leave the tree as it was.
 //
 //   test_limited_memory points    tables of a growing tree
+//   test_limited_memory copies    a stage that fails leaves no copy of the caller's points under way
 //   test_limited_memory compact   a run that ends for lack of records, taken up again with compaction
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
@@ -39,6 +40,23 @@ extern "C" hipError_t hipFree(void* p) {
         g_sizes.erase(it);
     }
     return real(p);
+}
+
+// copies from the caller's points not yet waited for
+static const char *g_lo = nullptr, *g_hi = nullptr;
+static int g_copies = 0, g_waited = 0;
+extern "C" hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+    using Fn = hipError_t (*)(void*, const void*, size_t, hipMemcpyKind, hipStream_t);
+    static const Fn real = (Fn)dlsym(RTLD_NEXT, "hipMemcpyAsync");
+    if ((const char*)src >= g_lo && (const char*)src < g_hi) ++g_copies;
+    return real(dst, src, bytes, kind, s);
+}
+extern "C" hipError_t hipStreamSynchronize(hipStream_t s) {
+    using Fn = hipError_t (*)(hipStream_t);
+    static const Fn real = (Fn)dlsym(RTLD_NEXT, "hipStreamSynchronize");
+    const hipError_t e = real(s);
+    g_waited = g_copies;
+    return e;
 }
 
 #define CHECK(x)                                                                                     \
@@ -84,6 +102,31 @@ static int run_points() {
     return 0;
 }
 
+static int run_copies() {
+    const int64_t n = 100000;
+    const std::vector<double> p = points(3, n, 4);
+    vo_tri* t = nullptr;
+    CHECK(vo_tri_create(0, 3, p.data(), 100, &t) == VO_OK);
+    g_lo = (const char*)p.data();
+    g_hi = g_lo + sizeof(double) * p.size();
+    // the tables fit (56 bytes a point), then less and less of what follows: scratch, the hint grid, records
+    int refused = 0;
+    for (size_t more = 5 << 20; more < ((size_t)64 << 20); more += 128 << 10) {
+        g_limit = g_used + more;
+        const int rc = vo_tri_stage(t, p.data(), n, 0);
+        CHECK(rc == VO_OK || rc == VO_ERR_OOM);
+        CHECK(g_waited == g_copies);
+        if (rc == VO_OK) break;
+        ++refused;
+    }
+    g_limit = SIZE_MAX;
+    CHECK(refused > 0);
+    g_lo = g_hi = nullptr;
+    vo_tri_destroy(t);
+    CHECK(g_used == 0);
+    return 0;
+}
+
 static int run_compact() {
     const int64_t n = 30000;
     for (const int dim : {3, 2}) {
@@ -121,6 +164,7 @@ int main(int argc, char** argv) {
     const char* what = argc > 1 ? argv[1] : "";
     int failed = 1;
     if (!std::strcmp(what, "points")) failed = run_points();
+    if (!std::strcmp(what, "copies")) failed = run_copies();
     if (!std::strcmp(what, "compact")) failed = run_compact();
     if (!failed) std::printf("%s: ok\n", what);
     return failed;

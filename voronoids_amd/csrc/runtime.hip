@@ -2266,45 +2266,24 @@ int vo_tri_stage(vo_tri* t, const double* pts, int64_t n, uint64_t seed) {
     // vertex ids are committed (n_pts) only once every upload and allocation has succeeded, so
     // that a failed stage leaves the handle as it was
     const int64_t v0 = M + t->n_pts, n_after = t->n_pts + n;
-    Scratch mem(t);
-    StagePlan p = {};
-    double* dpts;
-    if ((rc = mem.get(&dpts, (size_t)n * D))) return rc;
-    VO_HIP(hipMemcpyAsync(dpts, pts, sizeof(double) * (size_t)n * D, hipMemcpyHostToDevice, t->s));
-    p.pts = dpts;
-    p.seed = seed;
-    p.n = n;
-    p.id0 = 2 * M + t->n_pts;
-    p.D = D;
-    p.S = S;
-    for (int k = 0; k < 3; ++k) p.c[k] = t->c[k];
-    p.X64 = t->X64 + v0 * S;
-    p.X32 = t->X32 + v0 * S;
-    p.vmap = t->vmap + v0;
-    p.cp = t->cp + t->n_pts;
     const dim3 grid((unsigned)std::min<int64_t>((n + 255) / 256, 8192));
     std::vector<int32_t> perm;
     if (t->local_order) {
         // (sorted on the host, so checked there first)
         if (dev_check && !all_finite(pts, n * D)) return fail(VO_ERR_INVALID, "non-finite coordinate");
         perm = priority_order_local(D, pts, n, seed, t->c, t->r, t->local_order);
-        int32_t* dperm;
-        if ((rc = mem.get(&dperm, (size_t)n))) return rc;
-        VO_HIP(hipMemcpyAsync(dperm, perm.data(), sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, t->s));
-        p.perm = dperm;
-    } else if (n > 1) {
-        int *head, *next;
-        if ((rc = mem.get(&head, (size_t)n)) || (rc = mem.get(&next, (size_t)n))) return rc;
-        VO_HIP(hipMemsetAsync(head, 0xFF, sizeof(int) * (size_t)n, t->s));
-        hipLaunchKernelGGL(k_shuffle_links, grid, dim3(256), 0, t->s, seed, n, head, next);
-        p.head = head;
-        p.next = next;
     }
-    int bad = 0;
-    if (dev_check) {
-        if ((rc = mem.get(&p.bad, 1))) return rc;
-        VO_HIP(hipMemsetAsync(p.bad, 0, sizeof(int), t->s));
-    }
+    // every allocation before the first copy: none is under way from the caller's buffer when the
+    // call fails for lack of memory
+    Scratch mem(t);
+    StagePlan p = {};
+    double* dpts;
+    int32_t* dperm = nullptr;
+    int *head = nullptr, *next = nullptr;
+    if ((rc = mem.get(&dpts, (size_t)n * D)) || (t->local_order && (rc = mem.get(&dperm, (size_t)n))) ||
+        (!t->local_order && n > 1 && ((rc = mem.get(&head, (size_t)n)) || (rc = mem.get(&next, (size_t)n)))) ||
+        (dev_check && (rc = mem.get(&p.bad, 1))))
+        return rc;
     // walk-start hints: grids of 2^l cells per axis over the bounding sphere's box, finest
     // level about 4 points a cell; level 0 holds the initial simplex
     const int L = t->hinted ? t->hlevels : hint_levels(D, n_after);
@@ -2319,6 +2298,28 @@ int vo_tri_stage(vo_tri* t, const double* pts, int64_t n, uint64_t seed) {
         }
         p.hint = t->hint;
     }
+    p.pts = dpts;
+    p.perm = dperm;
+    p.head = head;
+    p.next = next;
+    p.seed = seed;
+    p.n = n;
+    p.id0 = 2 * M + t->n_pts;
+    p.D = D;
+    p.S = S;
+    for (int k = 0; k < 3; ++k) p.c[k] = t->c[k];
+    p.X64 = t->X64 + v0 * S;
+    p.X32 = t->X32 + v0 * S;
+    p.vmap = t->vmap + v0;
+    p.cp = t->cp + t->n_pts;
+    VO_HIP(hipMemcpyAsync(dpts, pts, sizeof(double) * (size_t)n * D, hipMemcpyHostToDevice, t->s));
+    if (dperm) VO_HIP(hipMemcpyAsync(dperm, perm.data(), sizeof(int32_t) * (size_t)n, hipMemcpyHostToDevice, t->s));
+    if (head) {
+        VO_HIP(hipMemsetAsync(head, 0xFF, sizeof(int) * (size_t)n, t->s));
+        hipLaunchKernelGGL(k_shuffle_links, grid, dim3(256), 0, t->s, seed, n, head, next);
+    }
+    int bad = 0;
+    if (dev_check) VO_HIP(hipMemsetAsync(p.bad, 0, sizeof(int), t->s));
     hipLaunchKernelGGL(k_stage_points, grid, dim3(256), 0, t->s, p);
     VO_HIP(hipGetLastError());
     if (dev_check) VO_HIP(hipMemcpyAsync(&bad, p.bad, sizeof(int), hipMemcpyDeviceToHost, t->s));
