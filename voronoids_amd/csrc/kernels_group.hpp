@@ -4,11 +4,11 @@
 // Same algorithm and state as kernels.hpp (the reference path they replace is cited there);
 // only the mapping of work to lanes changes, to shorten the dependent-load chain of a point:
 //   walk   : the D+1 face tests of a step run on D+1 lanes at once;
-//   cavity : breadth-first by levels; the (simplex, face) pairs of a level are spread over the
-//            G lanes, the cavity and facet lists live in LDS, new members are deduplicated and
-//            appended with group ballots and popcount prefixes;
+//   cavity : breadth-first; the (simplex, face) pairs of the members found so far are one queue
+//            spread over the G lanes, the cavity and facet lists live in LDS, new members are
+//            deduplicated and appended with group ballots and popcount prefixes;
 //   commit : one lane per boundary facet builds the new simplex, one lane per (facet, ridge)
-//            rotates around the ridge and finds the neighboring facet by an LDS scan.
+//            matches the ridge in LDS, or rotates around it where the facets outgrow LDS.
 #pragma once
 #include "kernels.hpp"
 #include "ridges.hpp"
@@ -133,9 +133,10 @@ template <int D, int G> struct alignas(16) CavityLds {
 // points of the coming windows, up to twice as many as the window has, 4 lanes a point: at most
 // kAheadSteps (kAheadFar from windows of kAheadBig on, where the launch lasts longer) from where
 // they are; they write only the conflict pointer, and the hint of a walk that ended.  When their
-// round comes they are a step or two away.  The tree does not change while this kernel runs, and a
-// point's walk has no part in which points win, so rounds and windows are the same with and
-// without.  Run at 3D n = 10^4 8.1 -> 6.8 ms and 10^5 12.8 -> 11.1 when the points ahead walked with
+// round comes they are a step or two away.  The tree does not change while this kernel runs.  Without
+// a walk budget a point's walk has no part in which points win, and rounds and windows are the same
+// with and without; with one (the tuned settings) a point that has not arrived sits its round out, so
+// the rounds differ, and the triangulation does not.  Run at 3D n = 10^4 8.1 -> 6.8 ms and 10^5 12.8 -> 11.1 when the points ahead walked with
 // the window's lanes and only beside small windows; with 4 lanes and beside all of them also
 // clustered 10^6 46.0 -> 41.4 and 4M 59.0 -> 57.1.  (kAheadSteps 8 or 24: 1% slower at 10^5;
 // kAheadFar 48 from 8,192 on: 58.5 at 4M; as many points ahead as the window, not twice: clustered

@@ -6,8 +6,13 @@
 // into a ring of pinned slots at the link's rate and several threads move the slots on, so that
 // faults and copies run beside each other and beside the link.  With huge pages for the results
 // and no further copy of them in Python: the canonical form at 3D n = 4M 225 -> 25 ms (7 of it on
-// the device), 2D n = 10M 157 -> 17.5 ms, the export at 3D n = 4M 92 -> 32 ms.  Eight or fifteen
-// threads instead of four measured the same.
+// the device), 2D n = 10M 157 -> 17.5 ms, the export at 3D n = 4M (868 MB into the caller's arrays,
+// on small pages) 92 -> 33 ms, 29 where the pages were there before.  Eight or fifteen threads
+// instead of four measured the same.
+//
+// For up to two seconds after a gigabyte or more of device memory was freed, by any process, the
+// driver clears it with the copy engine, and copies to the host run at a quarter of the rate (pieces
+// of a slot 12 GB/s instead of 45): then the canonical form takes 65 ms and the export 81.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <sys/mman.h>
