@@ -2126,7 +2126,7 @@ int vo_tri_create(int hip_device, int dim, const double* pts, int64_t n, vo_tri*
     const hipError_t counted = hipGetDeviceCount(&ndev);
     if (counted != hipSuccess || hip_device < 0 || hip_device >= ndev) {
         if (!all_finite(pts, n * dim)) return fail(VO_ERR_INVALID, "non-finite coordinate");
-        VO_HIP(counted);
+        if (counted != hipSuccess) return fail(VO_ERR_HIP, std::string("hipGetDeviceCount: ") + hipGetErrorString(counted));
         return fail(VO_ERR_INVALID, "no such HIP device");
     }
     if (n < kDeviceFrame && !all_finite(pts, n * dim)) return fail(VO_ERR_INVALID, "non-finite coordinate");
