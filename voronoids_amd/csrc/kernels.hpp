@@ -923,6 +923,23 @@ __device__ __forceinline__ uint32_t mix32(uint32_t x) {
     return x;
 }
 
+// Point p was dropped in simplex t, one of whose vertices it equals: the inserted point q that this is
+// is noted at p's conflict pointer, which nothing reads any more, as -2 - q.  The first of equal
+// points is the one that is kept; but a walk that pauses (walk_budget) or a cavity that is searched
+// again alone lets a later one in before it, and then the two change ids (k_equal_swap).
+template <int D> __device__ __forceinline__ void note_equal(const Ctx& c, int t, int p) {
+    constexpr int S = VT<D>::S;
+    const int4 v = ld_v<D>(c, t);
+    const double* x = c.X64 + (size_t)S * (c.M + p);
+    for (int k = 0; k < D + 1; ++k) {
+        const int u = comp(v, k);
+        const double* y = c.X64 + (size_t)S * u;
+        bool same = u >= c.M;
+        for (int i = 0; i < D; ++i) same &= x[i] == y[i];
+        if (same) c.cp[p] = -2 - (u - c.M);
+    }
+}
+
 // ---------------------------------------------------------------- k_cavity
 // One thread per window point: follow dead simplices forward, walk to the simplex that
 // contains p (orientation tests), BFS the conflict region (in-sphere tests), then reserve
@@ -991,7 +1008,10 @@ __global__ void __launch_bounds__(256) k_cavity(Ctx c, int nwin, unsigned long l
         if (st == ST_OK) {
             const int s0 = conflict_at<D>(c, a, t, pv, pf, lc);
             if (s0 == SIGN_UNDECIDED) st = ST_DEFER;
-            else if (s0 <= 0) st = ST_DUP;   // on the circumsphere of its own simplex: a vertex
+            else if (s0 <= 0) {              // on the circumsphere of its own simplex: a vertex
+                st = ST_DUP;
+                note_equal<D>(c, t, p);
+            }
         }
         const unsigned long long skey = key_hi | (unsigned)p;
         if (st == ST_OK) {

@@ -367,7 +367,13 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
     s0 = g.bcast(s0, 0);
     if (st == ST_OK) {
         if (s0 == SIGN_UNDECIDED) st = ST_DEFER;
-        else if (s0 <= 0) { st = ST_DUP; if (lead) lc.dups++; }
+        else if (s0 <= 0) {
+            st = ST_DUP;
+            if (lead) {
+                lc.dups++;
+                note_equal<D>(c, t, p);
+            }
+        }
     }
     // ---- cavity: breadth-first search.  The (member, face) pairs found so far form one queue,
     // M of the first member and D of each further one, whose entry face leads back to a member; a

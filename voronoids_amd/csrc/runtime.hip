@@ -418,6 +418,33 @@ __global__ void __launch_bounds__(256) k_find_id(const int* vmap, int n, int id,
         if (vmap[i] == id) *place = i;
 }
 
+// After a run that dropped points: an inserted point q with an equal one before it gives its id to the
+// first of them (note_equal).  cp: -2 - q at dropped points; INT_MIN + p at an inserted point whose
+// first equal is p (below every -2 - q, n being below 2^30).
+__global__ void __launch_bounds__(256) k_equal_first(int* cp, int n) {
+    for (int p = blockIdx.x * 256 + (int)threadIdx.x; p < n; p += gridDim.x * 256) {
+        const int e = cp[p];
+        if (e <= -2 && e >= -1 - n && p < -2 - e) atomicMin(&cp[-2 - e], INT32_MIN + p);
+    }
+}
+template <int D> __global__ void __launch_bounds__(256) k_equal_swap(int* cp, int n, int* vmap, double* X64) {
+    constexpr int S = VT<D>::S;
+    for (int q = blockIdx.x * 256 + (int)threadIdx.x; q < n; q += gridDim.x * 256) {
+        const int e = cp[q];
+        if (e >= -1) continue;
+        cp[q] = -1;
+        if (e >= -1 - n) continue;
+        const int p = e - INT32_MIN, id = vmap[q];
+        vmap[q] = vmap[p];
+        vmap[p] = id;
+        for (int k = 0; k < S; ++k) {              // (equal but for the signs of zeros)
+            const double x = X64[(size_t)q * S + k];
+            X64[(size_t)q * S + k] = X64[(size_t)p * S + k];
+            X64[(size_t)p * S + k] = x;
+        }
+    }
+}
+
 // a host-planned round: cleared round state, and the window = pending losers followed by fresh points
 // head .. head + nfresh - 1
 __global__ void k_open_round(RoundState* st, int* win, const int* pend, int npend, int head, int nfresh) {
@@ -2375,6 +2402,14 @@ int vo_tri_run(vo_tri* t) {
     const int64_t todo = t->n_pts - t->head + t->npend;
     const bool host_loop = !t->pipelined || tf.f || t->xcd || t->compact_ratio > 0 || todo <= t->small_run;
     if (todo > 0 && (rc = host_loop ? run_host_planned(t, tf.f) : run_device_planned(t))) return failed(rc);
+    if (t->dups > dups0) {
+        const dim3 grid((unsigned)std::min<int64_t>((t->n_pts + 255) / 256, 8192));
+        double* X64 = t->X64 + (size_t)t->M * t->S;
+        hipLaunchKernelGGL(k_equal_first, grid, dim3(256), 0, t->s, t->cp, (int)t->n_pts);
+        if (t->D == 3) hipLaunchKernelGGL(k_equal_swap<3>, grid, dim3(256), 0, t->s, t->cp, (int)t->n_pts, t->vmap + t->M, X64);
+        else hipLaunchKernelGGL(k_equal_swap<2>, grid, dim3(256), 0, t->s, t->cp, (int)t->n_pts, t->vmap + t->M, X64);
+        VO_HIP(hipGetLastError());
+    }
     VO_HIP(hipEventRecord(t->ev[1], t->s));
     VO_HIP(hipEventSynchronize(t->ev[1]));
     float ms = 0;
