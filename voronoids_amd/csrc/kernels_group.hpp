@@ -367,7 +367,7 @@ __device__ __forceinline__ void cavity_pass(const Ctx c, int nwin, unsigned long
     s0 = g.bcast(s0, 0);
     if (st == ST_OK) {
         if (s0 == SIGN_UNDECIDED) st = ST_DEFER;
-        else if (s0 <= 0) {
+        else if (__builtin_expect(s0 <= 0, 0)) {
             st = ST_DUP;
             if (lead) {
                 lc.dups++;
