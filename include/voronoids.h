@@ -71,7 +71,8 @@ int vo_tri_reset(vo_tri* t, const double* pts, int64_t n);
 
 /* add_points_to_tree (src/delaunay_tree.rs:336-386) / the insert_point loop of
  * voronoids.delaunay (src/lib.rs:104-125): inserts n points in a random priority order drawn
- * from seed.  Equivalent to vo_tri_stage followed by vo_tri_run. */
+ * from seed.  Of equal points the first in that order (of an earlier call before a later one's) is
+ * kept, the others are skipped (VO_ERR_DUPLICATE).  Equivalent to vo_tri_stage followed by vo_tri_run. */
 int vo_tri_insert(vo_tri* t, const double* pts, int64_t n, uint64_t seed);
 /* stage: copy n points to the device in priority order (no insertion) */
 int vo_tri_stage(vo_tri* t, const double* pts, int64_t n, uint64_t seed);

@@ -4,6 +4,7 @@
 //
 //   test_limited_memory points    tables of a growing tree
 //   test_limited_memory copies    a stage that fails leaves no copy of the caller's points under way
+//   test_limited_memory equal     equal points over such an end: the first of them are kept
 //   test_limited_memory compact   a run that ends for lack of records, taken up again with compaction
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
@@ -127,6 +128,43 @@ static int run_copies() {
     return 0;
 }
 
+static int run_equal() {
+    const int64_t n = 30000;
+    for (const int dim : {3, 2}) {
+        std::vector<double> p = points(dim, n, 5);
+        for (int64_t i = 0; i < n / 3; ++i)              // a third of the points twice
+            for (int k = 0; k < dim; ++k) p[(size_t)(n - 1 - i) * dim + k] = p[(size_t)i * dim + k];
+        int32_t *T[2] = {}, *E[2] = {};
+        int64_t nT[2] = {}, nE[2] = {};
+        for (int ended = 0; ended < 2; ++ended) {
+            vo_tri* t = nullptr;
+            CHECK(vo_tri_create(0, dim, p.data(), n, &t) == VO_OK);
+            // (windows as large as the tree, and records for less than that, as below)
+            CHECK(vo_tri_config(t, "alloc_stripes", 0) == VO_OK && vo_tri_config(t, "window_gamma_milli", 1000) == VO_OK);
+            CHECK(vo_tri_config(t, "small_frac_lo_milli", 1) == VO_OK && vo_tri_config(t, "small_frac_hi_milli", 999) == VO_OK);
+            CHECK(vo_tri_config(t, "walk_budget", 1) == VO_OK);
+            CHECK(vo_tri_stage(t, p.data(), n, 0) == VO_OK);
+            int rc = 0;
+            if (ended) {
+                g_limit = g_used + 1000000;
+                CHECK(vo_tri_run(t) == VO_ERR_OOM);
+                g_limit = SIZE_MAX;
+            }
+            rc = vo_tri_run(t);
+            CHECK(rc == VO_ERR_DUPLICATE || (ended && rc == VO_OK));
+            CHECK(vo_tri_canonical(t, &T[ended], &nT[ended], &E[ended], &nE[ended]) == VO_OK);
+            vo_tri_destroy(t);
+        }
+        CHECK(nT[0] == nT[1] && nE[0] == nE[1]);
+        CHECK(!std::memcmp(T[0], T[1], sizeof(int32_t) * nT[0] * (dim + 1)) && !std::memcmp(E[0], E[1], sizeof(int32_t) * nE[0] * 2));
+        for (int k = 0; k < 2; ++k) {
+            vo_free(T[k]);
+            vo_free(E[k]);
+        }
+    }
+    return 0;
+}
+
 static int run_compact() {
     const int64_t n = 30000;
     for (const int dim : {3, 2}) {
@@ -165,6 +203,7 @@ int main(int argc, char** argv) {
     int failed = 1;
     if (!std::strcmp(what, "points")) failed = run_points();
     if (!std::strcmp(what, "copies")) failed = run_copies();
+    if (!std::strcmp(what, "equal")) failed = run_equal();
     if (!std::strcmp(what, "compact")) failed = run_compact();
     if (!failed) std::printf("%s: ok\n", what);
     return failed;

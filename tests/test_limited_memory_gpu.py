@@ -9,7 +9,7 @@ BIN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "_bin", "t
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("what", ["points", "copies", "compact"])
+@pytest.mark.parametrize("what", ["points", "copies", "equal", "compact"])
 def test_limited_memory(what):
     r = subprocess.run([BIN, what], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and f"{what}: ok" in r.stdout, r.stdout + r.stderr

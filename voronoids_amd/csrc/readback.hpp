@@ -11,7 +11,7 @@
 // instead of four measured the same.
 //
 // For up to two seconds after a gigabyte or more of device memory was freed, by any process, the
-// driver clears it with the copy engine, and copies to the host run at a quarter of the rate (pieces
+// system clears it with the copy engine, and copies to the host run at a quarter of the rate (pieces
 // of a slot 12 GB/s instead of 45): then the canonical form takes 65 ms and the export 81.
 #pragma once
 #include <hip/hip_runtime.h>

@@ -212,6 +212,7 @@ struct vo_tri {
     int64_t lanes_target = 0;          // auto group size: largest G with window * G <= this (0 = default)
     int64_t commit_lanes_target = 0;   // the same for the commit kernel (0 = lanes_target)
     int64_t inserted = 0, dups = 0, rounds = 0, windows_total = 0;
+    int64_t dups_settled = 0;          // dropped points whose equals have the ids they should (k_equal_swap)
     int64_t rounds0 = 0;               // rounds before the last vo_tri_reset (keys keep decreasing)
     double ms_run = 0, ms_cav = 0, ms_com = 0, ms_ex = 0, ms_other = 0;
     int64_t n_cav = 0, n_com = 0, n_solo = 0;
@@ -2251,7 +2252,7 @@ int vo_tri_reset(vo_tri* t, const double* pts, int64_t n) {
     t->n_live = 1;
     t->retired = 0;
     t->cur = t->npend = 0;
-    t->inserted = t->dups = t->windows_total = 0;
+    t->inserted = t->dups = t->dups_settled = t->windows_total = 0;
     t->rounds0 = t->rounds;
     t->stalled = 0;
     t->exact_dev = 0;
@@ -2402,13 +2403,14 @@ int vo_tri_run(vo_tri* t) {
     const int64_t todo = t->n_pts - t->head + t->npend;
     const bool host_loop = !t->pipelined || tf.f || t->xcd || t->compact_ratio > 0 || todo <= t->small_run;
     if (todo > 0 && (rc = host_loop ? run_host_planned(t, tf.f) : run_device_planned(t))) return failed(rc);
-    if (t->dups > dups0) {
+    if (t->dups > t->dups_settled) {
         const dim3 grid((unsigned)std::min<int64_t>((t->n_pts + 255) / 256, 8192));
         double* X64 = t->X64 + (size_t)t->M * t->S;
         hipLaunchKernelGGL(k_equal_first, grid, dim3(256), 0, t->s, t->cp, (int)t->n_pts);
         if (t->D == 3) hipLaunchKernelGGL(k_equal_swap<3>, grid, dim3(256), 0, t->s, t->cp, (int)t->n_pts, t->vmap + t->M, X64);
         else hipLaunchKernelGGL(k_equal_swap<2>, grid, dim3(256), 0, t->s, t->cp, (int)t->n_pts, t->vmap + t->M, X64);
         VO_HIP(hipGetLastError());
+        t->dups_settled = t->dups;
     }
     VO_HIP(hipEventRecord(t->ev[1], t->s));
     VO_HIP(hipEventSynchronize(t->ev[1]));
