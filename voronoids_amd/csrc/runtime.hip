@@ -1410,9 +1410,13 @@ int finish_round(vo_tri* t, int nwin, int nfresh, FILE* trace, float ms_cav, flo
     const int n_big = t->st_host->n_big;
     int winners = totals ? t->st_host->n_winners : 0, live = totals ? t->st_host->n_live_delta : 0;
     int paused = totals ? t->st_host->n_paused : 0;
+    const bool queued = t->st_host->n_q > 0;
     if (n_big > 0 && (rc = run_solo(t, n_big))) return rc;
     const RoundState& r = *t->st_host;
-    if (r.n_q > 0 && !exact_done) {      // (exact_done: evaluated in the stream after the commit)
+    // (exact_done: the round's queue was evaluated in the stream after the commit and emptied, and what
+    // is in it now comes from the points re-run alone.  Left there, their predicates would be queued
+    // again by every round to come)
+    if (r.n_q > 0 && (!exact_done || n_big > 0)) {
         if ((rc = run_exact(t, r.n_q))) return rc;
         if ((rc = sync_state(t)) || (rc = check_err(t))) return rc;
     }
@@ -1450,7 +1454,7 @@ int finish_round(vo_tri* t, int nwin, int nfresh, FILE* trace, float ms_cav, flo
     else if (frac < lo && !walked) t->gamma = std::max(t->gamma * 0.7, 0.002);
     // every round either inserts, drops a duplicate, resolves queued predicates, or is followed by
     // longer walks
-    if (winners || consumed || r.n_q) t->stalled = 0;
+    if (winners || consumed || queued || r.n_q) t->stalled = 0;
     else if (!walked || t->walk_shift == kWalkShiftMax) t->stalled++;
     t->walk_shift = next_walk_shift(t->walk_shift, nwin, paused);
     if (t->stalled > 64) return fail(VO_ERR_INTERNAL, "no progress for 64 rounds");
